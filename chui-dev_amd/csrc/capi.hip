@@ -56,8 +56,8 @@ struct chui_treepm_context {
   std::size_t vjp_safe_cap = 0;  // accepted-list slots a recorded VJP sorts (learned by eager VJPs)
   DeviceBuffer src64, src32, htab;  // tree-ordered packed sources; H(t) table
   double htab_key[2] = {0.0, 0.0};
-  DeviceBuffer h64tab;              // FP64 box walk: degree-5 cells of H(t)
-  double h64_key[2] = {0.0, 0.0};
+  DeviceBuffer h64tab;              // FP64 box walk: degree-5 cells of -H(t) / 8a^3
+  double h64_key[3] = {0.0, 0.0, 0.0};
   // mixed timed walk: bit-indexed residual cells, keyed by (scale, eps, r_s)
   DeviceBuffer ltab;
   std::vector<float> ltab_host;
@@ -424,12 +424,12 @@ chui::WalkParams base_walk_params(const Ctx* c, const chui_treepm_options* o, co
     wp.contain2_sep = static_cast<float>(r2 * (1.0 - 1.0e-5));
   }
   for (int a = 0; a < 3; ++a) {
-    // box-classified walk for waves whose targets lie within +-2 r_cut of the
-    // box centre per axis. At 256^3 a bound of +-r_cut leaves 79% of the
-    // waves to the lane-by-lane walk; +-2 r_cut measured 13% faster in total,
-    // +-3 and +-4 r_cut slower again (more sources per wider box).
+    // a run of targets shares one traversal when it lies within +-r_cut of its
+    // box centre per axis; a wider run is halved. +-2 r_cut: 256^3 18.2 against
+    // 17.5 ms, 128^3 2.13 against 2.03 ms (the wider boxes reach more sources,
+    // and their larger offsets round coarser in FP32)
     const double sep = wp.cubic ? o->box_size[a] / 4294967296.0 : 1.0;
-    wp.box_half_max[a] = static_cast<float>(2.0 * sp.rcut / sep);
+    wp.box_half_max[a] = static_cast<float>(sp.rcut / sep);
   }
   for (int a = 0; a < 3; ++a) {
     // float offsets from a wave origin: targets within L/16 (precision) and
@@ -439,6 +439,8 @@ chui::WalkParams base_walk_params(const Ctx* c, const chui_treepm_options* o, co
     const double lim = std::min(268435456.0, 2147483648.0 - rcut_units - 16777216.0);
     wp.fast_half_extent[a] = lim > 0.0 ? static_cast<uint32_t>(lim) : 0u;
   }
+  wp.box_max64 = 2.0 * sp.rcut;
+  wp.box_single = std::min({wp.fast_half_extent[0], wp.fast_half_extent[1], wp.fast_half_extent[2]}) >= 2u ? 1 : 0;
   wp.node_count = static_cast<uint32_t>(c->tree.node_count);
   wp.mesh_row = mesh_row;
   return wp;
@@ -449,19 +451,24 @@ chui::WalkParams base_walk_params(const Ctx* c, const chui_treepm_options* o, co
 void prepare_h64(Ctx* c, chui::WalkParams& wp, const Split& sp, hipStream_t s) {
   const double t_max = wp.rcut2 * (0.25 / (sp.a * sp.a)) * (1.0 + 1.0e-3);
   const int cells = static_cast<int>(std::min<double>(chui::kH64MaxCells, std::max(16.0, std::ceil(t_max / 0.04))));
-  if (c->h64_key[0] != t_max || c->h64_key[1] != cells || !c->h64tab.ptr) {
-    const std::vector<double> tab = chui::gaussian_quintic_table(t_max, cells);
+  const double factor = -((0.125 / sp.a) / sp.a) / sp.a;  // -1 / 8a^3
+  if (c->h64_key[0] != t_max || c->h64_key[1] != cells || c->h64_key[2] != factor || !c->h64tab.ptr) {
+    const std::vector<double> tab = chui::gaussian_quintic_table(t_max, cells, factor);
     chui::require_not_capturing(s, "the FP64 residual table");
     c->h64tab.reserve(tab.size() * sizeof(double));
     CHUI_HIP(hipMemcpyAsync(c->h64tab.ptr, tab.data(), tab.size() * sizeof(double), hipMemcpyHostToDevice, s));
     CHUI_HIP(hipStreamSynchronize(s));
     c->h64_key[0] = t_max;
     c->h64_key[1] = cells;
+    c->h64_key[2] = factor;
   }
+  // a single target's box: r_cut below L/2 (the pairs' image rule)
+  wp.box_single = 1;
+  for (int a = 0; a < 3; ++a)
+    if (!(wp.rcut < 0.5 * wp.L[a] * (1.0 - 1.0e-9))) wp.box_single = 0;
   wp.h64_cells = cells;
   wp.h64_scale = (0.25 / (sp.a * sp.a)) / (t_max / cells);
-  wp.eps2_64 = wp.eps * wp.eps;
-  wp.c8_64 = ((0.125 / sp.a) / sp.a) / sp.a;
+  wp.eps2_64 = std::max(wp.eps * wp.eps, 1.0e-36);
 }
 
 // The mixed walks' pair arithmetic in H-table units (lengths times
@@ -918,6 +925,15 @@ void solve_device_impl(Ctx* c, const double* x, const double* y, const double* z
           wp.rcut2_tab = static_cast<float>(wp.rcut2 * scale);
           wp.eps2_tab = static_cast<float>(wp.eps * wp.eps * scale);
           wp.force_scale = static_cast<float>(wp.G * scale * (uniform ? um : 1.0));
+          // FP64 cutoff decisions up to 2^18 sources, where a pair on the wrong
+          // side of r_cut shows in the force field's relative L2 (see
+          // walkmix_box_kernel)
+          wp.exact_pairs = n <= 262144 ? 1 : 0;
+          const double unit = wp.cubic ? o->box_size[0] / 4294967296.0 : 1.0;
+          for (int a = 0; a < 3; ++a) wp.fx_to_len64[a] = o->box_size[a] / 4294967296.0;
+          wp.sep2_to_tab = scale * unit * unit;
+          wp.eps2_tab64 = wp.eps * wp.eps * scale;
+          wp.rcut2_sep64 = wp.rcut2 / (unit * unit);
           wp.log_cells = c->ltab_cells;
           wp.log_base = static_cast<uint32_t>(c->ltab_first_octave + 127) << chui::kLogCellBits;
         }

@@ -679,7 +679,7 @@ __global__ __launch_bounds__(256) void leaf_morton_kernel(const double4* __restr
 
 // ---------------------------------------------------------------------------
 // Level-synchronous node discovery on the sorted path keys (BFS numbering).
-// meta = depth | octant << 8 | leaf << 16
+// meta = depth | octant << 8 | leaf << 16 | last sibling << 17
 __device__ __forceinline__ uint32_t lower_bound_digit(const uint64_t* __restrict__ k, uint32_t b, uint32_t e,
                                                       int shift, uint32_t digit) {
   while (b < e) {
@@ -866,7 +866,7 @@ __global__ __launch_bounds__(256) void level_emit_dev_kernel(LevelDevArgs a, con
             const uint32_t ch = fc + j++;
             nb[ch] = lo;
             nc[ch] = hi - lo;
-            meta[ch] = (depth + 1u) | (o << 8);
+            meta[ch] = (depth + 1u) | (o << 8) | (j == c ? 1u << 17 : 0u);
             const double chh = 0.5 * g.w;  // tree_gravity.cpp:1180-1184
             double4 cg;
             cg.x = g.x + ((o & 4u) ? chh : -chh);
@@ -891,7 +891,7 @@ __global__ void root_init_kernel(uint32_t* nb, uint32_t* nc, uint32_t* meta, dou
                                  double cy, double cz, double h, const Frame* __restrict__ fr) {
   nb[0] = 0;
   nc[0] = n;
-  meta[0] = 0;
+  meta[0] = 1u << 17;
   geo[0] = fr ? make_double4(fr->centre[0], fr->centre[1], fr->centre[2], fr->half) : make_double4(cx, cy, cz, h);
 }
 
@@ -1198,7 +1198,7 @@ __global__ __launch_bounds__(256) void records_kernel(RecordArgs a, const uint32
                                                       NodeMom32* __restrict__ mom32,
                                                       NodeQuad32* __restrict__ quad32,
                                                       const double* __restrict__ box,
-                                                      NodeBox32* __restrict__ box32,
+                                                      NodeBox32* __restrict__ box32, WalkNode* __restrict__ wnode,
                                                       const uint32_t* __restrict__ total_dev) {
   const uint32_t total = total_dev ? *total_dev : a.total;
   for (uint32_t node = blockIdx.x * blockDim.x + threadIdx.x; node < total; node += gridDim.x * blockDim.x) {
@@ -1230,6 +1230,8 @@ __global__ __launch_bounds__(256) void records_kernel(RecordArgs a, const uint32
     quad32[p] = NodeQuad32{static_cast<float>(q[0]), static_cast<float>(q[1]), static_cast<float>(q[2]),
                            static_cast<float>(q[3]), static_cast<float>(q[4]), static_cast<float>(q[5]),
                            static_cast<float>(q[6]), static_cast<float>(q[7])};
+  }
+  if (wnode) {
     // Fixed point floors: the centre and every particle move by less than one
     // unit each, so two units on top of the half-extent keep every particle's
     // fixed-point position inside the box.
@@ -1250,7 +1252,10 @@ __global__ __launch_bounds__(256) void records_kernel(RecordArgs a, const uint32
     r.hz = hf[2];
     r.cell_half = static_cast<float>(g.w);
     r.pad = 0u;
-    box32[p] = r;
+    if (box32) box32[p] = r;
+    wnode[node] = WalkNode{r.cx, r.cy, r.cz, r.hx, r.hy, r.hz, r.cell_half,
+                           c | ((meta[node] >> 17) & 1u ? kLastSibling : 0u), c == 0 ? nb[node] : first_child[node],
+                           nc[node], p, subtree[node]};
   }
   }
 }
@@ -1498,6 +1503,9 @@ void launch_records(Tree& t, bool fp64, bool mixed, hipStream_t s) {
     t.quad64.reserve(nsz * sizeof(NodeQuad64));
     t.child_index.reserve(nsz * 8 * sizeof(uint32_t));
   }
+  // the walk records go with the build's own records, not with a later
+  // ensure_records64
+  const bool walk_nodes = mixed || !t.wnodes_current;
   RecordArgs ra{};
   ra.total = static_cast<uint32_t>(total);
   ra.fp64 = fp64 ? 1 : 0;
@@ -1511,9 +1519,11 @@ void launch_records(Tree& t, bool fp64, bool mixed, hipStream_t s) {
       t.link.as<NodeLink>(), fp64 ? t.geo64.as<NodeGeo64>() : nullptr, fp64 ? t.mom64.as<NodeMom64>() : nullptr,
       fp64 ? t.quad64.as<NodeQuad64>() : nullptr, fp64 ? t.child_index.as<uint32_t>() : nullptr,
       mixed ? t.geo32.as<NodeGeo32>() : nullptr, mixed ? t.mom32.as<NodeMom32>() : nullptr,
-      mixed ? t.quad32.as<NodeQuad32>() : nullptr, mixed ? t.bfs_box.as<double>() : nullptr,
-      mixed ? t.box32.as<NodeBox32>() : nullptr, device_node_count(t));
+      mixed ? t.quad32.as<NodeQuad32>() : nullptr, t.bfs_box.as<double>(),
+      mixed ? t.box32.as<NodeBox32>() : nullptr, walk_nodes ? t.wnode.as<WalkNode>() : nullptr,
+      device_node_count(t));
   CHUI_LAUNCH_CHECK("records_kernel");
+  t.wnodes_current = true;
   if (fp64) t.records64 = true;
 }
 
@@ -1815,7 +1825,9 @@ void build_tree(Tree& t, const double* x, const double* y, const double* z, cons
     t.quad32.reserve(nsz * sizeof(NodeQuad32));
     t.box32.reserve(nsz * sizeof(NodeBox32));
   }
+  t.wnode.reserve((nsz + kWalkNodePad) * sizeof(WalkNode));
   t.records64 = false;
+  t.wnodes_current = false;
   t.cubic = (P.L[0] == P.L[1] && P.L[0] == P.L[2]);
   for (int a = 0; a < 3; ++a) t.fscale[a] = 4294967296.0 / P.L[a];
   launch_records(t, !P.mixed, P.mixed, s);

@@ -36,6 +36,20 @@ struct alignas(32) NodeQuad32 { float qxx, qxy, qxz, qyy, qyz, qzz, trace, offse
 // size in length units.
 struct alignas(32) NodeBox32 { uint32_t cx, cy, cz; float hx, hy, hz, cell_half; uint32_t pad; };
 
+// Breadth-first record of the box-classified walks: a node's children are
+// consecutive, so a wave tests eight children of eight nodes with one load.
+// Tight particle box as in NodeBox32; kids = child count (0 for a leaf), with
+// kLastSibling set on the last child of its parent; first = first tree-order
+// particle (leaf) or the breadth-first index of the first child; pre, skip =
+// preorder index and subtree size (the lane-by-lane walks).
+struct alignas(16) WalkNode {
+  uint32_t cx, cy, cz;
+  float hx, hy, hz, cell_half;
+  uint32_t kids, first, count, pre, skip;
+};
+constexpr uint32_t kLastSibling = 0x100u;
+constexpr uint32_t kWalkNodePad = 8;  // records readable past the last node
+
 struct UnwrapResult {
   double anchor[3];
   double umin[3], umax[3];
@@ -98,6 +112,8 @@ struct Tree {
   // preorder node level
   DeviceBuffer link, geo64, mom64, quad64, child_index;  // child_index: uint32[8*nodes]
   DeviceBuffer geo32, mom32, quad32, box32;
+  DeviceBuffer wnode;      // WalkNode[nodes + kWalkNodePad], breadth first
+  bool wnodes_current = false;  // wnode belongs to the last built tree
   bool records64 = false;  // geo64, mom64, quad64 and child_index are current
   bool cubic = false;      // equal axes: the mixed records' separation unit is fixed point
   double fscale[3] = {0, 0, 0};  // 2^32 / L per axis

@@ -610,12 +610,19 @@ __device__ void interp32(const WalkParams& P, const float* __restrict__ fx, cons
     }
 }
 
-// XCD-aware block order: the dispatcher sends block b to XCD b % 8; give each
-// XCD a contiguous range of target chunks so neighbouring targets share an L2.
+// XCD-aware block order: the dispatcher sends block b to XCD b % 8; each XCD
+// takes runs of kXcdChunk consecutive target chunks, so neighbouring targets
+// share an L2 and the dense regions spread over the XCDs (one contiguous
+// eighth per XCD left the XCDs unevenly loaded: the 256^3 mixed walk took 20.7
+// ms so, 18.6 ms in runs of 4, 18.8 of 16 and 19.1 of 64).
+constexpr uint32_t kXcdChunk = 4;
 __device__ __forceinline__ uint32_t xcd_logical_block() {
+  constexpr uint32_t C = kXcdChunk;
   const uint32_t nb = gridDim.x, b = blockIdx.x;
-  const uint32_t q = nb / 8, r = nb % 8, x = b % 8;
-  return x * q + (x < r ? x : r) + b / 8;
+  const uint32_t full = nb / (8 * C) * (8 * C);
+  if (b >= full) return b;
+  const uint32_t x = b % 8, j = b / 8;
+  return ((j / C) * 8 + x) * C + j % C;
 }
 
 __device__ __forceinline__ void flush_counters(unsigned long long* counters, const uint32_t* c) {
@@ -765,8 +772,6 @@ struct WalkData {
   const double2* h64tab;
   // mixed timed walk: residual cells indexed by the float bits of r^2 + eps^2
   const float4* ltab;
-  // preorder index of each node's child per octant (kInvalid for none)
-  const uint32_t* child;
   // force VJP with accepted nodes: per preorder node U (3) and V (7)
   // accumulators, and the (target tree position << 32 | node) list
   double* vjp_node_acc;
@@ -776,6 +781,8 @@ struct WalkData {
   // after a capture-safe build the node count is on the device (P.node_count
   // is then the capacity); the mixed walks bound their traversal with it
   const uint32_t* node_count_dev;
+  // breadth-first records of the box-classified walks
+  const WalkNode* wnode;
 };
 
 // splitmix64 finaliser of the pair (target row, source row): the pair-set
@@ -1660,17 +1667,11 @@ constexpr int kPairGroup = 2;  // box walk: table reads in flight together
 // Hermite cells of relative width 1/32 to 1/64 keep F within 1.5e-7 of its
 // value.
 //
-// The box walk stages the sources of its kept leaves 64 at a time and drops
-// those farther than r_cut from the target box (they would all land in the
-// zero cell) before they enter the LDS window: the kept records are compacted
-// with a ballot and a lane prefix count, and the window is evaluated whenever
-// 64 records are in it.
-
 // 16-byte cell `cell` of an LDS table at LDS address `base`: the address is
 // one shift-add (the compiler folds a constant shift of a shifted value into
 // shift, and, add). Inline asm counts as convergent, so a loop holding it is
-// unrolled only with a constant trip count: the box walk's full windows use
-// it, the lane-by-lane walk (variable leaf counts) indexes the table plainly.
+// unrolled only with a constant trip count: the box walk's windows use it
+// (groups of kPairGroup), the lane-by-lane walk indexes the table plainly.
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 using lds_f32x4 = __attribute__((address_space(3))) const f32x4;
 __device__ __forceinline__ float4 lds_cell(uint32_t base, uint32_t cell) {
@@ -1680,39 +1681,26 @@ __device__ __forceinline__ float4 lds_cell(uint32_t base, uint32_t cell) {
   return make_float4(v.x, v.y, v.z, v.w);
 }
 
-// The box walk's last, partial window has a variable trip count, so its pair
-// loop stays rolled (see lds_cell); the unroller's warning about it is muted.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Wpass-failed"
-// DEVN: the traversal bound is the node count on the device (after a
-// capture-safe build); otherwise the kernel argument, which the timed walk
-// keeps (reading the bound from memory cost it 1 ms of 22 at 256^3).
-template <int SCHEME, bool CUBIC, bool COUNT, bool BOX = false, bool LOG = false, int WAVES = kWalkWaves,
-          bool DEVN = false>
-__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(COUNT ? 4 : 7)))
+// The counting walk (diagnostics, counters, the nearest-pair lane): lane by
+// lane, one pair kernel with the reciprocal square root and the Gaussian table.
+template <int SCHEME, bool CUBIC>
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4)))
 void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long long* __restrict__ counters,
                     const NodeLink* __restrict__ node_link, const NodeGeo32* __restrict__ node_geo,
                     const NodeMom32* __restrict__ node_mom, const NodeQuad32* __restrict__ node_quad,
                     const NodeBox32* __restrict__ node_box) {
   // node records are read-only for the kernel's lifetime and indexed by the
   // wave-uniform node number, so they come through the scalar cache
-  // the box walk's window holds up to 127 compacted records between evaluations
-  __shared__ float4 win[WAVES][BOX ? 2 * kWindow : kWindow];
-  __shared__ float4 htab[LOG ? 1 : kHTableCells];
-  __shared__ uint32_t list[WAVES][BOX ? kWindow : 1];  // box walk: listed source indices
+  __shared__ float4 win[kWalkWaves][kWindow];
+  __shared__ float4 htab[kHTableCells];
   // per lane: force totals [0..2] and their Kahan compensations [3..5]
-  __shared__ float ksum[WAVES][6][kWave];
-  extern __shared__ float4 ltab[];  // LOG: P.log_cells cells
-  if constexpr (LOG) {
-    for (int i = threadIdx.x; i < static_cast<int>(P.log_cells); i += (WAVES * kWave)) ltab[i] = D.ltab[i];
-  } else {
-    for (int i = threadIdx.x; i < kHTableCells; i += (WAVES * kWave)) htab[i] = D.htab[i];
-  }
+  __shared__ float ksum[kWalkWaves][6][kWave];
+  for (int i = threadIdx.x; i < kHTableCells; i += kWalkThreads) htab[i] = D.htab[i];
   __syncthreads();
-  const uint32_t node_count = DEVN ? *D.node_count_dev : P.node_count;
+  const uint32_t node_count = P.node_count;
   const int w = threadIdx.x / kWave;
   const int lane = threadIdx.x % kWave;
-  const uint32_t k = xcd_logical_block() * (WAVES * kWave) + threadIdx.x;
+  const uint32_t k = xcd_logical_block() * kWalkThreads + threadIdx.x;
   const bool valid = k < P.n_targets;
   const uint32_t tp = valid ? (P.identity_targets ? k : D.tpos[k]) : 0u;
   const uint32_t slot = valid ? (P.identity_targets ? D.order[k] : D.tslot[k]) : 0u;
@@ -1745,11 +1733,8 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
   // wave origin: centre of the valid targets' bounding box in fixed point
   uint32_t org[3];
   bool near = true;
-  float box_half[3];  // the box's half-extents, separation units (covers every target)
-  float box_tab[3];   // the same in table units
   {
     const uint32_t pp[3] = {px, py, pz};
-    const float sa[3] = {s0, s1, s2};
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
       const uint32_t o0 = readlane_u32(pp[a], 0);
@@ -1761,8 +1746,6 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
       org[a] = o0 + static_cast<uint32_t>(static_cast<int32_t>(mid));
       const int64_t half_extent = (static_cast<int64_t>(hi) - static_cast<int64_t>(lo)) / 2 + 1;
       near = near && half_extent <= static_cast<int64_t>(P.fast_half_extent[a]);
-      box_half[a] = static_cast<float>(half_extent + 1) * sa[a];
-      box_tab[a] = static_cast<float>(half_extent + 1) * P.tab_scale[a];
     }
   }
   const uint32_t ox = org[0], oy = org[1], oz = org[2];
@@ -1806,98 +1789,41 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
     accumulate(psx * gm, psy * gm, psz * gm);
     psx = psy = psz = 0.0f;
     pend = 0;
-    if (COUNT && lane == 0) ++cnt[7];
+    if (lane == 0) ++cnt[7];
   };
 
   // the residual pair kernel against the cn staged sources; UMASS: every
-  // source has the uniform mass, which the force scale already carries; SEL:
-  // lanes may carry a negative cutoff (they pruned the leaf or accepted an
-  // ancestor), so their terms are dropped explicitly
-  // LOG: cell (bits of s) >> 18 of the table is lcell[cell], at LDS address
-  // lbase + 16 * cell
-  const float4* const lcell = ltab - P.log_base;
-  const uint32_t lbase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_f32x4*)ltab - P.log_base));
-  auto pairs = [&]<bool NEAR, bool UMASS, bool SEL = true>(uint32_t c0, uint32_t cn, float lim) {
+  // source has the uniform mass, which the force scale already carries; lanes
+  // with a negative cutoff (they pruned the leaf or accepted an ancestor) drop
+  // their terms
+  auto pairs = [&]<bool NEAR, bool UMASS>(uint32_t c0, uint32_t cn, float lim) {
     float lx = 0.0f, ly = 0.0f, lz = 0.0f;
 #pragma unroll 4
     for (uint32_t si = 0; si < cn; ++si) {
       const float4 sj = win[w][si];
       float dx, dy, dz;
       separation.template operator()<NEAR>(sj, dx, dy, dz);
-      float f;
-      if constexpr (LOG) {
-        // s = r^2 + eps^2 clamped to [0, 1]: s >= eps^2 >= 2^first_octave, and
-        // s = 1 (r_cut and beyond) is the zero cell
-        const float sc = __builtin_amdgcn_fmed3f(fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2))), 0.0f, 1.0f);
-        const uint32_t bits = __float_as_uint(sc);
-        float4 c;
-        if constexpr (SEL) c = lcell[bits >> kLogMantissaShift];
-        else c = lds_cell(lbase, bits >> kLogMantissaShift);
-        const float u = static_cast<float>(bits & ((1u << kLogMantissaShift) - 1u));
-        float fr = fmaf(fmaf(fmaf(c.w, u, c.z), u, c.y), u, c.x);
-        if constexpr (!UMASS) fr *= sj.w;
-        f = (SEL && lim < 0.0f) ? 0.0f : fr;
-      } else {
-        const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));  // = table coordinate
-        const float rinv = __builtin_amdgcn_rsqf(r2 + eps2);
-        const float soft = rinv * rinv * rinv;
-        const int ci = static_cast<int>(fminf(r2, static_cast<float>(kHTableCells - 1)));
-        const float fu = __builtin_amdgcn_fractf(r2);
-        const float4 c = htab[ci];
-        const float hcoef = fmaf(fmaf(fmaf(c.w, fu, c.z), fu, c.y), fu, c.x);
-        float fr = fmaf(-hcoef, c8, soft);
-        if constexpr (!UMASS) fr *= sj.w;
-        // The target itself has r2 == 0 exactly (same fixed-point value), as
-        // does any coincident source: its term is exactly zero (dx = dy = dz = 0
-        // against a finite softened value), so no self test is needed. The
-        // counting variant counts coincident sources as the reference does.
-        const bool pair = r2 <= lim;
-        if constexpr (COUNT) {
-          const bool distinct = pair && (r2 != 0.0f || (c0 + si) != tp);
-          cnt[2] += distinct;
-          nearest = distinct ? fminf(nearest, r2) : nearest;
-        }
-        f = pair ? fr : 0.0f;
-      }
+      const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));  // = table coordinate
+      const float rinv = __builtin_amdgcn_rsqf(r2 + eps2);
+      const float soft = rinv * rinv * rinv;
+      const int ci = static_cast<int>(fminf(r2, static_cast<float>(kHTableCells - 1)));
+      const float fu = __builtin_amdgcn_fractf(r2);
+      const float4 c = htab[ci];
+      const float hcoef = fmaf(fmaf(fmaf(c.w, fu, c.z), fu, c.y), fu, c.x);
+      float fr = fmaf(-hcoef, c8, soft);
+      if constexpr (!UMASS) fr *= sj.w;
+      // The target itself has r2 == 0 exactly (same fixed-point value), as
+      // does any coincident source: its term is exactly zero (dx = dy = dz = 0
+      // against a finite softened value). Coincident sources are counted as
+      // the reference does.
+      const bool pair = r2 <= lim;
+      const bool distinct = pair && (r2 != 0.0f || (c0 + si) != tp);
+      cnt[2] += distinct;
+      nearest = distinct ? fminf(nearest, r2) : nearest;
+      const float f = pair ? fr : 0.0f;
       lx = fmaf(f, dx, lx);
       ly = fmaf(f, dy, ly);
       lz = fmaf(f, dz, lz);
-    }
-    psx += lx;
-    psy += ly;
-    psz += lz;
-  };
-  // A full window of the box walk (LOG): sources in groups of kPairGroup whose
-  // table reads are in flight together before their polynomials are evaluated.
-  auto window_pairs = [&]<bool UMASS>() {
-    constexpr int G = kPairGroup;
-    float lx = 0.0f, ly = 0.0f, lz = 0.0f;
-#pragma unroll 2
-    for (int s0 = 0; s0 < kWindow; s0 += G) {
-      float dx[G], dy[G], dz[G], mj[G];
-      uint32_t bits[G];
-      float4 c[G];
-#pragma unroll
-      for (int k = 0; k < G; ++k) {
-        const float4 sj = win[w][s0 + k];
-        dx[k] = sj.x - tx;
-        dy[k] = sj.y - ty;
-        dz[k] = sj.z - tz;
-        mj[k] = sj.w;
-        bits[k] = __float_as_uint(
-            __builtin_amdgcn_fmed3f(fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], fmaf(dz[k], dz[k], eps2))), 0.0f, 1.0f));
-      }
-#pragma unroll
-      for (int k = 0; k < G; ++k) c[k] = lds_cell(lbase, bits[k] >> kLogMantissaShift);
-#pragma unroll
-      for (int k = 0; k < G; ++k) {
-        const float u = static_cast<float>(bits[k] & ((1u << kLogMantissaShift) - 1u));
-        float fr = fmaf(fmaf(fmaf(c[k].w, u, c[k].z), u, c[k].y), u, c[k].x);
-        if constexpr (!UMASS) fr *= mj[k];
-        lx = fmaf(fr, dx[k], lx);
-        ly = fmaf(fr, dy[k], ly);
-        lz = fmaf(fr, dz[k], lz);
-      }
     }
     psx += lx;
     psy += ly;
@@ -1921,7 +1847,7 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
   auto walk = [&]<bool NEAR>(uint32_t end) {
     uint32_t n = wave_min_u32(nxt);
     while (n < end) {
-      if (COUNT && lane == 0) ++cnt[5];
+      if (lane == 0) ++cnt[5];
       const NodeLink lk = node_link[n];
       const NodeBox32 b = node_box[n];
       const bool act = nxt == n;
@@ -1942,7 +1868,7 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
           const uint32_t e0 = lk.begin + lk.count;
           for (uint32_t c0 = lk.begin; c0 < e0; c0 += kWindow) {
             const uint32_t cn = e0 - c0 < static_cast<uint32_t>(kWindow) ? e0 - c0 : static_cast<uint32_t>(kWindow);
-            if (COUNT && lane == 0) cnt[6] += cn;
+            if (lane == 0) cnt[6] += cn;
             if (pend + cn > static_cast<uint32_t>(kWindow)) fold();
             pend += cn;
             {
@@ -1977,171 +1903,13 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
     }
   };
 
-  // Box classification of node q against the wave's target box: 0 pruned,
-  // 1 kept leaf (sources [lb, lb + lc)), 3 opened, 4 a subtree some lane may
-  // accept a multipole in (walked lane by lane); next is q + 1 to descend,
-  // q + skip to move past the subtree.
-  auto box_classify = [&](uint32_t q, uint32_t& next, uint32_t& lb, uint32_t& lc, uint32_t& span,
-                          uint32_t& nchild) -> int {
-    const NodeLink lk = node_link[q];
-    const NodeBox32 b = node_box[q];
-    span = lk.skip;
-    nchild = lk.child_count;
-    const float ex = fmaxf(0.0f, fabsf(fx_delta(b.cx, ox, s0)) - b.hx - box_half[0]);
-    const float ey = fmaxf(0.0f, fabsf(fx_delta(b.cy, oy, s1)) - b.hy - box_half[1]);
-    const float ez = fmaxf(0.0f, fabsf(fx_delta(b.cz, oz, s2)) - b.hz - box_half[2]);
-    const bool keep = !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > prune2);
-    if (lk.child_count == 0) {
-      lb = lk.begin;
-      lc = lk.count;
-      return keep ? 1 : 0;
-    }
-    if (!keep) {
-      next = q + lk.skip;
-      return 0;
-    }
-    if (b.cell_half < P.accept_half_max) {
-      // every target within 25 h of the COM fails 2h/r < 0.08
-      const NodeMom32 M = node_mom[q];
-      const float dx = (fabsf(fx_delta(M.comx, ox, s0)) + box_half[0]) * to_len;
-      const float dy = (fabsf(fx_delta(M.comy, oy, s1)) + box_half[1]) * to_len;
-      const float dz = (fabsf(fx_delta(M.comz, oz, s2)) + box_half[2]) * to_len;
-      const float far2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-      if (!(far2 <= 624.9f * b.cell_half * b.cell_half)) {
-        next = q + lk.skip;
-        return 4;
-      }
-    }
-    return 3;
-  };
-
-  auto box_walk = [&]() {
-    const float lim = valid ? rc2 : -1.0f;
-    // a source whose offset from the box centre lies beyond r_cut of the box
-    // (outside half-extent + 1 fixed-point unit per axis) is beyond r_cut of
-    // every target; the 1e-5 margin covers the rounding of the offsets, so
-    // every dropped source is one whose s reaches the zero cell
-    const float cull2 = rc2 * 1.00001f;
-    uint32_t nl = 0;            // list[w][0, nl): listed sources, staged 64 at a time
-    uint32_t wn = 0;            // compacted records in win[w][0, wn)
-    auto evaluate = [&](uint32_t cn) {
-      __builtin_amdgcn_wave_barrier();
-      if (pend + cn > static_cast<uint32_t>(kWindow)) fold();
-      pend += cn;
-      // every lane sums every staged source (pairs beyond r_cut are zero);
-      // lanes without a target are never written out
-      if (LOG && cn == static_cast<uint32_t>(kWindow)) {
-        if (D.uniform_mass) window_pairs.template operator()<true>();
-        else window_pairs.template operator()<false>();
-      } else if (D.uniform_mass) {
-        pairs.template operator()<true, true, false>(0, cn, lim);
-      } else {
-        pairs.template operator()<true, false, false>(0, cn, lim);
-      }
-      __builtin_amdgcn_wave_barrier();
-    };
-    // stage the next cn listed sources, keep those within r_cut of the box
-    auto eval_window = [&](uint32_t cn) {
-      __builtin_amdgcn_wave_barrier();
-      const bool on = static_cast<uint32_t>(lane) < cn;
-      const uint4 sv = D.src32[list[w][on ? lane : 0]];
-      const float mj = D.uniform_mass ? 1.0f : __uint_as_float(sv.w);
-      const float4 rec = stage_record.template operator()<true>(sv, mj);
-      const float ex = fmaxf(fabsf(rec.x) - box_tab[0], 0.0f);
-      const float ey = fmaxf(fabsf(rec.y) - box_tab[1], 0.0f);
-      const float ez = fmaxf(fabsf(rec.z) - box_tab[2], 0.0f);
-      const bool keep = on && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > cull2);
-      const unsigned long long km = __ballot(keep);
-      const uint32_t at =
-          wn + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(km >> 32),
-                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(km), 0u));
-      if (keep) win[w][at] = rec;
-      wn += static_cast<uint32_t>(__popcll(km));
-      nl = 0;
-      if (wn >= static_cast<uint32_t>(kWindow)) {
-        evaluate(kWindow);
-        wn -= kWindow;
-        // wn < 64: move the records past the window to its front
-        if (static_cast<uint32_t>(lane) < wn) {
-          const float4 t = win[w][kWindow + lane];
-          win[w][lane] = t;
-        }
-      }
-    };
-    // the lanes' classified nodes: kept leaves' sources go to the list (a
-    // leaf may continue in the next batch), subtrees some lane may accept in
-    // are walked lane by lane
-    auto take = [&](bool on, int kind, uint32_t q, uint32_t lb, uint32_t lc, uint32_t next) {
-      unsigned long long rest = __ballot(on && kind == 1);
-      while (rest) {
-        const uint32_t l = static_cast<uint32_t>(__ffsll(static_cast<long long>(rest)) - 1);
-        rest &= rest - 1ull;
-        const uint32_t b0 = readlane_u32(lb, l), c = readlane_u32(lc, l);
-        for (uint32_t c0 = 0; c0 < c;) {
-          // nl < kWindow here: fill the list up to kWindow entries
-          const uint32_t room = static_cast<uint32_t>(kWindow) - nl;
-          const uint32_t cn = c - c0 < room ? c - c0 : room;
-          if (static_cast<uint32_t>(lane) < cn) list[w][nl + lane] = b0 + c0 + lane;
-          nl += cn;
-          c0 += cn;
-          if (nl == static_cast<uint32_t>(kWindow)) eval_window(kWindow);
-        }
-      }
-      unsigned long long sub = __ballot(on && kind == 4);
-      while (sub) {
-        const uint32_t l = static_cast<uint32_t>(__ffsll(static_cast<long long>(sub)) - 1);
-        sub &= sub - 1ull;
-        const uint32_t q4 = readlane_u32(q, l), end = readlane_u32(next, l);
-        // the lane-by-lane walk stages its leaves in the window's front
-        if (wn) {
-          evaluate(wn);
-          wn = 0;
-        }
-        nxt = valid ? q4 : end;
-        walk.template operator()<true>(end);
-      }
-    };
-    // windows of 64 consecutive preorder nodes of [start, end), following the
-    // visited chain through each window
-    auto chain_walk = [&](uint32_t start, uint32_t end) {
-      uint32_t p = start;
-      while (p < end) {
-        const uint32_t q = p + lane;
-        uint32_t next = q + 1, lb = 0, lc = 0, span = 1, nch = 0;
-        const int kind = q < end ? box_classify(q, next, lb, lc, span, nch) : 3;
-        unsigned long long chain = 0;
-        uint32_t cur = p;
-        while (cur < p + kWave && cur < end) {
-          const uint32_t l = cur - p;
-          chain |= 1ull << l;
-          cur = readlane_u32(next, l);
-        }
-        p = cur;
-        take((chain >> lane) & 1ull, kind, q, lb, lc, next);
-      }
-    };
-    chain_walk(0, node_count);
-    if (nl) eval_window(nl);
-    if (wn) evaluate(wn);
-  };
-
-  bool boxed = false;
-  if constexpr (BOX) {
-    boxed = near && box_half[0] <= P.box_half_max[0] && box_half[1] <= P.box_half_max[1] &&
-            box_half[2] <= P.box_half_max[2];
-  }
-  if (boxed) {
-    if constexpr (BOX) box_walk();
-  } else if (near) {
-    walk.template operator()<true>(node_count);
-  } else {
-    walk.template operator()<false>(node_count);
-  }
+  if (near) walk.template operator()<true>(node_count);
+  else walk.template operator()<false>(node_count);
   fold();
 
-  // Diagnostic launches also replay the reference's walk over the octree
+  // Replay the reference's walk over the octree
   // cells (no pair work) for its per-target node counters.
-  if constexpr (COUNT) {
+  {
     uint32_t cnxt = valid ? 0u : node_count;
     uint32_t n = wave_min_u32(cnxt);
     while (n < node_count) {
@@ -2174,7 +1942,7 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
     }
   }
 
-  if (COUNT) flush_counters(counters, cnt);
+  flush_counters(counters, cnt);
   if (!valid) return;
   const float ax = ksum[w][0][lane] - ksum[w][3][lane];
   const float ay = ksum[w][1][lane] - ksum[w][4][lane];
@@ -2193,10 +1961,655 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
     static_cast<float*>(out.sr_y)[row] = ay;
     static_cast<float*>(out.sr_z)[row] = az;
   }
-  if (COUNT && out.near2) static_cast<float*>(out.near2)[row] = nearest * P.tab_to_len2;
+  if (out.near2) static_cast<float*>(out.near2)[row] = nearest * P.tab_to_len2;
 }
 
-#pragma clang diagnostic pop
+
+// ---- box-classified traversal -----------------------------------------------------
+// The timed strict walks traverse the tree once per segment of consecutive
+// visit-ordered targets, against the segment's target box. A segment is a
+// power-of-two run of T targets inside a wave's targets: the whole run when
+// its box fits (half-extents up to box_half_max), else halves of it, down to
+// single targets, so a run that straddles a jump of the space-filling curve
+// costs two or three compact traversals instead of a lane-by-lane walk of the
+// union of distant neighbourhoods. The 64 lanes are T targets times 64 / T
+// source slices: every lane sums its slice of the staged sources for its
+// target, and the slices are added at the end. Small target sets launch fewer
+// targets per wave, so that they still fill the chip.
+//
+// Traversal: breadth-first records (WalkNode) keep a node's children
+// consecutive. The wave pops eight opened nodes from an LDS stack and its
+// lanes test their children with one load each; kept children are pushed,
+// kept leaves listed. A 256^3 walk visits about 500 nodes per wave, which
+// took one dependent load and a scalar chain for each of some 100 windows of
+// consecutive preorder nodes (11 of the walk's 24 ms); eight nodes per step
+// take 15 to 20 loads. The stack pops one node per step above kBoxWide
+// entries, so it never holds more than kBoxWide + 56 + 7 * 21 + 8 entries.
+//
+// Listed leaves are expanded 64 sources at a time: the leaves' source counts
+// are scanned across the lanes, each leaf marks its first slot of the batch,
+// and a running maximum spreads the leaf over its slots. The next batch's
+// records are in flight while the current one is culled and evaluated.
+constexpr uint32_t kBoxGroup = 16;     // targets per evaluation group: a DPP row
+constexpr uint32_t kBoxWindow = 128;   // records staged between evaluations
+constexpr uint32_t kBoxList = 80;      // 64 records in up to 16 slices, one slot of padding each (LDS banks)
+constexpr float kBoxCompact = 0.3f;    // half-extent in r_cut up to which a segment stays one group
+constexpr int kBoxWide = 96;
+constexpr int kBoxStack = kBoxWide + 56 + 7 * 21 + 13;
+
+struct BoxLds {
+  uint32_t stack[kBoxStack];
+  uint32_t leaf[2 * kWave];
+  uint32_t mark[kWave];
+};
+
+// Target box of a segment in fixed point: centre, half-extents in separation
+// units (they cover every target's fixed-point position), the node tests'
+// scales and cutoffs.
+struct BoxFrame {
+  uint32_t ox, oy, oz;
+  float hx, hy, hz;
+  float s0, s1, s2;
+  float prune2;
+  float accept_half_max;  // no acceptance for cells of this half size or more (length)
+  float to_len;
+};
+
+// inclusive sum / maximum over the lanes up to this one (all 64 active)
+__device__ __forceinline__ uint32_t wave_scan_sum(uint32_t v) {
+  v += CHUI_DPP(v, 0x111, 0xf, 0u);  // row_shr:1
+  v += CHUI_DPP(v, 0x112, 0xf, 0u);  // row_shr:2
+  v += CHUI_DPP(v, 0x114, 0xf, 0u);  // row_shr:4
+  v += CHUI_DPP(v, 0x118, 0xf, 0u);  // row_shr:8
+  v += CHUI_DPP(v, 0x142, 0xa, 0u);  // row_bcast:15
+  v += CHUI_DPP(v, 0x143, 0xc, 0u);  // row_bcast:31
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_scan_max(uint32_t v) {
+  v = dpp_max_step(v, CHUI_DPP(v, 0x111, 0xf, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x112, 0xf, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x114, 0xf, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x118, 0xf, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x142, 0xa, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x143, 0xc, 0u));
+  return v;
+}
+// centre and half-extent of v over this lane's row of 16 lanes (all active);
+// the half-extent covers the rounding of the centre
+__device__ __forceinline__ void row_bounds(float v, float& centre, float& half) {
+  auto step = [](float x, uint32_t y, bool mx) {
+    const float o = __uint_as_float(y);
+    return mx ? fmaxf(x, o) : fminf(x, o);
+  };
+#define CHUI_ROW(ctrl)                                                                                          \
+  {                                                                                                             \
+    const uint32_t a_ = __float_as_uint(lo), b_ = __float_as_uint(hi);                                          \
+    lo = step(lo, CHUI_DPP(a_, ctrl, 0xf, a_), false);                                                          \
+    hi = step(hi, CHUI_DPP(b_, ctrl, 0xf, b_), true);                                                           \
+  }
+  float lo = v, hi = v;
+  CHUI_ROW(0x121)  // row_ror:1
+  CHUI_ROW(0x122)  // row_ror:2
+  CHUI_ROW(0x124)  // row_ror:4
+  CHUI_ROW(0x128)  // row_ror:8
+#undef CHUI_ROW
+  centre = 0.5f * (lo + hi);
+  half = fmaxf(hi - centre, centre - lo);
+}
+__device__ __forceinline__ uint32_t lanes_below(unsigned long long m) {
+  return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
+}
+
+// Walks the tree (breadth-first records nodes, root 0) for one box. Wave-
+// uniform control flow throughout.
+//   load(j)        the source record of tree position j (any valid j)
+//   take(rec, on, last)  one batch of up to 64 records, `on` marking the lanes
+//                  with one; last: no batch follows
+//   candidate(pre, end)  an internal node [pre, end) in preorder that some
+//                  target may accept: true when no target does (it is opened
+//                  like any node), false when the callee has walked it
+template <class Load, class Take, class Candidate>
+__device__ __forceinline__ void box_traverse(const WalkNode* __restrict__ nodes, BoxLds& s, int lane,
+                                             const BoxFrame& F, Load&& load, Take&& take, Candidate&& candidate) {
+  const uint4* const raw = reinterpret_cast<const uint4*>(nodes);
+  uint32_t sp = 0, nleaf = 0;
+  // sources of the last m listed leaves; last: no leaf is left and none will come
+  auto drain = [&](uint32_t m, bool last) {
+    nleaf -= m;
+    __builtin_amdgcn_wave_barrier();
+    uint32_t begin = 0, count = 0;
+    if (static_cast<uint32_t>(lane) < m) {
+      const WalkNode& q = nodes[s.leaf[nleaf + lane]];
+      begin = q.first;
+      count = q.count;
+    }
+    const uint32_t incl = wave_scan_sum(count);
+    const uint32_t excl = incl - count;
+    const uint32_t total = readlane_u32(incl, kWave - 1);
+    const uint32_t shift = begin - excl;
+    uint32_t carry = 0;
+    auto index = [&](uint32_t base) -> uint32_t {
+      s.mark[lane] = 0;
+      __builtin_amdgcn_wave_barrier();
+      if (count && excl - base < static_cast<uint32_t>(kWave)) s.mark[excl - base] = static_cast<uint32_t>(lane);
+      __builtin_amdgcn_wave_barrier();
+      uint32_t v = s.mark[lane];
+      __builtin_amdgcn_wave_barrier();
+      if (lane == 0) v = v > carry ? v : carry;
+      v = wave_scan_max(v);
+      carry = readlane_u32(v, kWave - 1);
+      const uint32_t j = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>(v << 2),
+                                                                            static_cast<int>(shift))) + base + lane;
+      const uint32_t j0 = readlane_u32(j, 0);
+      return base + lane < total ? j : j0;
+    };
+    auto cur = load(index(0));  // leaves are never empty: total > 0
+    for (uint32_t base = 0; base < total; base += kWave) {
+      const bool more = base + kWave < total;
+      auto nxt = cur;
+      if (more) nxt = load(index(base + kWave));
+      take(cur, base + lane < total, last && !more);
+      cur = nxt;
+    }
+  };
+  // children of the top entries: lane group g = lane / 8 takes entry sp - 1 - g
+  uint4 a, b, c;
+  uint32_t idx = 0;
+  bool in = false;
+  auto pop = [&]() {
+    const uint32_t m = sp > static_cast<uint32_t>(kBoxWide) ? 1u : (sp < 8u ? sp : 8u);
+    const uint32_t g = static_cast<uint32_t>(lane) >> 3;
+    __builtin_amdgcn_wave_barrier();
+    in = g < m;
+    idx = s.stack[sp - 1 - (in ? g : 0u)] + (lane & 7u);
+    sp -= m;
+    const uint4* r = raw + 3ull * idx;
+    a = r[0];
+    b = r[1];
+    c = r[2];
+  };
+  if (lane == 0) s.stack[0] = 0;
+  sp = 1;
+  pop();
+  bool open = true;  // a, b, c hold popped nodes
+  do {
+    if (open) {
+      // a: cx cy cz hx | b: hy hz cell_half kids | c: first count pre skip
+      const uint32_t kids = b.w;
+      const uint32_t lastbits =
+          static_cast<uint32_t>(__ballot(in && (kids & kLastSibling)) >> (lane & 56)) & 0xFFu;
+      const bool on = in && !(lastbits & ((1u << (lane & 7)) - 1u));  // no last sibling before this lane
+      const float ex = fmaxf(0.0f, fabsf(fx_delta(a.x, F.ox, F.s0)) - __uint_as_float(a.w) - F.hx);
+      const float ey = fmaxf(0.0f, fabsf(fx_delta(a.y, F.oy, F.s1)) - __uint_as_float(b.x) - F.hy);
+      const float ez = fmaxf(0.0f, fabsf(fx_delta(a.z, F.oz, F.s2)) - __uint_as_float(b.y) - F.hz);
+      const bool keep = on && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > F.prune2);
+      const bool leaf = (kids & 0xFFu) == 0;
+      bool cand = false;
+      if (keep && !leaf) {
+        const float h = __uint_as_float(b.z);
+        if (h < F.accept_half_max) {
+          // a target within 25 h of the node fails 2h/r < 0.08: no candidate
+          // when the whole box (and the node's own extent) lies within 25 h
+          const float dx = (fabsf(fx_delta(a.x, F.ox, F.s0)) + __uint_as_float(a.w) + F.hx) * F.to_len;
+          const float dy = (fabsf(fx_delta(a.y, F.oy, F.s1)) + __uint_as_float(b.x) + F.hy) * F.to_len;
+          const float dz = (fabsf(fx_delta(a.z, F.oz, F.s2)) + __uint_as_float(b.y) + F.hz) * F.to_len;
+          cand = !(fmaf(dx, dx, fmaf(dy, dy, dz * dz)) <= 624.9f * h * h);
+        }
+      }
+      const unsigned long long lm = __ballot(keep && leaf);
+      if (keep && leaf) s.leaf[nleaf + lanes_below(lm)] = idx;
+      nleaf += static_cast<uint32_t>(__popcll(lm));
+      const unsigned long long om = __ballot(keep && !leaf && !cand);
+      if (keep && !leaf && !cand) s.stack[sp + lanes_below(om)] = c.x;
+      sp += static_cast<uint32_t>(__popcll(om));
+      unsigned long long rest = __ballot(cand);
+      while (rest) {
+        const uint32_t l = static_cast<uint32_t>(__ffsll(static_cast<long long>(rest)) - 1);
+        rest &= rest - 1ull;
+        // the lane reads come before any branch on the lane: an inactive
+        // lane's register may hold nothing (a spilled value is reloaded for
+        // the active lanes only)
+        const uint32_t pre = readlane_u32(c.z, l), end = pre + readlane_u32(c.w, l), child = readlane_u32(c.x, l);
+        if (candidate(pre, end)) {
+          if (lane == 0) s.stack[sp] = child;
+          ++sp;
+        }
+      }
+      open = sp != 0;
+      if (open) pop();  // the next nodes' loads are in flight while leaves are drained
+    }
+    // one leaf stays listed while nodes are open, so the last drain comes last
+    if (nleaf > static_cast<uint32_t>(kWave) || (!open && nleaf)) {
+      const uint32_t m = nleaf < static_cast<uint32_t>(kWave) ? nleaf : static_cast<uint32_t>(kWave);
+      drain(m, !open && m == nleaf);
+    }
+  } while (open || nleaf);
+}
+
+// Bounds of a segment [seg, seg + T) of the wave's targets: halves T until
+// fits() accepts the run (a single target always fits). Wave-uniform.
+template <class Fits>
+__device__ __forceinline__ uint32_t box_segment(uint32_t seg, uint32_t per_wave, Fits&& fits) {
+  uint32_t T = seg ? (seg & (0u - seg)) : per_wave;
+  while (!fits(T) && T > 1) T >>= 1;
+  return T;
+}
+
+// ---- mixed box walk ----------------------------------------------------------------
+// The timed mixed walk: fused PM interpolation and the residual walk of the
+// comment above walkmix_kernel, box-classified. Staged sources farther than
+// r_cut from the target box (all their pairs are zero) are dropped; the rest
+// are compacted into an LDS window and evaluated 64 at a time. Window slot of
+// record r for S = 64 / TL slices: (r % S) (TL + 1) + r / S, so a lane's TL
+// records are consecutive and the slices start in different LDS banks. The
+// second half of the window takes a batch's overflow and stages the leaves of
+// the lane-by-lane walks.
+//
+// EXACT (few sources): the pairs keep the sources' and targets' fixed-point
+// coordinates, and r^2 and its cutoff are evaluated in FP64. In FP32 a pair
+// within about 1e-7 of r_cut may fall on either side of it, and the residual
+// is still 1.8e-2 of Newtonian there: about one pair in 2.6e7 does, one per
+// 64^3 box, which moves a 32^3 box's force field by 2e-6 in relative L2 (2.5e-7
+// otherwise) when it happens. The FP64 form takes 27 VALU instructions per
+// pair against 16.
+template <int SCHEME, bool CUBIC, bool LOG, int WAVES, bool FRAME, bool EXACT>
+__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(5)))
+void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long long* __restrict__ counters,
+                        const NodeLink* __restrict__ node_link, const NodeGeo32* __restrict__ node_geo,
+                        const NodeMom32* __restrict__ node_mom, const NodeQuad32* __restrict__ node_quad,
+                        const NodeBox32* __restrict__ node_box, const WalkNode* __restrict__ wnode) {
+  __shared__ float4 win_all[WAVES][2 * kBoxList];
+  __shared__ BoxLds box_all[WAVES];
+  __shared__ float4 htab[LOG ? 1 : kHTableCells];
+  extern __shared__ float4 ltab[];  // LOG: P.log_cells cells
+  if constexpr (LOG) {
+    for (int i = threadIdx.x; i < static_cast<int>(P.log_cells); i += (WAVES * kWave)) ltab[i] = D.ltab[i];
+  } else {
+    for (int i = threadIdx.x; i < kHTableCells; i += (WAVES * kWave)) htab[i] = D.htab[i];
+  }
+  __syncthreads();
+  const uint32_t node_count = D.node_count_dev ? *D.node_count_dev : P.node_count;
+  const int w = static_cast<int>(readlane_u32(threadIdx.x / kWave, 0));
+  const int lane = threadIdx.x % kWave;
+  float4* const win = win_all[w];
+  BoxLds& lds = box_all[w];
+  const uint32_t per_wave = P.targets_per_wave;
+  const uint64_t k64 = (static_cast<uint64_t>(xcd_logical_block()) * WAVES + w) * per_wave;
+  if (k64 >= P.n_targets || node_count == 0) return;
+  const uint32_t k0 = static_cast<uint32_t>(k64);
+  const uint32_t here = P.n_targets - k0 < per_wave ? P.n_targets - k0 : per_wave;  // targets of this wave
+  // node tests: fixed-point units (CUBIC) or lengths
+  const float s0 = CUBIC ? 1.0f : P.fx_to_len[0];
+  const float s1 = CUBIC ? 1.0f : P.fx_to_len[1];
+  const float s2 = CUBIC ? 1.0f : P.fx_to_len[2];
+  const float to_len = CUBIC ? P.fx_to_len[0] : 1.0f;          // node separation unit -> length
+  const float inv_len = CUBIC ? 1.0f / P.fx_to_len[0] : 1.0f;  // length -> node separation unit
+  const float prune2 = P.prune2_sep;
+  // pairs: table units (lengths * sqrt(t_to_cell), or of the residual table)
+  const float u0 = P.tab_scale[0], u1 = P.tab_scale[1], u2 = P.tab_scale[2];
+  const float rc2 = P.rcut2_tab;
+  const float eps2 = P.eps2_tab;
+  const float c8 = P.c8_tab;
+  const MixFrame F{s0, s1, s2, to_len, inv_len, P.contain2_sep, static_cast<float>(P.theta * P.theta)};
+  const float4* const lcell = ltab - P.log_base;
+  const uint32_t lbase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_f32x4*)ltab - P.log_base));
+
+  for (uint32_t seg = 0; seg < here;) {
+    // --- the segment and its box ---
+    uint32_t px, py, pz;
+    uint32_t ox = 0, oy = 0, oz = 0;
+    float bh0 = 0.0f, bh1 = 0.0f, bh2 = 0.0f;  // half-extents, separation units
+    float bt0 = 0.0f, bt1 = 0.0f, bt2 = 0.0f;  // the same in table units
+    uint32_t T;
+    if constexpr (!FRAME) {
+      T = per_wave;
+    } else {
+      // lane i: target seg + i (the last valid one past the end)
+      const uint32_t i = seg + lane < here ? seg + lane : here - 1;
+      const uint4 t = D.src32[P.identity_targets ? k0 + i : D.tpos[k0 + i]];
+      T = box_segment(seg, per_wave, [&](uint32_t want) -> bool {
+        const bool in = static_cast<uint32_t>(lane) < want;
+        const uint32_t pp[3] = {t.x, t.y, t.z};
+        const float sa[3] = {s0, s1, s2};
+        uint32_t o[3];
+        float bh[3], bt[3];
+        bool ok = true;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const uint32_t o0 = readlane_u32(pp[a], 0);
+          // offsets from the first target, ordered as unsigned
+          const uint32_t off = in ? (pp[a] - o0) ^ 0x80000000u : 0x80000000u;
+          const int32_t lo = static_cast<int32_t>(wave_min_u32(off) ^ 0x80000000u);
+          const int32_t hi = static_cast<int32_t>(wave_max_u32(off) ^ 0x80000000u);
+          const int64_t mid = (static_cast<int64_t>(lo) + static_cast<int64_t>(hi)) / 2;
+          o[a] = o0 + static_cast<uint32_t>(static_cast<int32_t>(mid));
+          const int64_t half = (static_cast<int64_t>(hi) - static_cast<int64_t>(lo)) / 2 + 1;
+          bh[a] = static_cast<float>(half + 1) * sa[a];
+          bt[a] = static_cast<float>(half + 1) * P.tab_scale[a];
+          ok = ok && half <= static_cast<int64_t>(P.fast_half_extent[a]) && bh[a] <= P.box_half_max[a];
+        }
+        ox = o[0]; oy = o[1]; oz = o[2];
+        bh0 = bh[0]; bh1 = bh[1]; bh2 = bh[2];
+        bt0 = bt[0]; bt1 = bt[1]; bt2 = bt[2];
+        return ok;
+      });
+    }
+    // T targets as TL columns (at least 4) and 64 / TL source slices
+    const uint32_t TL = T < 4u ? 4u : T;
+    const uint32_t lgT = 31u - static_cast<uint32_t>(__builtin_clz(TL));
+    const uint32_t lgS = 6u - lgT;
+    const uint32_t col = static_cast<uint32_t>(lane) & (TL - 1u), slice = static_cast<uint32_t>(lane) >> lgT;
+    const bool valid = col < T && seg + col < here;
+    const uint32_t k = k0 + seg + (valid ? col : 0u);
+    const uint32_t tp = P.identity_targets ? k : D.tpos[k];
+    {
+      const uint4 t = D.src32[tp];
+      px = t.x;
+      py = t.y;
+      pz = t.z;
+    }
+    const float tx = fx_delta(px, ox, u0), ty = fx_delta(py, oy, u1), tz = fx_delta(pz, oz, u2);
+    float sum[3] = {0.0f, 0.0f, 0.0f}, comp[3] = {0.0f, 0.0f, 0.0f};  // Kahan totals of this lane's slice
+    auto accumulate = [&](float vx, float vy, float vz) {
+      kahan_add(sum[0], comp[0], vx);
+      kahan_add(sum[1], comp[1], vy);
+      kahan_add(sum[2], comp[2], vz);
+    };
+    uint32_t pend = 0;                         // sources in this lane's partial sums (wave-uniform)
+    float psx = 0.0f, psy = 0.0f, psz = 0.0f;  // partial pair sums since the last fold
+    auto fold = [&]() {
+      const float gm = P.force_scale;
+      accumulate(psx * gm, psy * gm, psz * gm);
+      psx = psy = psz = 0.0f;
+      pend = 0;
+    };
+    auto stage_record = [&]<bool NEAR>(const uint4& sv, float mj) -> float4 {
+      if constexpr (NEAR && !EXACT)
+        return make_float4(fx_delta(sv.x, ox, u0), fx_delta(sv.y, oy, u1), fx_delta(sv.z, oz, u2), mj);
+      else
+        return make_float4(__uint_as_float(sv.x), __uint_as_float(sv.y), __uint_as_float(sv.z), mj);
+    };
+    // EXACT: s of a fixed-point record, 1 beyond r_cut and below 1 inside it
+    auto exact_s = [&](const float4& sj) -> float {
+      double dx = static_cast<double>(static_cast<int32_t>(__float_as_uint(sj.x) - px));
+      double dy = static_cast<double>(static_cast<int32_t>(__float_as_uint(sj.y) - py));
+      double dz = static_cast<double>(static_cast<int32_t>(__float_as_uint(sj.z) - pz));
+      if constexpr (!CUBIC) {
+        dx *= P.fx_to_len64[0];
+        dy *= P.fx_to_len64[1];
+        dz *= P.fx_to_len64[2];
+      }
+      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+      const float sv = fminf(static_cast<float>(fma(r2, P.sep2_to_tab, P.eps2_tab64)), 0.99999994f);
+      return r2 <= P.rcut2_sep64 ? sv : 1.0f;
+    };
+    // One pair term; NEAR: offsets from the box centre, else fixed point.
+    // UMASS: the force scale carries the mass. SEL: lanes with a negative
+    // cutoff drop the term.
+    auto pair = [&]<bool NEAR, bool UMASS, bool SEL>(const float4& sj, float lim, float& lx, float& ly, float& lz) {
+      float dx, dy, dz;
+      if constexpr (NEAR && !EXACT) {
+        dx = sj.x - tx;
+        dy = sj.y - ty;
+        dz = sj.z - tz;
+      } else {
+        dx = fx_delta(__float_as_uint(sj.x), px, u0);
+        dy = fx_delta(__float_as_uint(sj.y), py, u1);
+        dz = fx_delta(__float_as_uint(sj.z), pz, u2);
+      }
+      float f;
+      if constexpr (LOG) {
+        // s = r^2 + eps^2 clamped to [0, 1]: s >= eps^2 >= 2^first_octave, and
+        // s = 1 (r_cut and beyond) is the zero cell
+        float sc = __builtin_amdgcn_fmed3f(fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2))), 0.0f, 1.0f);
+        if constexpr (EXACT) sc = exact_s(sj);
+        const uint32_t bits = __float_as_uint(sc);
+        const float4 c = lcell[bits >> kLogMantissaShift];
+        const float u = static_cast<float>(bits & ((1u << kLogMantissaShift) - 1u));
+        float fr = fmaf(fmaf(fmaf(c.w, u, c.z), u, c.y), u, c.x);
+        if constexpr (!UMASS) fr *= sj.w;
+        f = (SEL && lim < 0.0f) ? 0.0f : fr;
+      } else {
+        const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));  // = table coordinate
+        const float rinv = __builtin_amdgcn_rsqf(r2 + eps2);
+        const float soft = rinv * rinv * rinv;
+        const int ci = static_cast<int>(fminf(r2, static_cast<float>(kHTableCells - 1)));
+        const float fu = __builtin_amdgcn_fractf(r2);
+        const float4 c = htab[ci];
+        const float hcoef = fmaf(fmaf(fmaf(c.w, fu, c.z), fu, c.y), fu, c.x);
+        float fr = fmaf(-hcoef, c8, soft);
+        if constexpr (!UMASS) fr *= sj.w;
+        // the target itself (and any coincident source) has r2 == 0 exactly:
+        // zero separation against a finite softened value
+        f = r2 <= lim ? fr : 0.0f;
+      }
+      lx = fmaf(f, dx, lx);
+      ly = fmaf(f, dy, ly);
+      lz = fmaf(f, dz, lz);
+    };
+    // the cn leaf sources staged in the second half (lane-by-lane walks)
+    auto leaf_pairs = [&]<bool NEAR, bool UMASS>(uint32_t cn, float lim) {
+      float lx = 0.0f, ly = 0.0f, lz = 0.0f;
+#pragma unroll 2
+      for (uint32_t si = 0; si < cn; ++si)
+        pair.template operator()<NEAR, UMASS, true>(win[kBoxList + si], lim, lx, ly, lz);
+      psx += lx;
+      psy += ly;
+      psz += lz;
+    };
+    // Strict acceptance of internal node n for this lane, with the COM
+    // separation it needs left in mf*.
+    auto accepts = [&](uint32_t n, const NodeGeo32& g, float& mfx, float& mfy, float& mfz) -> bool {
+      return strict_accept32(P, F, g, node_mom[n], node_quad, n, px, py, pz, mfx, mfy, mfz);
+    };
+    // Lane-by-lane walk of the preorder range [nxt, end) (walkmix_kernel's
+    // walk): candidate subtrees, and whole walks without a box frame.
+    uint32_t nxt = 0;
+    auto walk = [&]<bool NEAR>(uint32_t end) {
+      uint32_t n = wave_min_u32(nxt);
+      while (n < end) {
+        const NodeLink lk = node_link[n];
+        const NodeBox32 b = node_box[n];
+        const bool act = nxt == n;
+        if (!__ballot(act)) {
+          if (lane == 0) atomicOr(&counters[kFaultSlot], 1ull);
+          break;
+        }
+        const float ax_ = fabsf(fx_delta(b.cx, px, s0)), ay_ = fabsf(fx_delta(b.cy, py, s1)),
+                    az_ = fabsf(fx_delta(b.cz, pz, s2));
+        const float ex = fmaxf(0.0f, ax_ - b.hx), ey = fmaxf(0.0f, ay_ - b.hy), ez = fmaxf(0.0f, az_ - b.hz);
+        const bool keep = act && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > prune2);
+        if (lk.child_count == 0) {
+          // a leaf's subtree is itself: every waiting lane moves on to n + 1,
+          // so that is the wave's next node too
+          nxt = act ? n + 1 : nxt;
+          if (__ballot(keep)) {
+            const float lim = keep ? rc2 : -1.0f;
+            const uint32_t e0 = lk.begin + lk.count;
+            for (uint32_t c0 = lk.begin; c0 < e0; c0 += kWindow) {
+              const uint32_t cn = e0 - c0 < static_cast<uint32_t>(kWindow) ? e0 - c0 : static_cast<uint32_t>(kWindow);
+              if (pend + cn > static_cast<uint32_t>(kWindow)) fold();
+              pend += cn;
+              const uint4 sv = D.src32[c0 + (static_cast<uint32_t>(lane) < cn ? lane : 0)];
+              const float mj = D.uniform_mass ? 1.0f : __uint_as_float(sv.w);
+              if (static_cast<uint32_t>(lane) < cn)
+                win[kBoxList + lane] = stage_record.template operator()<NEAR>(sv, mj);
+              __builtin_amdgcn_wave_barrier();
+              if (D.uniform_mass) leaf_pairs.template operator()<NEAR, true>(cn, lim);
+              else leaf_pairs.template operator()<NEAR, false>(cn, lim);
+              __builtin_amdgcn_wave_barrier();
+            }
+          }
+          ++n;
+          continue;
+        }
+        nxt = (act && !keep) ? n + lk.skip : nxt;
+        if (__ballot(keep)) {
+          bool take_mp = false;
+          float mfx = 0.0f, mfy = 0.0f, mfz = 0.0f;
+          if (b.cell_half < P.accept_half_max) {
+            if (keep) take_mp = accepts(n, node_geo[n], mfx, mfy, mfz);
+          }
+          if (keep) nxt = take_mp ? n + lk.skip : n + 1;
+          if (__ballot(take_mp) && take_mp) {
+            float cx = 0.0f, cy = 0.0f, cz = 0.0f;
+            node_accel32(node_mom[n], node_quad[n], mfx, mfy, mfz, P, cx, cy, cz);
+            accumulate(cx, cy, cz);
+          }
+        }
+        n = next_node(n, nxt);
+      }
+    };
+    const bool owner = valid && slice == 0;  // the lane-by-lane walks run on the first slice
+    if constexpr (FRAME) {
+      // a source whose offset from the box centre lies beyond r_cut of the box
+      // (outside half-extent + 1 fixed-point unit per axis) is beyond r_cut of
+      // every target; the 1e-5 margin covers the rounding of the offsets, so
+      // every dropped source is one whose pairs are all zero
+      const float cull2 = rc2 * 1.00001f;
+      uint32_t wn = 0;  // records in the window, below kWindow between batches
+      const float4* const mine = win + slice * (TL + 1u);
+      // iters records of every slice (a multiple of 4)
+      auto window_pairs = [&]<bool UMASS>(uint32_t iters) {
+        float lx = 0.0f, ly = 0.0f, lz = 0.0f;
+        if constexpr (LOG) {
+          // two table reads in flight before their polynomials are evaluated
+          for (uint32_t i0 = 0; i0 < iters; i0 += 4) {
+#pragma unroll
+            for (int h = 0; h < 4; h += kPairGroup) {
+              float dx[kPairGroup], dy[kPairGroup], dz[kPairGroup], mj[kPairGroup];
+              uint32_t bits[kPairGroup];
+              float4 c[kPairGroup];
+#pragma unroll
+              for (int q = 0; q < kPairGroup; ++q) {
+                const float4 sj = mine[i0 + h + q];
+                mj[q] = sj.w;
+                if constexpr (EXACT) {
+                  dx[q] = fx_delta(__float_as_uint(sj.x), px, u0);
+                  dy[q] = fx_delta(__float_as_uint(sj.y), py, u1);
+                  dz[q] = fx_delta(__float_as_uint(sj.z), pz, u2);
+                  bits[q] = __float_as_uint(exact_s(sj));
+                  continue;
+                }
+                dx[q] = sj.x - tx;
+                dy[q] = sj.y - ty;
+                dz[q] = sj.z - tz;
+                bits[q] = __float_as_uint(__builtin_amdgcn_fmed3f(
+                    fmaf(dx[q], dx[q], fmaf(dy[q], dy[q], fmaf(dz[q], dz[q], eps2))), 0.0f, 1.0f));
+              }
+#pragma unroll
+              for (int q = 0; q < kPairGroup; ++q) c[q] = lds_cell(lbase, bits[q] >> kLogMantissaShift);
+#pragma unroll
+              for (int q = 0; q < kPairGroup; ++q) {
+                const float u = static_cast<float>(bits[q] & ((1u << kLogMantissaShift) - 1u));
+                float fr = fmaf(fmaf(fmaf(c[q].w, u, c[q].z), u, c[q].y), u, c[q].x);
+                if constexpr (!UMASS) fr *= mj[q];
+                lx = fmaf(fr, dx[q], lx);
+                ly = fmaf(fr, dy[q], ly);
+                lz = fmaf(fr, dz[q], lz);
+              }
+            }
+          }
+        } else {
+#pragma unroll 4
+          for (uint32_t i0 = 0; i0 < iters; ++i0)
+            pair.template operator()<true, UMASS, false>(mine[i0], rc2, lx, ly, lz);
+        }
+        psx += lx;
+        psy += ly;
+        psz += lz;
+      };
+      // every lane sums its slice of the first cn records (pairs beyond r_cut
+      // are zero; lanes without a target are never written out)
+      auto evaluate = [&](uint32_t cn) {
+        __builtin_amdgcn_wave_barrier();
+        const uint32_t iters = (((cn + (1u << lgS) - 1u) >> lgS) + 3u) & ~3u;
+        if (pend + iters > static_cast<uint32_t>(kWindow)) fold();
+        pend += iters;
+        if (D.uniform_mass) window_pairs.template operator()<true>(iters);
+        else window_pairs.template operator()<false>(iters);
+        __builtin_amdgcn_wave_barrier();
+      };
+      auto slot_of = [&](uint32_t r) -> uint32_t {
+        const uint32_t q = r & (kWindow - 1u);
+        return (r >= static_cast<uint32_t>(kWindow) ? kBoxList : 0u) + (q & ((1u << lgS) - 1u)) * (TL + 1u) + (q >> lgS);
+      };
+      const BoxFrame frame{ox, oy, oz, bh0, bh1, bh2, s0, s1, s2, prune2, P.quad ? P.accept_half_max : 0.0f, to_len};
+      box_traverse(
+          wnode, lds, lane, frame, [&](uint32_t j) -> uint4 { return D.src32[j]; },
+          [&](const uint4& sv, bool on, bool last) {
+            const float mj = D.uniform_mass ? 1.0f : __uint_as_float(sv.w);
+            const float4 rec = stage_record.template operator()<true>(sv, mj);
+            const float ex = fmaxf(fabsf(EXACT ? fx_delta(sv.x, ox, u0) : rec.x) - bt0, 0.0f);
+            const float ey = fmaxf(fabsf(EXACT ? fx_delta(sv.y, oy, u1) : rec.y) - bt1, 0.0f);
+            const float ez = fmaxf(fabsf(EXACT ? fx_delta(sv.z, oz, u2) : rec.z) - bt2, 0.0f);
+            const bool keep = on && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > cull2);
+            const unsigned long long km = __ballot(keep);
+            __builtin_amdgcn_wave_barrier();
+            if (keep) win[slot_of(wn + lanes_below(km))] = rec;
+            wn += static_cast<uint32_t>(__popcll(km));
+            while (wn >= static_cast<uint32_t>(kWindow) || (last && wn)) {
+              const uint32_t cn = wn < static_cast<uint32_t>(kWindow) ? wn : static_cast<uint32_t>(kWindow);
+              if (static_cast<uint32_t>(lane) >= cn) {
+                // dummies beyond r_cut of everything fill the last window
+                // (EXACT: half a period from the box centre per axis)
+                const float far = 64.0f * sqrtf(rc2);
+                win[slot_of(lane)] = EXACT ? make_float4(__uint_as_float(ox ^ 0x80000000u),
+                                                         __uint_as_float(oy ^ 0x80000000u),
+                                                         __uint_as_float(oz ^ 0x80000000u), 0.0f)
+                                           : make_float4(far, far, far, 0.0f);
+              }
+              evaluate(cn);
+              wn -= cn;
+              // the records past the window move to its front, same slots
+              const uint32_t at = slot_of(lane);
+              win[at] = win[kBoxList + at];
+            }
+          },
+          [&](uint32_t pre, uint32_t end) -> bool {
+            float mx, my, mz;
+            if (!__ballot(owner && accepts(pre, node_geo[pre], mx, my, mz))) return true;
+            nxt = owner ? pre : end;
+            walk.template operator()<true>(end);
+            return false;
+          });
+    } else {
+      nxt = owner ? 0u : node_count;
+      walk.template operator()<false>(node_count);
+    }
+    fold();
+    // --- slices -> targets ---
+    double tot[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) tot[a] = static_cast<double>(sum[a]) - static_cast<double>(comp[a]);
+    for (uint32_t o = TL; o < static_cast<uint32_t>(kWave); o <<= 1) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) tot[a] += __shfl_xor(tot[a], static_cast<int>(o), kWave);
+    }
+    if (owner) {
+      const float ax = static_cast<float>(tot[0]), ay = static_cast<float>(tot[1]), az = static_cast<float>(tot[2]);
+      float gx = 0.0f, gy = 0.0f, gz = 0.0f;
+      if (P.pm_enabled) interp32<SCHEME>(P, D.f32x, D.f32y, D.f32z, px, py, pz, gx, gy, gz);
+      const uint32_t row = D.order[tp];
+      const uint32_t slot = P.identity_targets ? row : D.tslot[k];
+      static_cast<float*>(out.ax)[slot] = gx + ax;
+      static_cast<float*>(out.ay)[slot] = gy + ay;
+      static_cast<float*>(out.az)[slot] = gz + az;
+      if (out.pm_x) {
+        static_cast<float*>(out.pm_x)[slot] = gx;
+        static_cast<float*>(out.pm_y)[slot] = gy;
+        static_cast<float*>(out.pm_z)[slot] = gz;
+      }
+      if (out.sr_x) {
+        static_cast<float*>(out.sr_x)[row] = ax;
+        static_cast<float*>(out.sr_y)[row] = ay;
+        static_cast<float*>(out.sr_z)[row] = az;
+      }
+    }
+    seg += T;
+  }
+}
 
 // ---- mixed walk, one target per wave --------------------------------------------
 // For sparse active sets the 64 targets of a walkmix_kernel wave lie far
@@ -2475,73 +2888,56 @@ __global__ __launch_bounds__(kWalkThreads) void walk64_target_kernel(WalkParams 
 }
 
 // ---- FP64 strict walk, box-classified (the timed FP64 path) ----------------------
-// walkmix_kernel's box-classified traversal in FP64 for solves without
-// counters: a wave whose 64 targets lie in a box of half-extent at most 2 r_cut
-// (and below L/2 - r_cut, so that every pair inside r_cut has its minimum
-// image relative to the box centre) classifies 64 preorder nodes at a time
-// against the box (octree cells beyond r_cut of the box are pruned; internal
-// nodes that no target can accept are opened), lists the kept leaves'
-// sources in an LDS ring and evaluates them one 64-source window at a time;
-// subtrees some target may accept as a multipole (cells with h < 0.041 r_cut
-// farther than 25 h from some target) and waves that do not fit a box are
-// walked lane by lane with walk64_kernel's tests (cell prune, accept64,
-// node_accel64). Pair term: (r^2 + eps^2)^{-3/2} from v_rsq_f64 and two Newton
-// steps, L(r)/r^3 = H(r^2 / 4a^2) / 8a^3 from a degree-5 polynomial per cell
-// of an LDS table (Chebyshev interpolation, error below 1e-14 of H), in FP64
-// throughout. The pairs and multipoles are walk64_kernel's; the pair
-// arithmetic and the summation order differ at the round-off level.
+// The box-classified traversal in FP64 for solves without counters and for
+// the force VJP. Staged sources beyond r_cut of the segment's box are dropped,
+// the rest fill an LDS window of kBoxWindow records (half that in the JVP,
+// which also stages lam). A full window is evaluated group by group:
+// kBoxGroup consecutive targets of the segment, whose own box drops the
+// window's records again (the kept ones are copied to a list of 64) and whose
+// pairs all 64 lanes share, as 64 / kBoxGroup source slices. In the evenly
+// filled parts of a box the 64 targets of a segment span more than r_cut and a
+// record reaches few of them: groups of 16 cut the pair slots per 64 targets
+// from 1171 to 674 at 96^3 (10% in halos; counted on a CPU model of the walk).
+// An FP64 pair costs enough for that to pay (96^3: 3.27 ms without groups,
+// 2.97 with; the VJP of 64^3 3.10 against 2.75 ms); a mixed pair does not
+// (256^3: 18.2 against 21.9 ms). Segments whose box is small against r_cut
+// (kBoxCompact) stay one group. List slot of record r for S slices of TL
+// records: (r % S) (TL + 1) + r / S, so a lane's records are consecutive and
+// the slices start in different LDS banks. Subtrees some target may accept as
+// a multipole are walked lane by lane with walk64_kernel's tests (cell prune,
+// accept64, node_accel64). The pairs and multipoles are walk64_kernel's; the
+// pair arithmetic and the summation order differ at the round-off level.
 constexpr int kH64Cells = kH64MaxCells;
-
-// s^{-1/2} for s in [1e-30, 1e30]: the FP32 reciprocal square root (about
-// 2^-23 relative) refined by two Newton steps in FP64 (error squared each
-// step), so the result is within an ulp or two of FP64.
-__device__ __forceinline__ double rsq64(double s) {
-  double y = static_cast<double>(__builtin_amdgcn_rsqf(static_cast<float>(s)));
-  double e = fma(-s * y, y, 1.0);
-  y = fma(0.5 * y, e, y);
-  e = fma(-s * y, y, 1.0);
-  return fma(0.5 * y, e, y);
-}
 
 // JVP: the transpose of the acceleration Jacobian applied to lam, as in
 // walk64_kernel<..., JVP> (pair term G (F w + 2 F'(t) (r . w) r), w = m_k
-// lam_j - m_j lam_k, with F' = dF/d(r^2) from the same table), for
-// multipole_order 0 (no accepted nodes).
-template <int SCHEME, bool JVP = false>
-__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4))) void walk64_box_kernel(
+// lam_j - m_j lam_k, with F' = dF/d(r^2) from the same table); accepted nodes
+// add their Jacobian terms and are listed for vjp_node_corrections.
+template <int SCHEME, bool JVP, bool FRAME>
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(JVP ? 2 : 3))) void walk64_box_kernel(
     WalkParams P, WalkData D, WalkOutputs out, unsigned long long* __restrict__ counters) {
-  // forward: the box walk's window holds up to 127 compacted records
-  __shared__ double4 win[kWalkWaves][JVP ? kWindow : 2 * kWindow];
-  __shared__ double4 winl[JVP ? kWalkWaves : 1][JVP ? kWindow : 1];  // JVP: lam of the staged sources
-  __shared__ uint32_t list[kWalkWaves][kWindow];                       // box walk: listed source indices
-  __shared__ double2 htab[3 * kH64Cells];
-  for (int i = threadIdx.x; i < 3 * P.h64_cells; i += kWalkThreads) htab[i] = D.h64tab[i];
+  constexpr uint32_t kWin = JVP ? kBoxWindow / 2 : kBoxWindow;
+  __shared__ double4 win_all[kWalkWaves][kWin];
+  __shared__ double4 list_all[kWalkWaves][kBoxList];
+  // JVP: lam of the staged sources
+  __shared__ double4 winl_all[JVP ? kWalkWaves : 1][JVP ? kWin : 1];
+  __shared__ double4 listl_all[JVP ? kWalkWaves : 1][JVP ? kBoxList : 1];
+  __shared__ BoxLds box_all[kWalkWaves];
+  __shared__ double2 htab[3 * (kH64Cells + 1)];
+  for (int i = threadIdx.x; i < 3 * (P.h64_cells + 1); i += kWalkThreads) htab[i] = D.h64tab[i];
   __syncthreads();
   const uint32_t node_count = D.node_count_dev ? *D.node_count_dev : P.node_count;
-  const int w = threadIdx.x / kWave;
+  const int w = static_cast<int>(readlane_u32(threadIdx.x / kWave, 0));
   const int lane = threadIdx.x % kWave;
-  const uint32_t k = xcd_logical_block() * kWalkThreads + threadIdx.x;
-  const bool valid = k < P.n_targets;
-  const uint32_t tp = valid ? (P.identity_targets ? k : D.tpos[k]) : 0u;
-  const uint32_t slot = valid ? (P.identity_targets ? D.order[k] : D.tslot[k]) : 0u;
-  double px = 0.0, py = 0.0, pz = 0.0;
-  double gx = 0.0, gy = 0.0, gz = 0.0;
-  double4 lk_ = make_double4(0.0, 0.0, 0.0, 0.0);  // JVP: lam of the target
-  double mk = 0.0;                                  // JVP: mass of the target
-  if (valid) {
-    const double4 t = D.src64[tp];
-    px = t.x;
-    py = t.y;
-    pz = t.z;
-    if constexpr (JVP) {
-      lk_ = D.lam64[tp];
-      mk = D.uniform_mass ? P.uniform_mass : t.w;
-      if (P.pm_enabled)
-        vjp_gather64<SCHEME>(P, D.f64x, D.f64y, D.f64z, D.nu64, lk_.x, lk_.y, lk_.z, mk, px, py, pz, gx, gy, gz);
-    } else {
-      if (P.pm_enabled) interp64<SCHEME>(P, D.f64x, D.f64y, D.f64z, px, py, pz, gx, gy, gz);
-    }
-  }
+  double4* const win = win_all[w];
+  double4* const list = list_all[w];
+  double4* const winl = winl_all[JVP ? w : 0];
+  double4* const listl = listl_all[JVP ? w : 0];
+  const uint32_t per_wave = P.targets_per_wave;
+  const uint64_t k64 = (static_cast<uint64_t>(xcd_logical_block()) * kWalkWaves + w) * per_wave;
+  if (k64 >= P.n_targets || node_count == 0) return;
+  const uint32_t k0 = static_cast<uint32_t>(k64);
+  const uint32_t here = P.n_targets - k0 < per_wave ? P.n_targets - k0 : per_wave;  // targets of this wave
   const double L0 = P.L[0], L1 = P.L[1], L2 = P.L[2];
   const double iL0 = 1.0 / L0, iL1 = 1.0 / L1, iL2 = 1.0 / L2;
   // minimum image by a reciprocal multiply: d - L rint(d / L) up to the
@@ -2552,72 +2948,120 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4)
     const double iL = a == 0 ? iL0 : (a == 1 ? iL1 : iL2);
     return fma(-L, rint(d * iL), d);
   };
-  const double rc = P.rcut, rc2 = P.rcut2;
-  // target box: offsets from lane 0's target (lane 0 is valid whenever any lane is)
-  const double o0 = readlane_f64(px, 0), o1 = readlane_f64(py, 0), o2 = readlane_f64(pz, 0);
-  const double ux = valid ? mi_fast(px - o0, 0) : 0.0, uy = valid ? mi_fast(py - o1, 1) : 0.0,
-               uz = valid ? mi_fast(pz - o2, 2) : 0.0;
-  // wave-uniform values through readlane, so they live in scalar registers
-  const double lox = readlane_f64(wave_min(ux), 0), hix = readlane_f64(wave_max(ux), 0),
-               loy = readlane_f64(wave_min(uy), 0), hiy = readlane_f64(wave_max(uy), 0),
-               loz = readlane_f64(wave_min(uz), 0), hiz = readlane_f64(wave_max(uz), 0);
-  const double cx = 0.5 * (lox + hix), cy = 0.5 * (loy + hiy), cz = 0.5 * (loz + hiz);
-  const double ex = 0.5 * (hix - lox) * (1.0 + 1.0e-12), ey = 0.5 * (hiy - loy) * (1.0 + 1.0e-12),
-               ez = 0.5 * (hiz - loz) * (1.0 + 1.0e-12);
-  const bool any = __ballot(valid) != 0ull;
-  const double emax = 2.0 * rc;  // the mixed walk's bound on the box half-extent
-  const bool boxed = any && ex <= emax && ey <= emax && ez <= emax && ex + rc < 0.5 * L0 * (1.0 - 1.0e-9) &&
-                     ey + rc < 0.5 * L1 * (1.0 - 1.0e-9) && ez + rc < 0.5 * L2 * (1.0 - 1.0e-9);
-  // box centre in the tree frame. Boxed waves stage each source as its image
-  // nearest the box centre and take the target's image likewise: for waves
-  // away from the seam both are the tree-frame coordinates themselves (the
-  // shift is zero), so r = x_j - x_k is the reference's difference exactly.
-  const double bx = o0 + cx, by = o1 + cy, bz = o2 + cz;
   auto image = [&](double v, double b, int a) -> double {
     const double L = a == 0 ? L0 : (a == 1 ? L1 : L2);
     const double iL = a == 0 ? iL0 : (a == 1 ? iL1 : iL2);
     return fma(-L, rint((v - b) * iL), v);
   };
-  const double qx = image(px, bx, 0), qy = image(py, by, 1), qz = image(pz, bz, 2);
-  const double eps2 = P.eps2_64, c8 = P.c8_64, tscale = P.h64_scale;
-  const double cmax = static_cast<double>(P.h64_cells) - 1.0;
-  double ax = 0.0, ay = 0.0, az = 0.0;
-
-  // residual pair kernel in FP64: G m_j [(r^2+eps^2)^{-3/2} - H(r^2/4a^2)/8a^3] r_vec (G m_j applied by the
-  // caller); with the derivative fp = dF/d(r^2) when asked (JVP)
+  const double rc = P.rcut, rc2 = P.rcut2;
+  const double eps2 = P.eps2_64, tscale = P.h64_scale;
+  const uint32_t last_cell = static_cast<uint32_t>(P.h64_cells);
+  // node tests against the fixed-point tight boxes
+  const float s0 = P.cubic ? 1.0f : P.fx_to_len[0];
+  const float s1 = P.cubic ? 1.0f : P.fx_to_len[1];
+  const float s2 = P.cubic ? 1.0f : P.fx_to_len[2];
+  const float to_len = P.cubic ? P.fx_to_len[0] : 1.0f;
+  // F at r = 0 (the reference's limit: 0 without softening), for coincident pairs in the JVP
+  const double f_zero = JVP ? residual_inv_r3(0.0, P.eps, P.a) : 0.0;
+  // Residual pair kernel in FP64: G m_j [(r^2+eps^2)^{-3/2} - H(r^2/4a^2)/8a^3] r_vec
+  // (G m_j applied by the caller); with the derivative fp = dF/d(r^2) when asked (JVP).
+  // s^{-3/2} from the FP32 reciprocal square root y (whose square is exact in
+  // FP64): with e = 1 - s y^2, |e| < 2^-21, s^{-3/2} = y^3 (1 + 3/2 e + 15/8 e^2)
+  // up to e^3 < 2^-63. The cell of H is the integer nearest to r^2 tscale, read
+  // from the low word of the sum with 1.5 2^52; the cell's polynomial (-1/8a^3
+  // folded into it) runs in the offset from the cell's centre. The pair loop
+  // takes 36 VALU instructions per pair against 53 with two Newton steps and a
+  // truncated cell index.
+  constexpr double kRound = 6755399441055744.0;  // 1.5 * 2^52
   auto residual = [&](double r2, double* fp) -> double {
-    const double sft = fmax(r2 + eps2, 1.0e-30);  // coincident unsoftened pairs: finite, times a zero vector
-    const double y = rsq64(sft);
-    const double soft = y * y * y;
-    const double t = fmin(r2 * tscale, cmax + 0.999999999999);
-    const int ci = static_cast<int>(t);
-    const double u = t - static_cast<double>(ci);
+    const double s = r2 + eps2;  // eps2 > 0: coincident unsoftened pairs stay finite, times a zero vector
+    const double y = static_cast<double>(__builtin_amdgcn_rsqf(static_cast<float>(s)));
+    const double y2 = y * y;
+    const double e = fma(-s, y2, 1.0);
+    const double y3 = y2 * y;
+    const double soft = fma(y3, e * fma(1.875, e, 1.5), y3);
+    const double tm = fma(r2, tscale, kRound);
+    const uint32_t c = static_cast<uint32_t>(__double2loint(tm));
+    const uint32_t ci = c < last_cell ? c : last_cell;
+    const double u = fma(r2, tscale, kRound - tm);
     const double2 a01 = htab[3 * ci], a23 = htab[3 * ci + 1], a45 = htab[3 * ci + 2];
     const double hv = fma(fma(fma(fma(fma(a45.y, u, a45.x), u, a23.y), u, a23.x), u, a01.y), u, a01.x);
     if (fp) {
       const double dh = fma(fma(fma(fma(5.0 * a45.y, u, 4.0 * a45.x), u, 3.0 * a23.y), u, 2.0 * a23.x), u, a01.y);
-      *fp = fma(-1.5 * soft, y * y, -c8 * dh * tscale);
+      const double is = fma(y2, fma(e, e, e), y2);  // 1 / s
+      *fp = fma(-1.5 * soft, is, dh * tscale);
     }
-    return fma(-hv, c8, soft);
+    return soft + hv;
   };
-  // F at r = 0 (the reference's limit: 0 without softening), for coincident pairs in the JVP
-  const double f_zero = JVP ? residual_inv_r3(0.0, P.eps, P.a) : 0.0;
-  // the staged window against this lane's target: NEAR = images nearest the box
-  // centre (boxed waves), else tree-frame coordinates with a minimum image per pair
-  auto pairs = [&]<bool NEAR>(uint32_t cn, double lim) {
-    double lx = 0.0, ly = 0.0, lz = 0.0;
-#pragma unroll 2
-    for (uint32_t si = 0; si < cn; ++si) {
-      const double4 sj = win[w][si];
+
+  for (uint32_t seg = 0; seg < here;) {
+    // --- the segment and its box (offsets from its first target) ---
+    double bx = 0.0, by = 0.0, bz = 0.0, ex = 0.0, ey = 0.0, ez = 0.0;
+    uint32_t T;
+    if constexpr (!FRAME) {
+      T = per_wave;
+    } else {
+      const uint32_t i = seg + lane < here ? seg + lane : here - 1;
+      const double4 t = D.src64[P.identity_targets ? k0 + i : D.tpos[k0 + i]];
+      const double o0 = readlane_f64(t.x, 0), o1 = readlane_f64(t.y, 0), o2 = readlane_f64(t.z, 0);
+      const double vx = mi_fast(t.x - o0, 0), vy = mi_fast(t.y - o1, 1), vz = mi_fast(t.z - o2, 2);
+      T = box_segment(seg, per_wave, [&](uint32_t want) -> bool {
+        const bool in = static_cast<uint32_t>(lane) < want;
+        const double ux = in ? vx : 0.0, uy = in ? vy : 0.0, uz = in ? vz : 0.0;
+        // wave-uniform values through readlane, so they live in scalar registers
+        const double lox = readlane_f64(wave_min(ux), 0), hix = readlane_f64(wave_max(ux), 0),
+                     loy = readlane_f64(wave_min(uy), 0), hiy = readlane_f64(wave_max(uy), 0),
+                     loz = readlane_f64(wave_min(uz), 0), hiz = readlane_f64(wave_max(uz), 0);
+        bx = o0 + 0.5 * (lox + hix);
+        by = o1 + 0.5 * (loy + hiy);
+        bz = o2 + 0.5 * (loz + hiz);
+        ex = 0.5 * (hix - lox) * (1.0 + 1.0e-12);
+        ey = 0.5 * (hiy - loy) * (1.0 + 1.0e-12);
+        ez = 0.5 * (hiz - loz) * (1.0 + 1.0e-12);
+        return ex <= P.box_max64 && ey <= P.box_max64 && ez <= P.box_max64 && ex + rc < 0.5 * L0 * (1.0 - 1.0e-9) &&
+               ey + rc < 0.5 * L1 * (1.0 - 1.0e-9) && ez + rc < 0.5 * L2 * (1.0 - 1.0e-9);
+      });
+    }
+    const uint32_t TL = T < 4u ? 4u : T;
+    const uint32_t lgT = 31u - static_cast<uint32_t>(__builtin_clz(TL));
+    const uint32_t col = static_cast<uint32_t>(lane) & (TL - 1u), slice = static_cast<uint32_t>(lane) >> lgT;
+    const bool valid = col < T && seg + col < here;
+    const bool owner = valid && slice == 0;  // the lane-by-lane walks run on the first slice
+    const uint32_t k = k0 + seg + (valid ? col : 0u);
+    const uint32_t tp = P.identity_targets ? k : D.tpos[k];
+    double px, py, pz;
+    double4 lk_ = make_double4(0.0, 0.0, 0.0, 0.0);  // JVP: lam of the target
+    double mk = 0.0;                                  // JVP: mass of the target
+    {
+      const double4 t = D.src64[tp];
+      px = t.x;
+      py = t.y;
+      pz = t.z;
+      if constexpr (JVP) {
+        lk_ = D.lam64[tp];
+        mk = D.uniform_mass ? P.uniform_mass : t.w;
+      }
+    }
+    // Boxed segments stage each source as its image nearest the box centre and
+    // take the target's image likewise: away from the seam both are the
+    // tree-frame coordinates themselves (the shift is zero), so r = x_j - x_k
+    // is the reference's difference exactly.
+    const double qx = image(px, bx, 0), qy = image(py, by, 1), qz = image(pz, bz, 2);
+    double ax = 0.0, ay = 0.0, az = 0.0;
+    // One staged record against a target: NEAR = images nearest the box centre,
+    // else tree-frame coordinates with a minimum image per pair. tl, tm: lam
+    // and mass of the target (JVP).
+    auto pair = [&]<bool NEAR>(const double4& sj, const double4* lj_, double x, double y, double z, const double4& tl,
+                               double tm, double lim, double& lx, double& ly, double& lz) {
       double dx, dy, dz;
       if constexpr (NEAR) {
-        dx = sj.x - qx;
-        dy = sj.y - qy;
-        dz = sj.z - qz;
+        dx = sj.x - x;
+        dy = sj.y - y;
+        dz = sj.z - z;
       } else {
-        dx = mi_fast(sj.x - px, 0);
-        dy = mi_fast(sj.y - py, 1);
-        dz = mi_fast(sj.z - pz, 2);
+        dx = mi_fast(sj.x - x, 0);
+        dy = mi_fast(sj.y - y, 1);
+        dz = mi_fast(sj.z - z, 2);
       }
       const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
       if constexpr (JVP) {
@@ -2625,16 +3069,16 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4)
         double fp = 0.0;
         double f = residual(r2, &fp);
         f = r2 > 0.0 ? f : f_zero;
-        const double4 lj = winl[w][si];
+        const double4 lj = *lj_;
         double wx, wy, wz;
         if (D.uniform_mass) {  // w / m (the mass goes into the final scale)
-          wx = lj.x - lk_.x;
-          wy = lj.y - lk_.y;
-          wz = lj.z - lk_.z;
+          wx = lj.x - tl.x;
+          wy = lj.y - tl.y;
+          wz = lj.z - tl.z;
         } else {
-          wx = mk * lj.x - sj.w * lk_.x;
-          wy = mk * lj.y - sj.w * lk_.y;
-          wz = mk * lj.z - sj.w * lk_.z;
+          wx = tm * lj.x - sj.w * tl.x;
+          wy = tm * lj.y - sj.w * tl.y;
+          wz = tm * lj.z - sj.w * tl.z;
         }
         const bool in = r2 <= lim;
         f = in ? f : 0.0;
@@ -2650,63 +3094,60 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4)
         ly = fma(f, dy, ly);
         lz = fma(f, dz, lz);
       }
-    }
+    };
     const double gm = D.uniform_mass ? P.G * P.uniform_mass : P.G;
-    ax = fma(gm, lx, ax);
-    ay = fma(gm, ly, ay);
-    az = fma(gm, lz, az);
-  };
-  auto stage = [&]<bool NEAR>(uint32_t j, bool on) {
-    const double4 sv = D.src64[j];
-    if constexpr (JVP) {
-      const double4 lv = D.lam64[j];
-      if (on) winl[w][lane] = lv;
-    }
-    if (on) {
-      if constexpr (NEAR)
-        win[w][lane] = make_double4(image(sv.x, bx, 0), image(sv.y, by, 1), image(sv.z, bz, 2), sv.w);
-      else
-        win[w][lane] = sv;
-    }
-  };
+    // the n leaf sources staged in the list (lane-by-lane walks; the list is
+    // free between evaluations)
+    auto leaf_pairs = [&]<bool NEAR>(uint32_t n, double lim) {
+      double lx = 0.0, ly = 0.0, lz = 0.0;
+      const double x = NEAR ? qx : px, y = NEAR ? qy : py, z = NEAR ? qz : pz;
+      for (uint32_t si = 0; si < n; ++si)
+        pair.template operator()<NEAR>(list[si], listl + (JVP ? si : 0u), x, y, z, lk_, mk, lim, lx, ly, lz);
+      ax = fma(gm, lx, ax);
+      ay = fma(gm, ly, ay);
+      az = fma(gm, lz, az);
+    };
 
-  // lane-by-lane walk of [nxt, end) with walk64_kernel's tests
-  uint32_t nxt = valid ? 0u : node_count;
-  auto walk = [&]<bool NEAR>(uint32_t end) {
-    uint32_t n = wave_min_u32(nxt);
-    while (n < end) {
-      const NodeLink lk = D.link[n];
-      const NodeGeo64 g = D.geo64[n];
-      const bool act = nxt == n;
-      if (!__ballot(act)) {
-        if (lane == 0) atomicOr(&counters[kFaultSlot], 1ull);
-        break;
-      }
-      const double h = g.half;
-      const double ndx = mi_fast(g.cx - px, 0), ndy = mi_fast(g.cy - py, 1), ndz = mi_fast(g.cz - pz, 2);
-      const double ax_ = fabs(ndx), ay_ = fabs(ndy), az_ = fabs(ndz);
-      const double fx_ = fmax(0.0, ax_ - h), fy_ = fmax(0.0, ay_ - h), fz_ = fmax(0.0, az_ - h);
-      const bool keep = act && within_cutoff(fx_ * fx_ + fy_ * fy_ + fz_ * fz_, P.rcut, P.rcut2);
-      if (act && !keep) nxt = n + lk.skip;
-      if (lk.child_count == 0) {
-        if (keep) nxt = n + 1;
-        if (__ballot(keep)) {
-          const double lim = keep ? rc2 : -1.0;
-          const uint32_t e0 = lk.begin + lk.count;
-          for (uint32_t c0 = lk.begin; c0 < e0; c0 += kWindow) {
-            const uint32_t cn = e0 - c0 < static_cast<uint32_t>(kWindow) ? e0 - c0 : static_cast<uint32_t>(kWindow);
-            __builtin_amdgcn_wave_barrier();
-            stage.template operator()<NEAR>(c0 + (static_cast<uint32_t>(lane) < cn ? lane : 0),
-                                            static_cast<uint32_t>(lane) < cn);
-            __builtin_amdgcn_wave_barrier();
-            pairs.template operator()<NEAR>(cn, lim);
-          }
-          __builtin_amdgcn_wave_barrier();
+    // lane-by-lane walk of the preorder range [nxt, end) with walk64_kernel's tests
+    uint32_t nxt = 0;
+    auto walk = [&]<bool NEAR>(uint32_t end) {
+      uint32_t n = wave_min_u32(nxt);
+      while (n < end) {
+        const NodeLink lk = D.link[n];
+        const NodeGeo64 g = D.geo64[n];
+        const bool act = nxt == n;
+        if (!__ballot(act)) {
+          if (lane == 0) atomicOr(&counters[kFaultSlot], 1ull);
+          break;
         }
-      } else if (__ballot(keep)) {
-        if constexpr (JVP) {
-          // the forward's strict acceptance; an accepted node's Jacobian terms
-          // go to the target and to the node's accumulators
+        const double h = g.half;
+        const double ndx = mi_fast(g.cx - px, 0), ndy = mi_fast(g.cy - py, 1), ndz = mi_fast(g.cz - pz, 2);
+        const double ax_ = fabs(ndx), ay_ = fabs(ndy), az_ = fabs(ndz);
+        const double fx_ = fmax(0.0, ax_ - h), fy_ = fmax(0.0, ay_ - h), fz_ = fmax(0.0, az_ - h);
+        const bool keep = act && within_cutoff(fx_ * fx_ + fy_ * fy_ + fz_ * fz_, P.rcut, P.rcut2);
+        if (act && !keep) nxt = n + lk.skip;
+        if (lk.child_count == 0) {
+          if (keep) nxt = n + 1;
+          if (__ballot(keep)) {
+            const double lim = keep ? rc2 : -1.0;
+            const uint32_t e0 = lk.begin + lk.count;
+            for (uint32_t c0 = lk.begin; c0 < e0; c0 += kWindow) {
+              const uint32_t cn = e0 - c0 < static_cast<uint32_t>(kWindow) ? e0 - c0 : static_cast<uint32_t>(kWindow);
+              __builtin_amdgcn_wave_barrier();
+              if (static_cast<uint32_t>(lane) < cn) {
+                const double4 sv = D.src64[c0 + lane];
+                if constexpr (JVP) listl[lane] = D.lam64[c0 + lane];
+                list[lane] =
+                    NEAR ? make_double4(image(sv.x, bx, 0), image(sv.y, by, 1), image(sv.z, bz, 2), sv.w) : sv;
+              }
+              __builtin_amdgcn_wave_barrier();
+              leaf_pairs.template operator()<NEAR>(cn, lim);
+            }
+            __builtin_amdgcn_wave_barrier();
+          }
+        } else if (__ballot(keep)) {
+          // the forward's strict acceptance; in the JVP an accepted node's
+          // Jacobian terms go to the target and to the node's accumulators
           bool take_mp = false;
           double mdx = 0.0, mdy = 0.0, mdz = 0.0;
           if (keep && P.quad) {
@@ -2721,192 +3162,204 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(4)
           }
           if (keep) nxt = take_mp ? n + lk.skip : n + 1;
           if (__ballot(take_mp) && take_mp) {
-            jvp_node64(D.mom64[n], D.quad64[n], mdx, mdy, mdz, P, lk_.x, lk_.y, lk_.z, D.vjp_node_acc + 10ull * n,
-                       ax, ay, az);
-            const unsigned int slot_i = atomicAdd(D.vjp_accepted_count, 1u);
-            if (slot_i < D.vjp_accepted_cap)
-              D.vjp_accepted[slot_i] = (static_cast<unsigned long long>(tp) << 32) | n;
+            if constexpr (JVP) {
+              jvp_node64(D.mom64[n], D.quad64[n], mdx, mdy, mdz, P, lk_.x, lk_.y, lk_.z, D.vjp_node_acc + 10ull * n,
+                         ax, ay, az);
+              const unsigned int slot_i = atomicAdd(D.vjp_accepted_count, 1u);
+              if (slot_i < D.vjp_accepted_cap)
+                D.vjp_accepted[slot_i] = (static_cast<unsigned long long>(tp) << 32) | n;
+            } else {
+              node_accel64(D.mom64[n], D.quad64[n], mdx, mdy, mdz, P, ax, ay, az);
+            }
           }
-        } else {
-          bool take_mp = false;
-          double mdx = 0.0, mdy = 0.0, mdz = 0.0;
-          if (keep) {
-            const bool inside = ax_ <= h && ay_ <= h && az_ <= h;
-            const double mx = ax_ + h, my = ay_ + h, mz = az_ + h;
-            const bool contained = within_cutoff(mx * mx + my * my + mz * mz, P.rcut, P.rcut2);
-            const NodeMom64 M = D.mom64[n];
-            mdx = mi_fast(M.comx - px, 0);
-            mdy = mi_fast(M.comy - py, 1);
-            mdz = mi_fast(M.comz - pz, 2);
-            take_mp = accept64(h, D.quad64[n].offset, inside, contained, mdx * mdx + mdy * mdy + mdz * mdz, P);
-            nxt = take_mp ? n + lk.skip : n + 1;
-          }
-          if (__ballot(take_mp) && take_mp) node_accel64(D.mom64[n], D.quad64[n], mdx, mdy, mdz, P, ax, ay, az);
         }
+        n = next_node(n, nxt);
       }
-      n = next_node(n, nxt);
-    }
-  };
+    };
 
-  if (boxed) {
-    // box classification of node q: 0 pruned, 1 kept leaf, 3 opened, 4 a
-    // subtree walked lane by lane
-    auto classify = [&](uint32_t q, uint32_t& next, uint32_t& lb, uint32_t& lc) -> int {
-      const NodeLink lk = D.link[q];
-      const NodeGeo64 g = D.geo64[q];
-      const double h = g.half;
-      const double dx = fmax(0.0, fabs(mi_fast(g.cx - bx, 0)) - h - ex);
-      const double dy = fmax(0.0, fabs(mi_fast(g.cy - by, 1)) - h - ey);
-      const double dz = fmax(0.0, fabs(mi_fast(g.cz - bz, 2)) - h - ez);
-      const bool keep = dx * dx + dy * dy + dz * dz <= rc2 * (1.0 + 1.0e-9);
-      if (lk.child_count == 0) {
-        lb = lk.begin;
-        lc = lk.count;
-        return keep ? 1 : 0;
+    if constexpr (FRAME) {
+      // staged sources beyond r_cut of the target box (every pair with them
+      // lies beyond r_cut, so their terms are zero) are dropped
+      const double cull2 = rc2 * (1.0 + 1.0e-9);
+      uint32_t wn = 0;  // records in the window
+      // evaluation groups as in walkmix_box_kernel
+      const double compact = kBoxCompact * rc;
+      const bool one = TL <= kBoxGroup || (ex <= compact && ey <= compact && ez <= compact);
+      const uint32_t lgG = one ? lgT : 4u, GL = 1u << lgG, lgGS = 6u - lgG;
+      const uint32_t groups = one ? 1u : TL >> lgG;
+      const uint32_t gcol = static_cast<uint32_t>(lane) & (GL - 1u), gslice = static_cast<uint32_t>(lane) >> lgG;
+      const uint32_t mine = gslice * (GL + 1u);
+      // group boxes about the box centre in FP32; the half-extents' margin
+      // covers the rounding of the offsets (box and r_cut are of one order)
+      const float bm = static_cast<float>(1.0e-6 * (rc + ex + ey + ez));
+      float qc0 = 0.0f, qc1 = 0.0f, qc2 = 0.0f;
+      float qh0 = static_cast<float>(ex) + bm, qh1 = static_cast<float>(ey) + bm, qh2 = static_cast<float>(ez) + bm;
+      if (!one) {
+        row_bounds(static_cast<float>(qx - bx), qc0, qh0);
+        row_bounds(static_cast<float>(qy - by), qc1, qh1);
+        row_bounds(static_cast<float>(qz - bz), qc2, qh2);
+        qh0 += bm;
+        qh1 += bm;
+        qh2 += bm;
       }
-      if (!keep) {
-        next = q + lk.skip;
-        return 0;
-      }
-      if (P.quad && h < 0.041 * rc) {
-        // accept64 needs 2h/r < 0.08: every target within 25 h of the COM fails it
-        const NodeMom64 M = D.mom64[q];
-        const double fx_ = fabs(mi_fast(M.comx - bx, 0)) + ex, fy_ = fabs(mi_fast(M.comy - by, 1)) + ey,
-                     fz_ = fabs(mi_fast(M.comz - bz, 2)) + ez;
-        if (!(fx_ * fx_ + fy_ * fy_ + fz_ * fz_ <= 625.0 * h * h * (1.0 - 1.0e-9))) {
-          next = q + lk.skip;
-          return 4;
-        }
-      }
-      return 3;
-    };
-    const double lim = valid ? rc2 : -1.0;
-    // forward: staged sources beyond r_cut of the target box (every pair with
-    // them lies beyond r_cut, so their terms are zero) are dropped before the
-    // window, as in walkmix_kernel's box walk
-    const double cull2 = rc2 * (1.0 + 1.0e-9);
-    uint32_t nl = 0;  // list[w][0, nl): listed sources, staged 64 at a time
-    uint32_t wn = 0;  // forward: compacted records in win[w][0, wn)
-    auto evaluate = [&](uint32_t cn) {
-      __builtin_amdgcn_wave_barrier();
-      pairs.template operator()<true>(cn, lim);
-      __builtin_amdgcn_wave_barrier();
-    };
-    auto eval_window = [&](uint32_t cn) {
-      __builtin_amdgcn_wave_barrier();
-      const bool on = static_cast<uint32_t>(lane) < cn;
-      const uint32_t j = list[w][on ? lane : 0];
-      nl = 0;
-      if constexpr (JVP) {
-        // the same drop without a second window: kept sources beyond the
-        // window's free room go back to the front of the list (as indices)
-        // and are staged again with the next batch
-        const double4 sv = D.src64[j];
-        const double4 rec = make_double4(image(sv.x, bx, 0), image(sv.y, by, 1), image(sv.z, bz, 2), sv.w);
-        const double fx_ = fmax(0.0, fabs(rec.x - bx) - ex), fy_ = fmax(0.0, fabs(rec.y - by) - ey),
-                     fz_ = fmax(0.0, fabs(rec.z - bz) - ez);
-        const bool keep = on && fx_ * fx_ + fy_ * fy_ + fz_ * fz_ <= cull2;
-        const unsigned long long km = __ballot(keep);
-        const uint32_t pos = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(km >> 32),
-                                                       __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(km), 0u));
-        const uint32_t room = static_cast<uint32_t>(kWindow) - wn;
-        const uint32_t kept = static_cast<uint32_t>(__popcll(km));
-        if (keep && pos < room) {
-          win[w][wn + pos] = rec;
-          winl[w][wn + pos] = D.lam64[j];
-        }
-        if (keep && pos >= room) list[w][pos - room] = j;
-        const uint32_t taken = kept < room ? kept : room;
-        wn += taken;
-        nl = kept - taken;
-        if (wn == static_cast<uint32_t>(kWindow)) {
-          evaluate(kWindow);
-          wn = 0;
-        }
-      } else {
-        const double4 sv = D.src64[j];
-        const double4 rec = make_double4(image(sv.x, bx, 0), image(sv.y, by, 1), image(sv.z, bz, 2), sv.w);
-        const double fx_ = fmax(0.0, fabs(rec.x - bx) - ex), fy_ = fmax(0.0, fabs(rec.y - by) - ey),
-                     fz_ = fmax(0.0, fabs(rec.z - bz) - ez);
-        const bool keep = on && fx_ * fx_ + fy_ * fy_ + fz_ * fz_ <= cull2;
-        const unsigned long long km = __ballot(keep);
-        const uint32_t at =
-            wn + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(km >> 32),
-                                           __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(km), 0u));
-        if (keep) win[w][at] = rec;
-        wn += static_cast<uint32_t>(__popcll(km));
-        if (wn >= static_cast<uint32_t>(kWindow)) {
-          evaluate(kWindow);
-          wn -= kWindow;
-          if (static_cast<uint32_t>(lane) < wn) {
-            const double4 t = win[w][kWindow + lane];
-            win[w][lane] = t;
+      const float gcull2 = static_cast<float>(cull2) * 1.000001f;
+      auto slot_of = [&](uint32_t r) -> uint32_t { return (r & ((1u << lgGS) - 1u)) * (GL + 1u) + (r >> lgGS); };
+      const double far = 8.0 * (rc + ex + ey + ez);
+      auto process = [&]() {
+        __builtin_amdgcn_wave_barrier();
+        for (uint32_t g = 0; g < groups; ++g) {
+          const uint32_t row = g << lgG;
+          const int from = static_cast<int>(row + gcol);
+          const double x = __shfl(qx, from, kWave), y = __shfl(qy, from, kWave), z = __shfl(qz, from, kWave);
+          double4 tl = make_double4(0.0, 0.0, 0.0, 0.0);
+          double tm = 0.0;
+          if constexpr (JVP) {
+            tl.x = __shfl(lk_.x, from, kWave);
+            tl.y = __shfl(lk_.y, from, kWave);
+            tl.z = __shfl(lk_.z, from, kWave);
+            tm = __shfl(mk, from, kWave);
+          }
+          const float c0 = readlane_f32(qc0, row), c1 = readlane_f32(qc1, row), c2 = readlane_f32(qc2, row);
+          const float h0 = readlane_f32(qh0, row), h1 = readlane_f32(qh1, row), h2 = readlane_f32(qh2, row);
+          double lx = 0.0, ly = 0.0, lz = 0.0;
+          uint32_t n2 = 0;
+          for (uint32_t b = 0;; b += kWave) {
+            const bool end = b >= wn;
+            double4 rec = make_double4(0.0, 0.0, 0.0, 0.0);
+            bool keep = false;
+            if (b + lane < wn) {
+              rec = win[b + lane];
+              const float dx = fmaxf(fabsf(static_cast<float>(rec.x - bx) - c0) - h0, 0.0f);
+              const float dy = fmaxf(fabsf(static_cast<float>(rec.y - by) - c1) - h1, 0.0f);
+              const float dz = fmaxf(fabsf(static_cast<float>(rec.z - bz) - c2) - h2, 0.0f);
+              keep = !(fmaf(dx, dx, fmaf(dy, dy, dz * dz)) > gcull2);
+            }
+            const unsigned long long km = __ballot(keep);
+            const uint32_t kept = static_cast<uint32_t>(__popcll(km));
+            if (n2 && (end || n2 + kept > static_cast<uint32_t>(kWindow))) {
+              // dummies beyond r_cut of every target fill the last iterations
+              const uint32_t iters = (((n2 + (1u << lgGS) - 1u) >> lgGS) + 1u) & ~1u;
+              if (static_cast<uint32_t>(lane) >= n2 && static_cast<uint32_t>(lane) < iters << lgGS) {
+                list[slot_of(lane)] = make_double4(bx + far, by + far, bz + far, 0.0);
+                if constexpr (JVP) listl[slot_of(lane)] = make_double4(0.0, 0.0, 0.0, 0.0);
+              }
+              __builtin_amdgcn_wave_barrier();
+#pragma unroll 2
+              for (uint32_t si = 0; si < iters; ++si)
+                pair.template operator()<true>(list[mine + si], listl + (JVP ? mine + si : 0u), x, y, z, tl, tm, rc2,
+                                               lx, ly, lz);
+              __builtin_amdgcn_wave_barrier();
+              n2 = 0;
+            }
+            if (end) break;
+            if (keep) {
+              const uint32_t at = slot_of(n2 + lanes_below(km));
+              list[at] = rec;
+              if constexpr (JVP) listl[at] = winl[b + lane];
+            }
+            n2 += kept;
+          }
+          // slices -> the group's own lanes
+          for (uint32_t o = GL; o < static_cast<uint32_t>(kWave); o <<= 1) {
+            lx += __shfl_xor(lx, static_cast<int>(o), kWave);
+            ly += __shfl_xor(ly, static_cast<int>(o), kWave);
+            lz += __shfl_xor(lz, static_cast<int>(o), kWave);
+          }
+          if (gslice == g) {
+            ax = fma(gm, lx, ax);
+            ay = fma(gm, ly, ay);
+            az = fma(gm, lz, az);
           }
         }
+        wn = 0;
+        __builtin_amdgcn_wave_barrier();
+      };
+      // the box in fixed point: the centre's floor and the conversion of the
+      // half-extents move a face by less than four units
+      const double fs0 = 4294967296.0 * iL0, fs1 = 4294967296.0 * iL1, fs2 = 4294967296.0 * iL2;
+      auto fixed = [](double v, double scale) -> uint32_t {
+        return static_cast<uint32_t>(static_cast<uint64_t>(static_cast<int64_t>(floor(v * scale))));
+      };
+      auto half = [&](double e, double fs, float unit) -> float {
+        return static_cast<float>((e * fs + 4.0) * (1.0 + 1.0e-6)) * unit;
+      };
+      const BoxFrame frame{fixed(bx, fs0), fixed(by, fs1), fixed(bz, fs2), half(ex, fs0, s0), half(ey, fs1, s1),
+                           half(ez, fs2, s2), s0, s1, s2, P.prune2_sep,
+                           P.quad ? static_cast<float>(0.041 * rc) : 0.0f, to_len};
+      struct Record {
+        double4 s;
+        uint32_t j;
+      };
+      box_traverse(
+          D.wnode, box_all[w], lane, frame, [&](uint32_t j) -> Record { return Record{D.src64[j], j}; },
+          [&](const Record& r, bool on, bool last) {
+            const double4 rec =
+                make_double4(image(r.s.x, bx, 0), image(r.s.y, by, 1), image(r.s.z, bz, 2), r.s.w);
+            const double fx_ = fmax(0.0, fabs(rec.x - bx) - ex), fy_ = fmax(0.0, fabs(rec.y - by) - ey),
+                         fz_ = fmax(0.0, fabs(rec.z - bz) - ez);
+            const bool keep = on && fx_ * fx_ + fy_ * fy_ + fz_ * fz_ <= cull2;
+            const unsigned long long km = __ballot(keep);
+            const uint32_t kept = static_cast<uint32_t>(__popcll(km));
+            bool todo = true, go = wn + kept > kWin;
+            do {  // evaluate a full window, add the batch, evaluate the last window
+              if (go) process();
+              if (todo) {
+                if (keep) {
+                  const uint32_t at = wn + lanes_below(km);
+                  win[at] = rec;
+                  if constexpr (JVP) winl[at] = D.lam64[r.j];
+                }
+                wn += kept;
+                todo = false;
+              }
+              go = last && wn;
+            } while (go);
+          },
+          [&](uint32_t pre, uint32_t end) -> bool {
+            const NodeGeo64 g = D.geo64[pre];
+            const NodeMom64 M = D.mom64[pre];
+            const double h = g.half;
+            const double ax_ = fabs(mi_fast(g.cx - px, 0)), ay_ = fabs(mi_fast(g.cy - py, 1)),
+                         az_ = fabs(mi_fast(g.cz - pz, 2));
+            const double mx = ax_ + h, my = ay_ + h, mz = az_ + h;
+            const double mdx = mi_fast(M.comx - px, 0), mdy = mi_fast(M.comy - py, 1), mdz = mi_fast(M.comz - pz, 2);
+            const bool acc = accept64(h, D.quad64[pre].offset, ax_ <= h && ay_ <= h && az_ <= h,
+                                      within_cutoff(mx * mx + my * my + mz * mz, P.rcut, P.rcut2),
+                                      mdx * mdx + mdy * mdy + mdz * mdz, P);
+            if (!__ballot(owner && acc)) return true;
+            nxt = owner ? pre : end;
+            walk.template operator()<true>(end);
+            return false;
+          });
+    } else {
+      nxt = owner ? 0u : node_count;
+      walk.template operator()<false>(node_count);
+    }
+    if (owner) {
+      double gx = 0.0, gy = 0.0, gz = 0.0;
+      if (P.pm_enabled) {
+        if constexpr (JVP)
+          vjp_gather64<SCHEME>(P, D.f64x, D.f64y, D.f64z, D.nu64, lk_.x, lk_.y, lk_.z, mk, px, py, pz, gx, gy, gz);
+        else
+          interp64<SCHEME>(P, D.f64x, D.f64y, D.f64z, px, py, pz, gx, gy, gz);
       }
-    };
-    uint32_t p = 0;
-    while (p < node_count) {
-      const uint32_t q = p + lane;
-      uint32_t next = q + 1, lb = 0, lc = 0;
-      const int kind = q < node_count ? classify(q, next, lb, lc) : 3;
-      unsigned long long chain = 0;
-      uint32_t cur = p;
-      while (cur < p + kWave && cur < node_count) {
-        const uint32_t l = cur - p;
-        chain |= 1ull << l;
-        cur = readlane_u32(next, l);
+      const uint32_t row = D.order[tp];
+      const uint32_t slot = P.identity_targets ? row : D.tslot[k];
+      static_cast<double*>(out.ax)[slot] = gx + ax;
+      static_cast<double*>(out.ay)[slot] = gy + ay;
+      static_cast<double*>(out.az)[slot] = gz + az;
+      if (out.pm_x) {
+        static_cast<double*>(out.pm_x)[slot] = gx;
+        static_cast<double*>(out.pm_y)[slot] = gy;
+        static_cast<double*>(out.pm_z)[slot] = gz;
       }
-      const uint32_t base = p;
-      p = cur;
-      const bool on = (chain >> lane) & 1ull;
-      unsigned long long rest = __ballot(on && kind == 1);
-      while (rest) {
-        const uint32_t l = static_cast<uint32_t>(__ffsll(static_cast<long long>(rest)) - 1);
-        rest &= rest - 1ull;
-        const uint32_t b0 = readlane_u32(lb, l), c = readlane_u32(lc, l);
-        for (uint32_t c0 = 0; c0 < c;) {
-          const uint32_t room = static_cast<uint32_t>(kWindow) - nl;
-          const uint32_t cn = c - c0 < room ? c - c0 : room;
-          if (static_cast<uint32_t>(lane) < cn) list[w][nl + lane] = b0 + c0 + lane;
-          nl += cn;
-          c0 += cn;
-          if (nl == static_cast<uint32_t>(kWindow)) eval_window(kWindow);
-        }
-      }
-      unsigned long long sub = __ballot(on && kind == 4);
-      while (sub) {
-        const uint32_t l = static_cast<uint32_t>(__ffsll(static_cast<long long>(sub)) - 1);
-        sub &= sub - 1ull;
-        const uint32_t end = readlane_u32(next, l);
-        // the lane-by-lane walk stages its leaves in the window's front
-        if (wn) {
-          evaluate(wn);
-          wn = 0;
-        }
-        nxt = valid ? base + l : end;
-        walk.template operator()<true>(end);
+      if (out.sr_x) {
+        static_cast<double*>(out.sr_x)[row] = ax;
+        static_cast<double*>(out.sr_y)[row] = ay;
+        static_cast<double*>(out.sr_z)[row] = az;
       }
     }
-    while (nl) eval_window(nl);  // JVP: each call takes at least one source or evaluates a full window
-    if (wn) evaluate(wn);
-  } else {
-    walk.template operator()<false>(node_count);
-  }
-  if (!valid) return;
-  static_cast<double*>(out.ax)[slot] = gx + ax;
-  static_cast<double*>(out.ay)[slot] = gy + ay;
-  static_cast<double*>(out.az)[slot] = gz + az;
-  if (out.pm_x) {
-    static_cast<double*>(out.pm_x)[slot] = gx;
-    static_cast<double*>(out.pm_y)[slot] = gy;
-    static_cast<double*>(out.pm_z)[slot] = gz;
-  }
-  const uint32_t row = D.order[tp];
-  if (out.sr_x) {
-    static_cast<double*>(out.sr_x)[row] = ax;
-    static_cast<double*>(out.sr_y)[row] = ay;
-    static_cast<double*>(out.sr_z)[row] = az;
+    seg += T;
   }
 }
 
@@ -3052,41 +3505,71 @@ void launch64(const WalkParams& p, const WalkData& d, const WalkOutputs& out, un
   walk64_kernel<SCHEME, JVP><<<grid_for(p.n_targets, kWalkThreads), kWalkThreads, 0, s>>>(p, d, out, counters);
   CHUI_LAUNCH_CHECK("walk64_kernel");
 }
+// Targets per wave of the box walks: 64, or fewer (down to 8) until the
+// launch has kBoxMinWaves waves, four for each of the 1024 SIMDs.
+constexpr uint32_t kBoxMinWaves = 4096;
+WalkParams box_params(const WalkParams& p) {
+  WalkParams q = p;
+  q.targets_per_wave = kWave;
+  if (q.box_single)
+    while (q.targets_per_wave > 8 && p.n_targets / q.targets_per_wave < kBoxMinWaves) q.targets_per_wave >>= 1;
+  return q;
+}
+unsigned box_blocks(const WalkParams& p, unsigned waves) {
+  return grid_for((static_cast<std::size_t>(p.n_targets) + p.targets_per_wave - 1) / p.targets_per_wave, waves);
+}
+
+template <int SCHEME, bool CUBIC, bool LOG, int WAVES>
+void launch_box(const WalkParams& p, const WalkData& d, const WalkOutputs& out, unsigned long long* counters,
+                hipStream_t s) {
+  const WalkParams q = box_params(p);
+  const std::size_t lds = LOG ? p.log_cells * sizeof(float4) : 0;
+  if (LOG && q.box_single && q.exact_pairs)
+    walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, true, LOG><<<box_blocks(q, WAVES), WAVES * kWave, lds, s>>>(
+        q, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32, d.wnode);
+  else if (q.box_single)
+    walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, true, false><<<box_blocks(q, WAVES), WAVES * kWave, lds, s>>>(
+        q, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32, d.wnode);
+  else
+    walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, false, false><<<box_blocks(q, WAVES), WAVES * kWave, lds, s>>>(
+        q, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32, d.wnode);
+  CHUI_LAUNCH_CHECK("walkmix_box_kernel");
+}
+
+template <bool JVP>
+void launch_box64(const WalkParams& p, const WalkData& d, const WalkOutputs& out, unsigned long long* counters,
+                  hipStream_t s) {
+  const WalkParams q = box_params(p);
+  const unsigned grid = box_blocks(q, kWalkWaves);
+  if (q.box_single && p.assignment == 0)
+    walk64_box_kernel<0, JVP, true><<<grid, kWalkThreads, 0, s>>>(q, d, out, counters);
+  else if (q.box_single)
+    walk64_box_kernel<1, JVP, true><<<grid, kWalkThreads, 0, s>>>(q, d, out, counters);
+  else if (p.assignment == 0)
+    walk64_box_kernel<0, JVP, false><<<grid, kWalkThreads, 0, s>>>(q, d, out, counters);
+  else
+    walk64_box_kernel<1, JVP, false><<<grid, kWalkThreads, 0, s>>>(q, d, out, counters);
+  CHUI_LAUNCH_CHECK("walk64_box_kernel");
+}
+
 template <int SCHEME, bool CUBIC>
 void launchmix(const WalkParams& p, const WalkData& d, const WalkOutputs& out, unsigned long long* counters,
                hipStream_t s) {
-  const bool devn = d.node_count_dev != nullptr;
-  if (p.count && !devn)
-    walkmix_kernel<SCHEME, CUBIC, true><<<grid_for(p.n_targets, kWalkThreads), kWalkThreads, 0, s>>>(
+  if (p.count) {
+    if (d.node_count_dev) throw std::logic_error("counting walk after a capture-safe build");
+    walkmix_kernel<SCHEME, CUBIC><<<grid_for(p.n_targets, kWalkThreads), kWalkThreads, 0, s>>>(
         p, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32);
-  else if (p.count)
-    throw std::logic_error("counting walk after a capture-safe build");
-  else if (p.target_per_wave)
+    CHUI_LAUNCH_CHECK("walkmix_kernel");
+  } else if (p.target_per_wave) {
     walkmix_target_kernel<SCHEME, CUBIC><<<grid_for(p.n_targets, kWalkWaves), kWalkThreads, 0, s>>>(p, d, out);
-  else if (p.log_cells > 0 && devn)
-    walkmix_kernel<SCHEME, CUBIC, false, true, true, kWalkWaves, true>
-        <<<grid_for(p.n_targets, kWalkThreads), kWalkThreads, p.log_cells * sizeof(float4), s>>>(
-            p, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32);
-  else if (p.log_cells > 0 && p.walk_waves == 8)
-    walkmix_kernel<SCHEME, CUBIC, false, true, true, 8>
-        <<<grid_for(p.n_targets, 8 * kWave), 8 * kWave, p.log_cells * sizeof(float4), s>>>(
-            p, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32);
-  else if (p.log_cells > 0 && p.walk_waves == 2)
-    walkmix_kernel<SCHEME, CUBIC, false, true, true, 2>
-        <<<grid_for(p.n_targets, 2 * kWave), 2 * kWave, p.log_cells * sizeof(float4), s>>>(
-            p, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32);
-  else if (p.log_cells > 0)
-    walkmix_kernel<SCHEME, CUBIC, false, true, true>
-        <<<grid_for(p.n_targets, kWalkThreads), kWalkThreads, p.log_cells * sizeof(float4), s>>>(
-            p, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32);
-  else if (devn)
-    walkmix_kernel<SCHEME, CUBIC, false, true, false, kWalkWaves, true>
-        <<<grid_for(p.n_targets, kWalkThreads), kWalkThreads, 0, s>>>(p, d, out, counters, d.link, d.geo32, d.mom32,
-                                                                       d.quad32, d.box32);
-  else
-    walkmix_kernel<SCHEME, CUBIC, false, true><<<grid_for(p.n_targets, kWalkThreads), kWalkThreads, 0, s>>>(
-        p, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32);
-  CHUI_LAUNCH_CHECK("walkmix_kernel");
+    CHUI_LAUNCH_CHECK("walkmix_target_kernel");
+  } else if (p.log_cells > 0) {
+    if (p.walk_waves == 8) launch_box<SCHEME, CUBIC, true, 8>(p, d, out, counters, s);
+    else if (p.walk_waves == 2) launch_box<SCHEME, CUBIC, true, 2>(p, d, out, counters, s);
+    else launch_box<SCHEME, CUBIC, true, 4>(p, d, out, counters, s);
+  } else {
+    launch_box<SCHEME, CUBIC, false, 4>(p, d, out, counters, s);
+  }
 }
 
 }  // namespace
@@ -3129,28 +3612,28 @@ std::vector<float> log_residual_table(double scale, double eps, double a, int32_
   return tab;
 }
 
-std::vector<double> gaussian_quintic_table(double t_max, int cells) {
+std::vector<double> gaussian_quintic_table(double t_max, int cells, double factor) {
   // Interpolation at the Chebyshev points of each cell: error below
   // 2 (h/4)^6 max|H^(6)| / 6!, under 1e-16 for cells of width 0.04 and
-  // about 1e-13 at width 0.2 (t_max = 50 on 256 cells). The 6 x 6
-  // Vandermonde system in u is solved in long double.
-  const int K = cells;
-  const double h = t_max / K;
-  std::vector<double> tab(6 * static_cast<std::size_t>(K));
+  // about 1e-13 at width 0.2 (t_max = 50 on 255 cells). The 6 x 6
+  // Vandermonde system in u is solved in long double. The first cell covers
+  // t >= 0 only, u in [0, 1/2].
+  const double h = t_max / cells;
+  std::vector<double> tab(6 * static_cast<std::size_t>(cells + 1));
   constexpr int D = 6;
-  long double un[D];
-  for (int j = 0; j < D; ++j)
-    un[j] = 0.5L + 0.5L * std::cos(static_cast<long double>(3.14159265358979323846264338327950288L) *
-                                   (2 * j + 1) / (2 * D));
-  for (int i = 0; i < K; ++i) {
+  for (int i = 0; i <= cells; ++i) {
+    const long double lo = i == 0 ? 0.0L : -0.5L, hi = 0.5L;
     long double A[D][D + 1];
     for (int j = 0; j < D; ++j) {
+      const long double cj = std::cos(static_cast<long double>(3.14159265358979323846264338327950288L) * (2 * j + 1) /
+                                      (2 * D));
+      const long double un = 0.5L * (lo + hi) + 0.5L * (hi - lo) * cj;
       long double pw = 1.0L;
       for (int c = 0; c < D; ++c) {
         A[j][c] = pw;
-        pw *= un[j];
+        pw *= un;
       }
-      A[j][D] = gaussian_h_exact((i + static_cast<double>(un[j])) * h);
+      A[j][D] = gaussian_h_exact((i + static_cast<double>(un)) * h);
     }
     for (int c = 0; c < D; ++c) {  // Gaussian elimination with partial pivoting
       int piv = c;
@@ -3163,7 +3646,8 @@ std::vector<double> gaussian_quintic_table(double t_max, int cells) {
         for (int q = c; q <= D; ++q) A[r][q] -= f * A[c][q];
       }
     }
-    for (int c = 0; c < D; ++c) tab[6 * static_cast<std::size_t>(i) + c] = static_cast<double>(A[c][D] / A[c][c]);
+    for (int c = 0; c < D; ++c)
+      tab[6 * static_cast<std::size_t>(i) + c] = static_cast<double>(factor * A[c][D] / A[c][c]);
   }
   return tab;
 }
@@ -3218,10 +3702,8 @@ void walk_fp64(const Tree& t, const WalkParams& p, const double4* src, int unifo
   }
   if (p.box64) {
     d.h64tab = h64tab;
-    const unsigned grid = grid_for(p.n_targets, kWalkThreads);
-    if (p.assignment == 0) walk64_box_kernel<0><<<grid, kWalkThreads, 0, s>>>(p, d, out, counters);
-    else walk64_box_kernel<1><<<grid, kWalkThreads, 0, s>>>(p, d, out, counters);
-    CHUI_LAUNCH_CHECK("walk64_box_kernel");
+    d.wnode = t.wnode.as<WalkNode>();
+    launch_box64<false>(p, d, out, counters, s);
     return;
   }
   if (p.assignment == 0) launch64<0>(p, d, out, counters, s);
@@ -3426,10 +3908,8 @@ void walk_fp64_vjp(const Tree& t, const WalkParams& p, const double4* src, int u
   }
   if (p.box64) {
     d.h64tab = h64tab;
-    const unsigned grid = grid_for(p.n_targets, kWalkThreads);
-    if (p.assignment == 0) walk64_box_kernel<0, true><<<grid, kWalkThreads, 0, s>>>(p, d, out, counters);
-    else walk64_box_kernel<1, true><<<grid, kWalkThreads, 0, s>>>(p, d, out, counters);
-    CHUI_LAUNCH_CHECK("walk64_box_kernel (JVP)");
+    d.wnode = t.wnode.as<WalkNode>();
+    launch_box64<true>(p, d, out, counters, s);
     return;
   }
   if (p.assignment == 0) launch64<0, true>(p, d, out, counters, s);
@@ -3478,7 +3958,7 @@ void walk_mixed(const Tree& t, const WalkParams& p, const uint4* src, int unifor
   d.src32 = src;
   d.htab = htab;
   d.ltab = ltab;
-  d.child = t.child_index.as<uint32_t>();
+  d.wnode = t.wnode.as<WalkNode>();
   d.uniform_mass = uniform_mass;
   d.tpos = target_pos;
   d.tslot = target_slot;

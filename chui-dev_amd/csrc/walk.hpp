@@ -59,17 +59,25 @@ struct WalkParams {
   // (separation units, per axis) for which the wave walks the tree once for
   // its box instead of lane by lane.
   float box_half_max[3];
+  double box_max64;      // the same for the FP64 walk (length)
+  int box_single;        // a single target always has a box frame (r_cut clear of L/2)
+  uint32_t targets_per_wave;  // box walks: consecutive targets of a wave (8..64, a power of two)
   // FP64 box-classified walk (solves without counters or nearest-pair lane):
-  // degree-5 cells of H on [0, t_max] (h64_cells of them, t = r^2 / 4a^2),
-  // r^2 -> cell coordinate, eps^2 and 1/(8 a^3).
+  // degree-5 cells of -H / 8 a^3 on [0, t_max] (centres 0..h64_cells, t = r^2 /
+  // 4a^2), r^2 -> cell coordinate and eps^2 (at least 1e-36).
   // Mixed timed walk with the residual table indexed by the float bits of
   // s = r^2 + eps^2 (log_cells > 0): cells (the last one, at s = 1, is zero)
   // and the (exponent, top-5-mantissa) field of the first cell.
   uint32_t log_cells, log_base;
+  // the same walk with r^2 and the cutoff in FP64 (few sources): lengths per
+  // fixed-point unit, separation unit^2 -> table units, eps^2 there, r_cut^2 in
+  // separation units
+  int exact_pairs;
+  double fx_to_len64[3], sep2_to_tab, eps2_tab64, rcut2_sep64;
   int box64;
   int h64_cells;
   double h64_scale;
-  double eps2_64, c8_64;
+  double eps2_64;
   // Adaptive acceptance (TreePmAcceptancePolicy::kAdaptiveRelative; FP64 walk):
   // estimator, com-distance cutoff policy, Gaussian-table leaf pairs, radial-
   // coefficient node expansion, maximum opening angle, alpha, acceleration
@@ -232,10 +240,11 @@ void walk_mixed(const Tree& t, const WalkParams& p, const uint4* src, int unifor
 // Host FP64 table of H(t) on [0, t_max] (kHTableCells cubic cells, 4 floats
 // each); sets p.t_to_cell.
 std::vector<float> gaussian_coefficient_table(WalkParams& p, double t_max);
-// Host table of the FP64 box walk: H(t) on [0, t_max] in `cells` cells, per
-// cell the monomial coefficients a0..a5 of the degree-5 polynomial in the cell
-// coordinate u in [0, 1) through the 6 Chebyshev points of the cell.
-std::vector<double> gaussian_quintic_table(double t_max, int cells);
+// Host table of the FP64 box walk: factor * H(t) around the centres t = i h,
+// i = 0..cells, h = t_max / cells: per cell the monomial coefficients a0..a5 of
+// the degree-5 polynomial in u = t / h - i, |u| <= 1/2, through the 6
+// Chebyshev points of the cell.
+std::vector<double> gaussian_quintic_table(double t_max, int cells, double factor);
 // Host table of the mixed timed walk: the residual coefficient as a function
 // of s = (r^2 + eps^2) * scale on 32 cubic cells per octave from the octave of
 // eps^2 * scale up to s = 1, plus one zero cell; 4 floats per cell (the
@@ -246,6 +255,6 @@ constexpr int kLogCellBits = 5;  // 32 cells per octave
 constexpr int kLogCellsPerOctave = 1 << kLogCellBits;
 constexpr int kLogMantissaShift = 23 - kLogCellBits;
 std::vector<float> log_residual_table(double scale, double eps, double a, int32_t& first_octave, uint32_t& cells);
-constexpr int kH64MaxCells = 256;
+constexpr int kH64MaxCells = 255;  // and one half cell at t = 0
 
 }  // namespace chui
