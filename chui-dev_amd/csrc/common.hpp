@@ -71,7 +71,7 @@ inline void require_not_capturing(hipStream_t s, const char* what) {
 // block: the copy lands directly in host memory instead of going through the
 // runtime's staging pass for pageable destinations.
 struct PinnedReadback {
-  static constexpr std::size_t kBytes = 256;
+  static constexpr std::size_t kBytes = 512;
   void* ptr = nullptr;
   PinnedReadback() = default;
   PinnedReadback(const PinnedReadback&) = delete;

@@ -65,7 +65,7 @@ template <class K>
 __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(
     const K* __restrict__ keys, const uint32_t* __restrict__ vals, K* __restrict__ okeys,
     uint32_t* __restrict__ ovals, std::size_t n, int shift, uint32_t dmask,
-    const uint32_t* __restrict__ offsets, uint32_t tiles) {
+    const uint32_t* __restrict__ offsets, const uint32_t* __restrict__ digit_totals, uint32_t tiles) {
   __shared__ uint32_t wcount[kSortWaves][256];
   __shared__ uint32_t gbase[256];
   __shared__ uint32_t lbase[256];
@@ -74,7 +74,12 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(
   const int w = threadIdx.x / kWave;
   const int lane = threadIdx.x % kWave;
   for (int i = threadIdx.x; i < kSortWaves * 256; i += kSortThreads) (&wcount[0][0])[i] = 0;
-  gbase[threadIdx.x] = offsets[static_cast<std::size_t>(threadIdx.x) * tiles + blockIdx.x];
+  {
+    // digit d's first position: the digits before it, then its tiles before this one
+    uint32_t all;
+    const uint32_t before = block_exclusive_sum(digit_totals[threadIdx.x], &all);
+    gbase[threadIdx.x] = before + offsets[static_cast<std::size_t>(threadIdx.x) * tiles + blockIdx.x];
+  }
   __syncthreads();
 
   const std::size_t base = static_cast<std::size_t>(blockIdx.x) * kSortTile +
@@ -147,6 +152,33 @@ __global__ __launch_bounds__(kSortThreads) void sort_scatter_kernel(
   }
 }
 
+// One block per row: exclusive prefix sums of the row in place, its total to
+// totals[row].
+__global__ __launch_bounds__(kScanThreads) void scan_rows_kernel(uint32_t* __restrict__ rows,
+                                                                 uint32_t* __restrict__ totals, uint32_t len) {
+  uint32_t* r = rows + static_cast<std::size_t>(blockIdx.x) * len;
+  uint32_t run = 0;
+  for (uint32_t base = 0; base < len; base += kScanTile) {
+    uint32_t x[kScanItems];
+    uint32_t sum = 0;
+    const uint32_t first = base + threadIdx.x * kScanItems;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+      x[k] = first + k < len ? r[first + k] : 0u;
+      sum += x[k];
+    }
+    uint32_t tot;
+    uint32_t at = run + block_exclusive_sum(sum, &tot);
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+      if (first + k < len) r[first + k] = at;
+      at += x[k];
+    }
+    run += tot;
+  }
+  if (threadIdx.x == 0) totals[blockIdx.x] = run;
+}
+
 __global__ __launch_bounds__(kScanThreads) void scan_reduce_kernel(const uint32_t* __restrict__ in, std::size_t n,
                                                                    uint32_t* __restrict__ partial) {
   const std::size_t base = static_cast<std::size_t>(blockIdx.x) * kScanTile;
@@ -208,13 +240,15 @@ void fill_any(T* p, T v, std::size_t n, hipStream_t s) {
 
 std::size_t tiles_for(std::size_t n) { return (n + kSortTile - 1) / kSortTile; }
 
+// A pass: tile histograms, one row of prefix sums per digit, scatter (which
+// adds the digits before). Returns whether the result is in the alt buffers.
 template <class K>
-void radix_sort_impl(K* keys, uint32_t* vals, K* keys_alt, uint32_t* vals_alt, std::size_t n, int begin_bit,
+bool radix_sort_impl(K* keys, uint32_t* vals, K* keys_alt, uint32_t* vals_alt, std::size_t n, int begin_bit,
                      int end_bit, void* scratch, hipStream_t s) {
-  if (n < 2 || end_bit <= begin_bit) return;
+  if (n < 2 || end_bit <= begin_bit) return false;
   const std::size_t tiles = tiles_for(n);
   uint32_t* hist = static_cast<uint32_t*>(scratch);
-  void* scan_scratch = hist + tiles * 256;
+  uint32_t* totals = hist + tiles * 256;
   K* src_k = keys;
   uint32_t* src_v = vals;
   K* dst_k = keys_alt;
@@ -225,16 +259,22 @@ void radix_sort_impl(K* keys, uint32_t* vals, K* keys_alt, uint32_t* vals_alt, s
     sort_hist_kernel<K><<<static_cast<unsigned>(tiles), kSortThreads, 0, s>>>(src_k, n, shift, dmask, hist,
                                                                              static_cast<uint32_t>(tiles));
     CHUI_LAUNCH_CHECK("sort_hist_kernel");
-    exclusive_scan_u32(hist, hist, tiles * 256, nullptr, scan_scratch, s);
+    exclusive_scan_rows(hist, totals, 256, static_cast<uint32_t>(tiles), s);
     sort_scatter_kernel<K><<<static_cast<unsigned>(tiles), kSortThreads, 0, s>>>(
-        src_k, src_v, dst_k, dst_v, n, shift, dmask, hist, static_cast<uint32_t>(tiles));
+        src_k, src_v, dst_k, dst_v, n, shift, dmask, hist, totals, static_cast<uint32_t>(tiles));
     CHUI_LAUNCH_CHECK("sort_scatter_kernel");
     std::swap(src_k, dst_k);
     std::swap(src_v, dst_v);
   }
-  if (src_k != keys) {
-    CHUI_HIP(hipMemcpyAsync(keys, src_k, n * sizeof(K), hipMemcpyDeviceToDevice, s));
-    CHUI_HIP(hipMemcpyAsync(vals, src_v, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
+  return src_k != keys;
+}
+
+template <class K>
+void radix_sort_back(K* keys, uint32_t* vals, K* keys_alt, uint32_t* vals_alt, std::size_t n, int begin_bit,
+                     int end_bit, void* scratch, hipStream_t s) {
+  if (radix_sort_impl<K>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, scratch, s)) {
+    CHUI_HIP(hipMemcpyAsync(keys, keys_alt, n * sizeof(K), hipMemcpyDeviceToDevice, s));
+    CHUI_HIP(hipMemcpyAsync(vals, vals_alt, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
   }
 }
 
@@ -270,18 +310,28 @@ void exclusive_scan_u32(const uint32_t* in, uint32_t* out, std::size_t n, uint32
   CHUI_LAUNCH_CHECK("scan_apply_kernel");
 }
 
+void exclusive_scan_rows(uint32_t* rows, uint32_t* totals, uint32_t count, uint32_t len, hipStream_t s) {
+  if (count == 0 || len == 0) return;
+  scan_rows_kernel<<<count, kScanThreads, 0, s>>>(rows, totals, len);
+  CHUI_LAUNCH_CHECK("scan_rows_kernel");
+}
+
 std::size_t radix_sort_scratch_bytes(std::size_t n) {
   const std::size_t tiles = tiles_for(std::max<std::size_t>(n, 1));
-  return tiles * 256 * sizeof(uint32_t) + scan_scratch_bytes(tiles * 256) + 256;
+  return (tiles + 1) * 256 * sizeof(uint32_t);
 }
 
 void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, std::size_t n,
                       int begin_bit, int end_bit, void* scratch, hipStream_t s) {
-  radix_sort_impl<uint64_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, scratch, s);
+  radix_sort_back<uint64_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, scratch, s);
+}
+bool radix_sort_pairs_swap(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, std::size_t n,
+                           int begin_bit, int end_bit, void* scratch, hipStream_t s) {
+  return radix_sort_impl<uint64_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, scratch, s);
 }
 void radix_sort_pairs32(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt, std::size_t n,
                         int begin_bit, int end_bit, void* scratch, hipStream_t s) {
-  radix_sort_impl<uint32_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, scratch, s);
+  radix_sort_back<uint32_t>(keys, vals, keys_alt, vals_alt, n, begin_bit, end_bit, scratch, s);
 }
 
 void fill_u32(uint32_t* p, uint32_t v, std::size_t n, hipStream_t s) { fill_any(p, v, n, s); }

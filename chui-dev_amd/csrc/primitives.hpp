@@ -15,6 +15,9 @@ std::size_t radix_sort_scratch_bytes(std::size_t n);
 // property the reference's Morton sort relies on (tree_ordering.cpp:13-71).
 void radix_sort_pairs(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt,
                       std::size_t n, int begin_bit, int end_bit, void* scratch, hipStream_t s);
+// The same without the copy back: returns whether the result is in the alt buffers.
+bool radix_sort_pairs_swap(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt, uint32_t* vals_alt, std::size_t n,
+                           int begin_bit, int end_bit, void* scratch, hipStream_t s);
 // Same for 32-bit keys.
 void radix_sort_pairs32(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint32_t* vals_alt,
                         std::size_t n, int begin_bit, int end_bit, void* scratch, hipStream_t s);
@@ -24,6 +27,10 @@ void radix_sort_pairs32(uint32_t* keys, uint32_t* vals, uint32_t* keys_alt, uint
 std::size_t scan_scratch_bytes(std::size_t n);
 void exclusive_scan_u32(const uint32_t* in, uint32_t* out, std::size_t n, uint32_t* total_dev,
                         void* scratch, hipStream_t s);
+
+// Exclusive prefix sums of `count` rows of `len` values in place, one block per
+// row; the row totals go to totals.
+void exclusive_scan_rows(uint32_t* rows, uint32_t* totals, uint32_t count, uint32_t len, hipStream_t s);
 
 void fill_u32(uint32_t* p, uint32_t v, std::size_t n, hipStream_t s);
 void fill_u64(uint64_t* p, uint64_t v, std::size_t n, hipStream_t s);

@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void popc_kernel(const uint32_t* __restrict__ 
 }
 
 constexpr int kGapThreads = 256;
-constexpr int kGapItems = 8;
+constexpr int kGapItems = 2;  // 8 left the walks of small boxes to a block per axis (17 us a pass)
 constexpr int kGapTile = kGapThreads * kGapItems;
 
 __device__ __forceinline__ uint64_t block_max_u64(uint64_t v) {
@@ -644,27 +644,609 @@ __global__ __launch_bounds__(256) void morton_keys_kernel(Axes3 p, std::size_t n
   vals[i] = static_cast<uint32_t>(i);
 }
 
-// Tree-order copy of the sources: canonical coordinates (wrap_coord) and mass.
-// One gather through the sort order of path_key_kernel's input-order records;
-// everything after it reads the copy.
-__global__ __launch_bounds__(256) void gather_sources_kernel(const double4* __restrict__ packed, std::size_t n,
-                                                             const uint32_t* __restrict__ order,
-                                                             double4* __restrict__ pk) {
-  const std::size_t i = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  pk[i] = packed[order[i]];
-}
-
 // unwrap_coord of a canonical coordinate
 __device__ __forceinline__ double unwrap_canonical(double v, double anchor, double L) {
   return v < anchor ? v + L : v;
 }
 
-__global__ __launch_bounds__(256) void leaf_morton_kernel(const double4* __restrict__ pk, std::size_t n, UnwrapArgs u,
-                                                          MortonArgs a, uint64_t* __restrict__ mk,
-                                                          const Frame* __restrict__ fr) {
-  const std::size_t i = static_cast<std::size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// ---------------------------------------------------------------------------
+// Octree from the sorted path keys, without a pass per level.
+//
+// Let cl(i) be the number of octant digits that the keys of particles i - 1
+// and i share (-1 for i = 0), and ld(i) the depth of particle i's leaf. A cell
+// of depth d holds more than leaf_size particles around i exactly when two
+// sorted keys leaf_size apart, at and around i, share d digits, so
+//   ld(i) = 1 + max over j in [i - leaf_size, i] of common(j, j + leaf_size),
+// capped by the depth whose cells reach the smallest half size
+// (tree_gravity.cpp:1133). The nodes that begin at particle i are those of
+// depths cl(i) + 1 .. ld(i). Preorder is the order of (begin, depth), so one
+// scan of the counts ld - cl numbers the nodes in preorder; a scan per depth
+// numbers them breadth first, a node's children being consecutive and its
+// first child the next depth's node at the same particle. A node ends at the
+// first later key outside its cell, which also gives its subtree size. The
+// former discovery took three launches per level to split the nodes and two
+// more for subtree sizes and preorder (60 to 75 launches of 4 to 40 us).
+// meta = depth | octant << 8 | leaf << 16 | last sibling << 17
+constexpr int kMaxLevels = kPathLevels + 1;             // depths 0..21
+constexpr int kLvTooDeep = kMaxLevels + 1;              // lv[0, kMaxLevels]: level starts
+constexpr int kLvOverflow = kLvTooDeep + 1;             // nodes beyond the node capacity
+constexpr int kLvDeepSplit = kLvTooDeep + 2;            // a node below the partial sort's depth splits
+constexpr int kLvLeaves = kLvTooDeep + 3;               // nodes without children
+constexpr int kLvTotal = kLvTooDeep + 4;                // node count
+constexpr int kLvDepth = kLvTooDeep + 5;                // deepest level with nodes
+constexpr int kLvSubs = kLvTooDeep + 6;                 // moment subtrees
+constexpr int kLvTops = kLvTooDeep + 7;                 // per depth: nodes above the moment subtrees
+constexpr int kLvWords = kLvTops + kMaxLevels;
+
+constexpr int kNodeThreads = 512;                       // particles per block of the node passes
+constexpr int kNodeRows = kMaxLevels + 1;               // per-block counts: nodes of each depth, all nodes
+constexpr uint32_t kMaxLeafSize = 1024;
+
+// What a build reads back: the level words, and with a device frame the source
+// statistics and the unwrap result.
+struct BuildReport {
+  uint32_t lv[kLvWords];
+  uint32_t pad;
+  SourceStats stats;
+  UnwrapResult unwrap;
+};
+
+struct NodeArgs {
+  uint32_t n, leaf_size;
+  int sorted_levels;   // digits the keys are sorted by
+  uint32_t nblk;       // blocks of kNodeThreads particles
+  double c0[3], h0;    // root cube (unless a frame is given)
+  uint32_t capacity;   // node arrays
+  uint32_t cut;        // moment subtrees hold at most this many particles
+  uint32_t max_top;    // nodes of one depth above them, at most
+};
+
+// octant digits two keys share, at most `levels`
+__device__ __forceinline__ int common_digits(uint64_t a, uint64_t b, int levels) {
+  const uint64_t x = a ^ b;
+  const int c = x == 0 ? kPathLevels : (__clzll(static_cast<long long>(x)) - 1) / 3;
+  return c < levels ? c : levels;
+}
+
+// depth whose cells have half <= 1e-12 (they are leaves whatever they hold), or kMaxLevels
+__device__ __forceinline__ int smallest_cell_depth(double half) {
+  int d = 0;
+  while (d < kMaxLevels && !(half <= 1.0e-12)) {
+    half = 0.5 * half;
+    ++d;
+  }
+  return d;
+}
+
+// cl + 1 and ld of every particle (cld = cl + 1 | ld << 8), and per block the
+// node counts of each depth and in all (cnt[row * nblk + block]).
+__global__ __launch_bounds__(kNodeThreads) void node_count_kernel(NodeArgs a, const uint64_t* __restrict__ keys,
+                                                                  uint16_t* __restrict__ cld,
+                                                                  uint32_t* __restrict__ cnt,
+                                                                  uint32_t* __restrict__ flags,
+                                                                  const Frame* __restrict__ fr) {
+  __shared__ int win[2][kNodeThreads + kMaxLeafSize];
+  __shared__ uint32_t hist[kNodeRows];
+  __shared__ uint32_t leaves;
+  const int t = threadIdx.x;
+  const int64_t base = static_cast<int64_t>(blockIdx.x) * kNodeThreads;
+  const int leaf = static_cast<int>(a.leaf_size), len = kNodeThreads + leaf;
+  if (t < kNodeRows) hist[t] = 0;
+  if (t == 0) leaves = 0;
+  for (int k = t; k < len; k += kNodeThreads) {
+    const int64_t j = base - leaf + k;
+    win[0][k] = j >= 0 && j + leaf < static_cast<int64_t>(a.n)
+                    ? common_digits(keys[j], keys[j + leaf], a.sorted_levels)
+                    : -1;
+  }
+  __syncthreads();
+  // maxima over 2, 4, .. entries while they fit the window of leaf + 1
+  int cur = 0, span = 1;
+  while (2 * span <= leaf + 1) {
+    for (int k = t; k < len; k += kNodeThreads) {
+      const int v = win[cur][k], o = k + span < len ? win[cur][k + span] : -1;
+      win[cur ^ 1][k] = v > o ? v : o;
+    }
+    cur ^= 1;
+    span *= 2;
+    __syncthreads();
+  }
+  const int64_t i = base + t;
+  const bool in = i < static_cast<int64_t>(a.n);
+  const int s0 = win[cur][t], s1 = win[cur][t + leaf + 1 - span];
+  const int split = s0 > s1 ? s0 : s1;  // deepest cell around i with more than leaf_size particles
+  const int cap = smallest_cell_depth(fr ? fr->half : a.h0);
+  int cl = -1, ld = -1;
+  bool deep = false, too = false;
+  if (in) {
+    cl = i == 0 ? -1 : common_digits(keys[i - 1], keys[i], a.sorted_levels);
+    ld = split + 1 < cap ? split + 1 : cap;
+    if (split >= a.sorted_levels && cap > a.sorted_levels) {
+      deep = a.sorted_levels < kPathLevels;
+      too = !deep;
+      ld = a.sorted_levels;
+    }
+    cld[i] = static_cast<uint16_t>((cl + 1) | (ld << 8));
+  }
+  if (__ballot(deep) && lane_id() == 0) atomicOr(&flags[kLvDeepSplit], 1u);
+  if (__ballot(too) && lane_id() == 0) atomicOr(&flags[kLvTooDeep], 1u);
+  const int dmax = static_cast<int>(wave_max_u32(static_cast<uint32_t>(ld + 1))) - 1;
+  uint32_t all = 0;
+  for (int d = 0; d <= dmax; ++d) {
+    const uint32_t c = static_cast<uint32_t>(__popcll(__ballot(in && cl < d && d <= ld)));
+    all += c;
+    if (c && lane_id() == 0) atomicAdd(&hist[d], c);
+  }
+  const uint32_t lf = static_cast<uint32_t>(__popcll(__ballot(in && cl < ld)));
+  if (lane_id() == 0) {
+    if (all) atomicAdd(&hist[kMaxLevels], all);
+    if (lf) atomicAdd(&leaves, lf);
+  }
+  __syncthreads();
+  if (t < kNodeRows) cnt[static_cast<std::size_t>(t) * a.nblk + blockIdx.x] = hist[t];
+  if (t == 0 && leaves) atomicAdd(&flags[kLvLeaves], leaves);
+}
+
+// Level starts, node count and deepest level from the row totals; the report
+// of the build. A capture-safe build reads nothing back: a tree beyond the
+// prepared capacity or sorted depth, or deeper than 21 levels, sets fault bits
+// and becomes empty.
+__global__ __launch_bounds__(64) void node_levels_kernel(NodeArgs a, const uint32_t* __restrict__ totals,
+                                                         BuildReport* __restrict__ rep,
+                                                         const SourceStats* __restrict__ stats,
+                                                         const UnwrapResult* __restrict__ unwrap,
+                                                         unsigned long long* __restrict__ fault) {
+  const int t = threadIdx.x;
+  uint32_t* lv = rep->lv;
+  if (t < kMaxLevels) lv[kLvTops + t] = 0;
+  if (t != 0) return;
+  uint32_t run = 0, depth = 0;
+  for (int d = 0; d < kMaxLevels; ++d) {
+    lv[d] = run;
+    if (totals[d]) depth = static_cast<uint32_t>(d);
+    run += totals[d];
+  }
+  lv[kMaxLevels] = run;
+  lv[kLvTotal] = run;
+  lv[kLvDepth] = depth;
+  lv[kLvSubs] = 0;
+  lv[kLvOverflow] = run > a.capacity ? 1u : 0u;
+  if (stats) rep->stats = *stats;
+  if (unwrap) rep->unwrap = *unwrap;
+  if (fault) {
+    unsigned long long f = 0;
+    if (lv[kLvOverflow] || lv[kLvDeepSplit]) f |= kFaultPrepared;
+    if (lv[kLvTooDeep]) f |= kFaultTooDeep;
+    if (f) {
+      for (int d = 0; d <= kMaxLevels; ++d) lv[d] = 0;
+      lv[kLvTotal] = 0;
+      atomicOr(fault, f);
+    }
+  }
+}
+
+struct NodeArrays {
+  uint32_t *begin, *count, *first_child, *nchild, *meta, *pre, *subtree;
+  double4* geo;
+};
+
+// Writes the nodes that begin at each particle (breadth-first slots): begin,
+// depth and octant, preorder index, cell, first child. The cell is the root's
+// halved along the key's digits, the arithmetic of the path keys.
+__global__ __launch_bounds__(kNodeThreads) void node_emit_kernel(NodeArgs a, const uint64_t* __restrict__ keys,
+                                                                 const uint16_t* __restrict__ cld,
+                                                                 const uint32_t* __restrict__ offs,
+                                                                 const uint32_t* __restrict__ lv, NodeArrays o,
+                                                                 uint32_t* __restrict__ pbase,
+                                                                 const Frame* __restrict__ fr) {
+  __shared__ uint32_t wcnt[kNodeThreads / kWave][kNodeRows];
+  __shared__ uint32_t start[kNodeRows];
+  if (lv[kLvTotal] == 0 || lv[kLvTotal] > a.capacity) return;  // block-uniform
+  const int t = threadIdx.x, w = t / kWave, lane = lane_id();
+  const uint32_t i = blockIdx.x * kNodeThreads + t;
+  const bool in = i < a.n;
+  int cl = -1, ld = -2;
+  uint64_t key = 0;
+  if (in) {
+    const uint32_t v = cld[i];
+    cl = static_cast<int>(v & 0xFFu) - 1;
+    ld = static_cast<int>(v >> 8);
+    key = keys[i];
+  }
+  const int dmax = static_cast<int>(wave_max_u32(static_cast<uint32_t>(ld + 2))) - 2;
+  if (t < kNodeRows) {
+    start[t] = (t < kMaxLevels ? lv[t] : 0u) + offs[static_cast<std::size_t>(t) * a.nblk + blockIdx.x];
+  }
+  if (lane < kNodeRows) wcnt[w][lane] = 0;
+  __builtin_amdgcn_wave_barrier();
+  const uint32_t mine = in && ld > cl ? static_cast<uint32_t>(ld - cl) : 0u;
+  for (int d = 0; d <= dmax; ++d) {
+    const uint32_t c = static_cast<uint32_t>(__popcll(__ballot(in && cl < d && d <= ld)));
+    if (lane == 0) wcnt[w][d] = c;
+  }
+  uint32_t inc = mine;
+#pragma unroll
+  for (int off = 1; off < kWave; off <<= 1) {
+    const uint32_t u = __shfl_up(inc, off, kWave);
+    if (lane >= off) inc += u;
+  }
+  if (lane == kWave - 1) wcnt[w][kMaxLevels] = inc;
+  __syncthreads();
+  uint32_t pb = start[kMaxLevels] + inc - mine;
+  for (int k = 0; k < w; ++k) pb += wcnt[k][kMaxLevels];
+  if (in) pbase[i] = pb;
+  double cx, cy, cz, h;
+  if (fr) {
+    cx = fr->centre[0];
+    cy = fr->centre[1];
+    cz = fr->centre[2];
+    h = fr->half;
+  } else {
+    cx = a.c0[0];
+    cy = a.c0[1];
+    cz = a.c0[2];
+    h = a.h0;
+  }
+  uint32_t prev = kInvalidIndex;  // this particle's node one depth up
+  for (int d = 0; d <= dmax; ++d) {
+    const bool on = in && cl < d && d <= ld;
+    uint32_t oct = 0;
+    if (d > 0) {
+      oct = static_cast<uint32_t>(key >> (3 * (kPathLevels - d))) & 7u;
+      const double ch = 0.5 * h;
+      cx = cx + ((oct & 4u) ? ch : -ch);
+      cy = cy + ((oct & 2u) ? ch : -ch);
+      cz = cz + ((oct & 1u) ? ch : -ch);
+      h = ch;
+    }
+    const unsigned long long m = __ballot(on);
+    if (m == 0) continue;
+    uint32_t slot = start[d] + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
+    for (int k = 0; k < w; ++k) slot += wcnt[k][d];
+    if (on) {
+      o.begin[slot] = i;
+      o.meta[slot] = static_cast<uint32_t>(d) | (oct << 8) | (d == ld ? 1u << 16 : 0u) | (d == 0 ? 1u << 17 : 0u);
+      o.pre[slot] = pb + static_cast<uint32_t>(d - cl - 1);
+      o.geo[slot] = make_double4(cx, cy, cz, h);
+      if (d == ld) o.first_child[slot] = kInvalidIndex;
+      if (prev != kInvalidIndex) o.first_child[prev] = slot;
+      prev = slot;
+    }
+  }
+}
+
+// Per node: particle count, subtree size, child count and the last child's
+// mark; the moment passes' work lists: subtrees of at most a.cut particles
+// whose parent holds more, and the nodes above them by depth.
+__global__ __launch_bounds__(256) void node_links_kernel(NodeArgs a, const uint64_t* __restrict__ keys,
+                                                         uint32_t* __restrict__ lv, NodeArrays o,
+                                                         const uint32_t* __restrict__ pbase,
+                                                         uint32_t* __restrict__ subs, uint32_t* __restrict__ tops) {
+  const uint32_t total = lv[kLvTotal];
+  if (total > a.capacity) return;
+  for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < total; b += gridDim.x * blockDim.x) {
+    const uint32_t i = o.begin[b], meta = o.meta[b];
+    const int d = static_cast<int>(meta & 0xFFu);
+    const bool leaf = (meta >> 16) & 1u;
+    uint32_t end = a.n;
+    if (d > 0) {
+      const int sh = 3 * (kPathLevels - d);
+      const uint64_t cell = keys[i] >> sh;
+      // keys[lo] is in the cell, keys[hi] is not (or hi = n)
+      uint32_t lo = i, step = a.leaf_size < 16u ? a.leaf_size : 16u;
+      uint32_t hi = i + step < a.n && i + step > i ? i + step : a.n;
+      while (hi < a.n && (keys[hi] >> sh) == cell) {
+        lo = hi;
+        step *= 2u;
+        hi = a.n - hi > step ? hi + step : a.n;
+      }
+      while (hi - lo > 1u) {
+        const uint32_t mid = lo + (hi - lo) / 2u;
+        if ((keys[mid] >> sh) == cell) lo = mid;
+        else hi = mid;
+      }
+      end = hi;
+    }
+    const uint32_t count = end - i;
+    o.count[b] = count;
+    o.subtree[b] = (end < a.n ? pbase[end] : total) - o.pre[b];
+    uint32_t c = 0;
+    const uint32_t fc = o.first_child[b];
+    if (!leaf) {
+      const uint32_t le = lv[d + 2];
+      uint32_t first = i;  // begin of child c
+      while (c < 8u && fc + c < le && first < end) {
+        const uint32_t nxt = fc + c + 1u < le ? o.begin[fc + c + 1u] : a.n;
+        const uint32_t ce = nxt < end ? nxt : end;
+        if (count > a.cut && ce - first <= a.cut) subs[atomicAdd(&lv[kLvSubs], 1u)] = fc + c;
+        first = nxt;
+        ++c;
+      }
+      if (c) atomicOr(&o.meta[fc + c - 1u], 1u << 17);
+    }
+    o.nchild[b] = c;
+    if (d == 0 && count <= a.cut) subs[atomicAdd(&lv[kLvSubs], 1u)] = b;
+    if (count > a.cut) tops[static_cast<std::size_t>(d) * a.max_top + atomicAdd(&lv[kLvTops + d], 1u)] = b;
+  }
+}
+
+// Multipoles, bottom up (tree_gravity.cpp:1208-1380, same operation order). A
+// particle or child has a lane: its terms go to LDS, and one lane per sum adds
+// them in tree order, so a wave's loads are independent and contiguous. One
+// thread per node left a wave to chains of dependent loads (all nodes: 128^3
+// 270 us, 256^3 983 us).
+struct MomArgs {
+  UnwrapArgs u;
+  int quad;
+  uint32_t done;  // leaves of at most this many particles have their moments from the leaf pass
+};
+
+struct MomArrays {
+  const double4* pk;
+  const uint32_t *begin, *count, *nchild, *first_child;
+  const double4* geo;
+  double4* mom;
+  double* quad;  // 8 per node
+  double* box;   // 6 per node: the tight bounding box of its particles (unwrapped), lo[3], hi[3]
+};
+
+constexpr int kSumTerms = 7;
+constexpr int kSumStride = kWave + 2;  // doubles: the lanes of a group's sums read different banks
+using WaveTerms = double[kSumTerms * kSumStride];
+
+// Lane l < N of every group of G lanes adds term l of the group's first
+// `steps` lanes to `acc`, in lane order. All lanes active, steps wave-uniform.
+template <int G, int N>
+__device__ __forceinline__ double ordered_sums(WaveTerms& buf, const double (&v)[N], uint32_t steps, double acc) {
+  const int lane = lane_id(), l = lane % G;
+#pragma unroll
+  for (int k = 0; k < N; ++k) buf[k * kSumStride + lane] = v[k];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  const double* src = &buf[(l < N ? l : 0) * kSumStride + lane - l];
+  for (uint32_t j = 0; j < steps; ++j) acc += src[j];
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  return acc;
+}
+
+// Minima and maxima over groups of G consecutive lanes (8, 16 or 64), in every
+// lane. All lanes must be active.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const uint64_t b = static_cast<uint64_t>(__double_as_longlong(v));
+  const uint32_t lo = CHUI_DPP(static_cast<uint32_t>(b), CTRL, 0xf, 0u);
+  const uint32_t hi = CHUI_DPP(static_cast<uint32_t>(b >> 32), CTRL, 0xf, 0u);
+  return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
+}
+template <int G, class Op>
+__device__ __forceinline__ double group_reduce(double v, Op op) {
+  v = op(v, dpp_f64<0xb1>(v));                // quad_perm [1,0,3,2]
+  v = op(v, dpp_f64<0x4e>(v));                // quad_perm [2,3,0,1]
+  v = op(v, dpp_f64<0x141>(v));               // row_half_mirror: the other quad of 8
+  if (G >= 16) v = op(v, dpp_f64<0x140>(v));  // row_mirror: the other 8 of 16
+  if (G >= 32) v = op(v, __shfl_xor(v, 16, kWave));
+  if (G >= 64) v = op(v, __shfl_xor(v, 32, kWave));
+  return v;
+}
+template <int G>
+__device__ __forceinline__ double group_min(double v) {
+  return group_reduce<G>(v, [](double x, double y) { return fmin(x, y); });
+}
+template <int G>
+__device__ __forceinline__ double group_max(double v) {
+  return group_reduce<G>(v, [](double x, double y) { return fmax(x, y); });
+}
+
+// The centre of mass from lane l < 4's sums (mass and first moments), in every
+// lane; lane l stores its component.
+template <int G>
+__device__ __forceinline__ double4 mass_centre(const MomArrays& o, uint32_t node, bool store, const double4& g,
+                                               double sum) {
+  const int lane = lane_id(), l = lane % G, first = lane - l;
+  const double tm = __shfl(sum, first, kWave);
+  const bool on = tm > 0.0;
+  const double c = l == 1 ? g.x : l == 2 ? g.y : g.z;
+  const double v = l == 0 ? tm : on ? sum / tm : c;
+  if (store && l < 4) reinterpret_cast<double*>(o.mom + node)[(l + 3) & 3] = v;
+  return make_double4(__shfl(v, first + 1, kWave), __shfl(v, first + 2, kWave), __shfl(v, first + 3, kWave), tm);
+}
+
+// Lane l < 7 stores its quadrupole value, lane 7 the distance of the centre of
+// mass from the cell's centre; the box is stored by lane 0.
+template <int G>
+__device__ __forceinline__ void store_quad_box(const MomArrays& o, uint32_t node, bool store, const double4& g,
+                                               const double4& M, double q, const double (&lo)[3],
+                                               const double (&hi)[3]) {
+  const int l = lane_id() % G;
+  if (store && l < 8) {
+    const double ox = g.x - M.x, oy = g.y - M.y, oz = g.z - M.z;
+    o.quad[8ull * node + l] = l == 7 ? sqrt(ox * ox + oy * oy + oz * oz) : M.w > 0.0 ? q : 0.0;
+  }
+  if (store && l == 0) {
+    double2* bx = reinterpret_cast<double2*>(o.box + 6ull * node);
+    bx[0] = make_double2(lo[0], lo[1]);
+    bx[1] = make_double2(lo[2], hi[0]);
+    bx[2] = make_double2(hi[1], hi[2]);
+  }
+}
+
+// Lane l < 6's second moments (xx, xy, xz, yy, yz, zz) to the traceless
+// quadrupole, lane 6 the trace.
+template <int G>
+__device__ __forceinline__ double traceless(double s) {
+  const int lane = lane_id(), l = lane % G, first = lane - l;
+  const double tr = __shfl(s, first, kWave) + __shfl(s, first + 3, kWave) + __shfl(s, first + 5, kWave);
+  return l == 6 ? tr : l == 0 || l == 3 || l == 5 ? 3.0 * s - tr : 3.0 * s;
+}
+
+// Moments of leaves whose particles lie one to a lane of a group of G lanes in
+// tree order (on: mass and unwrapped position), at most `steps` in a group.
+template <int G>
+__device__ __forceinline__ void leaf_moments(const MomArgs& a, const MomArrays& o, WaveTerms& buf, uint32_t node,
+                                             bool leaf, bool any, bool on, uint32_t steps, double mass, double ux,
+                                             double uy, double uz) {
+  const double4 g = leaf ? o.geo[node] : make_double4(0.0, 0.0, 0.0, 0.0);
+  const double mm = on ? mass : 0.0;
+  double lo[3] = {group_min<G>(on ? ux : INFINITY), group_min<G>(on ? uy : INFINITY), group_min<G>(on ? uz : INFINITY)};
+  double hi[3] = {group_max<G>(on ? ux : -INFINITY), group_max<G>(on ? uy : -INFINITY),
+                  group_max<G>(on ? uz : -INFINITY)};
+  if (!any) {
+    lo[0] = hi[0] = g.x;
+    lo[1] = hi[1] = g.y;
+    lo[2] = hi[2] = g.z;
+  }
+  const double t4[4] = {mm, on ? mm * ux : 0.0, on ? mm * uy : 0.0, on ? mm * uz : 0.0};
+  const double4 M = mass_centre<G>(o, node, leaf, g, ordered_sums<G>(buf, t4, steps, 0.0));
+  double q = 0.0;
+  if (a.quad) {  // wave-uniform
+    const double rx = ux - M.x, ry = uy - M.y, rz = uz - M.z;
+    const double t6[6] = {on ? mm * rx * rx : 0.0, on ? mm * rx * ry : 0.0, on ? mm * rx * rz : 0.0,
+                          on ? mm * ry * ry : 0.0, on ? mm * ry * rz : 0.0, on ? mm * rz * rz : 0.0};
+    q = traceless<G>(ordered_sums<G>(buf, t6, steps, 0.0));
+  }
+  store_quad_box<G>(o, node, leaf, g, M, q, lo, hi);
+}
+
+// Moments of a leaf of any size by one whole wave, 64 particles at a time.
+__device__ __forceinline__ void leaf_moments_wave(const MomArgs& a, const MomArrays& o, WaveTerms& buf,
+                                                  uint32_t node) {
+  const uint32_t b = o.begin[node], c = o.count[node];
+  const double4 g = o.geo[node];
+  double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  double sum = 0.0;
+  for (uint32_t k = 0; k < c; k += kWave) {  // wave-uniform
+    const uint32_t left = c - k, steps = left < kWave ? left : kWave;
+    double t4[4] = {0.0, 0.0, 0.0, 0.0};
+    if (lane_id() < steps) {
+      const double4 p = o.pk[b + k + lane_id()];
+      const double u[3] = {unwrap_canonical(p.x, a.u.anchor[0], a.u.L[0]),
+                           unwrap_canonical(p.y, a.u.anchor[1], a.u.L[1]),
+                           unwrap_canonical(p.z, a.u.anchor[2], a.u.L[2])};
+      t4[0] = p.w;
+      for (int ax = 0; ax < 3; ++ax) {
+        t4[ax + 1] = p.w * u[ax];
+        lo[ax] = fmin(lo[ax], u[ax]);
+        hi[ax] = fmax(hi[ax], u[ax]);
+      }
+    }
+    sum = ordered_sums<kWave>(buf, t4, steps, sum);
+  }
+  for (int ax = 0; ax < 3; ++ax) {
+    lo[ax] = group_min<kWave>(lo[ax]);
+    hi[ax] = group_max<kWave>(hi[ax]);
+  }
+  const double4 M = mass_centre<kWave>(o, node, true, g, sum);
+  double q = 0.0;
+  if (a.quad) {
+    for (uint32_t k = 0; k < c; k += kWave) {
+      const uint32_t left = c - k, steps = left < kWave ? left : kWave;
+      double t6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+      if (lane_id() < steps) {
+        const double4 p = o.pk[b + k + lane_id()];
+        const double rx = unwrap_canonical(p.x, a.u.anchor[0], a.u.L[0]) - M.x;
+        const double ry = unwrap_canonical(p.y, a.u.anchor[1], a.u.L[1]) - M.y;
+        const double rz = unwrap_canonical(p.z, a.u.anchor[2], a.u.L[2]) - M.z;
+        t6[0] = p.w * rx * rx;
+        t6[1] = p.w * rx * ry;
+        t6[2] = p.w * rx * rz;
+        t6[3] = p.w * ry * ry;
+        t6[4] = p.w * ry * rz;
+        t6[5] = p.w * rz * rz;
+      }
+      q = ordered_sums<kWave>(buf, t6, steps, q);
+    }
+    q = traceless<kWave>(q);
+  }
+  store_quad_box<kWave>(o, node, true, g, M, q, lo, hi);
+}
+
+// Moments of eight nodes per wave, a child to a lane (c: children of the
+// group's node, 0 for none).
+__device__ __forceinline__ void inner_moments(const MomArgs& a, const MomArrays& o, WaveTerms& buf, uint32_t node,
+                                              uint32_t c) {
+  const uint32_t j = lane_id() & 7u;
+  const bool inner = c > 0u, child = j < c;
+  double4 g = make_double4(0.0, 0.0, 0.0, 0.0), cm = g;
+  double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  double cq[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  if (inner) g = o.geo[node];
+  if (child) {
+    const uint32_t ch = o.first_child[node] + j;
+    cm = o.mom[ch];
+    const double2* bx = reinterpret_cast<const double2*>(o.box + 6ull * ch);
+    const double2 b0 = bx[0], b1 = bx[1], b2 = bx[2];
+    lo[0] = b0.x; lo[1] = b0.y; lo[2] = b1.x;
+    hi[0] = b1.y; hi[1] = b2.x; hi[2] = b2.y;
+    if (a.quad) {
+      const double4* qd = reinterpret_cast<const double4*>(o.quad + 8ull * ch);
+      const double4 q0 = qd[0], q1 = qd[1];
+      cq[0] = q0.x; cq[1] = q0.y; cq[2] = q0.z; cq[3] = q0.w;
+      cq[4] = q1.x; cq[5] = q1.y; cq[6] = q1.z;
+    }
+  }
+#pragma unroll
+  for (int ax = 0; ax < 3; ++ax) {
+    lo[ax] = group_min<8>(lo[ax]);
+    hi[ax] = group_max<8>(hi[ax]);
+  }
+  const double t4[4] = {cm.w, cm.w * cm.x, cm.w * cm.y, cm.w * cm.z};
+  const double4 M = mass_centre<8>(o, node, inner, g, ordered_sums<8>(buf, t4, 8u, 0.0));
+  double q = 0.0;
+  if (a.quad) {  // wave-uniform
+    const double dx = child ? cm.x - M.x : 0.0, dy = child ? cm.y - M.y : 0.0, dz = child ? cm.z - M.z : 0.0;
+    const double mm = cm.w, d2 = dx * dx + dy * dy + dz * dz;
+    const double t7[7] = {cq[0] + mm * (3.0 * dx * dx - d2), cq[1] + mm * (3.0 * dx * dy),
+                          cq[2] + mm * (3.0 * dx * dz),      cq[3] + mm * (3.0 * dy * dy - d2),
+                          cq[4] + mm * (3.0 * dy * dz),      cq[5] + mm * (3.0 * dz * dz - d2),
+                          cq[6] + mm * d2};
+    q = ordered_sums<8>(buf, t7, 8u, 0.0);
+  }
+  store_quad_box<8>(o, node, inner, g, M, q, lo, hi);
+}
+
+// Moments of eight nodes (on: the lane's group has one). Leaves beyond the leaf
+// pass are summed by the whole wave, one by one.
+__device__ __forceinline__ void node_moments(const MomArgs& a, const MomArrays& o, WaveTerms& buf, uint32_t node,
+                                             bool on) {
+  const uint32_t c = on ? o.nchild[node] : 0u;
+  if (__ballot(c > 0u)) inner_moments(a, o, buf, node, c);
+  unsigned long long big = __ballot(on && c == 0u && (lane_id() & 7u) == 0u && o.count[node] > a.done);
+  while (big) {
+    const int l = __ffsll(static_cast<long long>(big)) - 1;
+    big &= big - 1ull;
+    leaf_moments_wave(a, o, buf, readlane_u32(node, l));
+  }
+}
+
+// In-leaf Morton order (tree_ordering.cpp:151): the (Morton key, row) ranks of
+// a leaf's particles by comparison, G lanes per node; leaves of more than G
+// particles are ranked by the whole wave. Reads the sort's order and the
+// input-order records, writes the final order and the tree-order copy of the
+// sources (canonical coordinates and mass), so the gather, the Morton keys and
+// the permutation are one pass (256^3: 0.85 ms in three). The records move to
+// their rank's lane first: the stores are contiguous, and the leaf's moments
+// are summed in tree order while its particles are in registers.
+// v moved to the lane at byte address `to` / 4; all lanes active, `to` a permutation
+__device__ __forceinline__ double permute_f64(int to, double v) {
+  const uint64_t b = static_cast<uint64_t>(__double_as_longlong(v));
+  const uint32_t lo = __builtin_amdgcn_ds_permute(to, static_cast<int>(static_cast<uint32_t>(b)));
+  const uint32_t hi = __builtin_amdgcn_ds_permute(to, static_cast<int>(static_cast<uint32_t>(b >> 32)));
+  return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void leaf_order_kernel(uint32_t total_nodes, const uint32_t* __restrict__ total_dev,
+                                                         MomArgs mo, MomArrays o,
+                                                         MortonArgs a,
+                                                         const double4* __restrict__ packed,
+                                                         const uint32_t* __restrict__ order_in,
+                                                         uint32_t* __restrict__ order_out, double4* __restrict__ pk,
+                                                         const Frame* __restrict__ fr) {
+  const uint32_t total = total_dev ? *total_dev : total_nodes;
+  __shared__ WaveTerms terms[256 / kWave];
+  UnwrapArgs& u = mo.u;
   if (fr) {
     for (int ax = 0; ax < 3; ++ax) {
       u.anchor[ax] = fr->anchor[ax];
@@ -672,493 +1254,136 @@ __global__ __launch_bounds__(256) void leaf_morton_kernel(const double4* __restr
     }
     a.extent = fr->mext;
   }
-  const double4 q = pk[i];
-  mk[i] = morton_key(unwrap_canonical(q.x, u.anchor[0], u.L[0]), unwrap_canonical(q.y, u.anchor[1], u.L[1]),
-                     unwrap_canonical(q.z, u.anchor[2], u.L[2]), a);
-}
-
-// ---------------------------------------------------------------------------
-// Level-synchronous node discovery on the sorted path keys (BFS numbering).
-// meta = depth | octant << 8 | leaf << 16 | last sibling << 17
-__device__ __forceinline__ uint32_t lower_bound_digit(const uint64_t* __restrict__ k, uint32_t b, uint32_t e,
-                                                      int shift, uint32_t digit) {
-  while (b < e) {
-    const uint32_t mid = b + ((e - b) >> 1);
-    if (static_cast<uint32_t>((k[mid] >> shift) & 7u) < digit) b = mid + 1;
-    else e = mid;
-  }
-  return b;
-}
-
-// ---- level discovery driven from the device ---------------------------------
-// One level of the octree per three launches, with the level's node range read
-// from the device (lv[d], lv[d + 1]), so the host issues every level without
-// reading anything back and reads the level starts and flags once at the end.
-// A level's nodes are split into up to kLevelBlocks contiguous chunks, one per
-// block. Count: eight threads per node, thread o of a splitting node
-// binary-searches the first particle of octant o (the searches are
-// independent, so a level costs one search depth rather than seven); the
-// octant boundaries are kept for the emit pass and the group counts the
-// non-empty octants. Offsets: one block turns the block sums into offsets and
-// the next level's start. Emit: each block numbers its children in node order,
-// so children are in BFS order and each node's children are contiguous in
-// octant order.
-constexpr int kLevelBlocks = 2048;
-constexpr int kMaxLevels = kPathLevels + 1;            // depths 0..21
-constexpr int kLvTooDeep = kMaxLevels + 2;              // lv[0, kMaxLevels + 2): level starts
-constexpr int kLvOverflow = kLvTooDeep + 1;             // children beyond the node capacity
-constexpr int kLvDeepSplit = kLvTooDeep + 2;            // a node below the partial sort's depth splits
-constexpr int kLvLeaves = kLvTooDeep + 3;               // nodes without children
-constexpr int kLvTotal = kLvTooDeep + 4;                // node count (capture-safe builds)
-constexpr int kLvWords = kLvTooDeep + 5;
-
-// nblocks: the grid of the count and emit passes of level d (at most
-// kLevelBlocks); the offsets pass scans that many block sums.
-struct LevelDevArgs {
-  uint32_t d, leaf_size, capacity, sorted_levels, nblocks;
-};
-
-// Grid of the count and emit passes of level d: level d holds at most
-// min(8^d, n) nodes and a block decides 32 nodes per step, so the shallow
-// levels launch a few blocks instead of kLevelBlocks.
-inline uint32_t level_blocks(int d, std::size_t n) {
-  const uint64_t bound = d >= 8 ? static_cast<uint64_t>(n) : std::min<uint64_t>(1ull << (3 * d), n);
-  return static_cast<uint32_t>(std::max<uint64_t>(1, std::min<uint64_t>(kLevelBlocks, (bound + 31) / 32)));
-}
-
-// exclusive prefix sum over the block (blockDim.x a multiple of the wave); total to *total
-__device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* wsum, uint32_t* total) {
-  const int lane = lane_id(), w = threadIdx.x / kWave, nw = blockDim.x / kWave;
-  uint32_t inc = v;
-#pragma unroll
-  for (int off = 1; off < kWave; off <<= 1) {
-    const uint32_t t = __shfl_up(inc, off, kWave);
-    if (lane >= off) inc += t;
-  }
-  if (lane == kWave - 1) wsum[w] = inc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t run = 0;
-    for (int i = 0; i < nw; ++i) {
-      const uint32_t t = wsum[i];
-      wsum[i] = run;
-      run += t;
+  auto key_of = [&](const double4& q) -> uint64_t {
+    return morton_key(unwrap_canonical(q.x, u.anchor[0], u.L[0]), unwrap_canonical(q.y, u.anchor[1], u.L[1]),
+                      unwrap_canonical(q.z, u.anchor[2], u.L[2]), a);
+  };
+  const int lane = lane_id(), sub = lane / G, l = lane % G;
+  const uint32_t per = kWave / G;
+  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave, waves = gridDim.x * blockDim.x / kWave;
+  for (uint32_t first = wave * per; first < total; first += waves * per) {  // wave-uniform
+    const uint32_t node = first + sub;
+    uint32_t b = 0, c = 0;
+    const bool leaf = node < total && o.nchild[node] == 0;
+    if (leaf) {
+      b = o.begin[node];
+      c = o.count[node];
     }
-    *total = run;
-  }
-  __syncthreads();
-  const uint32_t r = wsum[w] + inc - v;
-  __syncthreads();
-  return r;
-}
-
-__global__ __launch_bounds__(256) void level_count_dev_kernel(LevelDevArgs a, uint32_t* __restrict__ lv,
-                                                              const uint32_t* __restrict__ nb,
-                                                              const uint32_t* __restrict__ nc,
-                                                              uint32_t* __restrict__ meta,
-                                                              const double4* __restrict__ geo,
-                                                              const uint64_t* __restrict__ keys,
-                                                              uint32_t* __restrict__ nchild,
-                                                              uint32_t* __restrict__ bounds,
-                                                              uint32_t* __restrict__ bsum) {
-  __shared__ uint32_t wsum[256 / kWave];
-  __shared__ uint32_t tot;
-  const uint32_t lb = lv[a.d], cnt = lv[a.d + 1] - lb;
-  const uint32_t chunk = (cnt + gridDim.x - 1) / gridDim.x;
-  const uint32_t k0 = min(cnt, blockIdx.x * chunk), k1 = min(cnt, k0 + chunk);
-  uint32_t sum = 0, leaves = 0;
-  bool deep = false, too = false;
-  for (uint32_t base = k0; base < k1; base += blockDim.x / 8) {  // the same trip count for the whole block
-    const uint32_t k = base + threadIdx.x / 8, o = threadIdx.x & 7u;
-    const bool in = k < k1;
-    const uint32_t node = lb + (in ? k : k0);
-    const uint32_t count = in ? nc[node] : 0u;
-    const double half = in ? geo[node].w : 0.0;
-    const uint32_t depth = in ? (meta[node] & 0xFFu) : 0u;
-    const bool leaf = count <= a.leaf_size || half <= 1.0e-12;  // tree_gravity.cpp:1133
-    const bool too_deep = in && !leaf && depth >= static_cast<uint32_t>(kPathLevels);
-    const bool split = in && !leaf && !too_deep;
-    const uint32_t b = in ? nb[node] : 0u, e = b + count;
-    uint32_t lo = b;
-    if (split && o > 0) lo = lower_bound_digit(keys, b, e, 3 * (kPathLevels - 1 - static_cast<int>(depth)), o);
-    const uint32_t nxt = __shfl_down(lo, 1, 8);
-    const uint32_t hi = o == 7u ? e : nxt;
-    uint32_t c = split && hi > lo ? 1u : 0u;
-    c += __shfl_xor(c, 1, 8);
-    c += __shfl_xor(c, 2, 8);
-    c += __shfl_xor(c, 4, 8);
-    if (split) bounds[8ull * k + o] = lo;
-    if (in && o == 0u) {
-      if (split) {
-        nchild[node] = c;
-        sum += c;
-        deep = deep || depth + 1u > a.sorted_levels;
-      } else {
-        nchild[node] = 0;
-        meta[node] |= 1u << 16;
-        too = too || too_deep;
-        ++leaves;
-      }
+    const bool small = c <= static_cast<uint32_t>(G);
+    const bool on = small && static_cast<uint32_t>(l) < c;
+    uint32_t row = 0;
+    double4 q = make_double4(0.0, 0.0, 0.0, 0.0);
+    uint64_t mk = 0;
+    if (on) {
+      row = order_in[b + l];
+      q = packed[row];
+      mk = key_of(q);
     }
-  }
-  if (deep) atomicOr(&lv[kLvDeepSplit], 1u);
-  if (too) atomicOr(&lv[kLvTooDeep], 1u);
-  (void)block_exclusive_scan(leaves, wsum, &tot);
-  if (threadIdx.x == 0 && tot) atomicAdd(&lv[kLvLeaves], tot);
-  (void)block_exclusive_scan(sum, wsum, &tot);
-  if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
-}
-
-// One block of kLevelBlocks / 2 threads: block sums -> exclusive offsets and
-// the next level's start (or the overflow flag).
-__global__ __launch_bounds__(kLevelBlocks / 2) void level_offsets_dev_kernel(LevelDevArgs a, uint32_t* __restrict__ lv,
-                                                                            uint32_t* __restrict__ bsum) {
-  __shared__ uint32_t wsum[kLevelBlocks / 2 / kWave];
-  __shared__ uint32_t tot;
-  const uint32_t i = 2 * threadIdx.x;
-  const uint32_t v0 = i < a.nblocks ? bsum[i] : 0u, v1 = i + 1 < a.nblocks ? bsum[i + 1] : 0u;
-  const uint32_t off = block_exclusive_scan(v0 + v1, wsum, &tot);
-  if (i < a.nblocks) bsum[i] = off;
-  if (i + 1 < a.nblocks) bsum[i + 1] = off + v0;
-  if (threadIdx.x == 0) {
-    const uint32_t le = lv[a.d + 1];
-    const uint64_t next = static_cast<uint64_t>(le) + tot;
-    const bool over = lv[kLvOverflow] != 0u || next > a.capacity;
-    if (over) lv[kLvOverflow] = 1u;
-    lv[a.d + 2] = over ? le : static_cast<uint32_t>(next);
-  }
-}
-
-__global__ __launch_bounds__(256) void level_emit_dev_kernel(LevelDevArgs a, const uint32_t* __restrict__ lv,
-                                                             uint32_t* __restrict__ nb, uint32_t* __restrict__ nc,
-                                                             uint32_t* __restrict__ meta, double4* __restrict__ geo,
-                                                             const uint32_t* __restrict__ bounds,
-                                                             const uint32_t* __restrict__ nchild,
-                                                             const uint32_t* __restrict__ bsum,
-                                                             uint32_t* __restrict__ first_child) {
-  __shared__ uint32_t wsum[256 / kWave];
-  __shared__ uint32_t tot;
-  if (lv[kLvOverflow]) return;  // block-uniform
-  const uint32_t lb = lv[a.d], le = lv[a.d + 1], cnt = le - lb;
-  const uint32_t chunk = (cnt + gridDim.x - 1) / gridDim.x;
-  const uint32_t k0 = min(cnt, blockIdx.x * chunk), k1 = min(cnt, k0 + chunk);
-  uint32_t run = le + bsum[blockIdx.x];
-  for (uint32_t base = k0; base < k1; base += blockDim.x) {
-    const uint32_t k = base + threadIdx.x;
-    const bool in = k < k1;
-    const uint32_t node = lb + (in ? k : k0);
-    const uint32_t c = in ? nchild[node] : 0u;
-    const uint32_t pre = block_exclusive_scan(c, wsum, &tot);
-    if (in) {
-      if (c == 0) {
-        first_child[node] = kInvalidIndex;
-      } else {
-        const uint32_t depth = meta[node] & 0xFFu;
-        const uint32_t e = nb[node] + nc[node];
-        const double4 g = geo[node];
-        const uint32_t fc = run + pre;
-        first_child[node] = fc;
-        uint32_t j = 0;
-        for (uint32_t o = 0; o < 8; ++o) {
-          const uint32_t lo = bounds[8ull * k + o];
-          const uint32_t hi = o == 7 ? e : bounds[8ull * k + o + 1];
-          if (hi > lo) {
-            const uint32_t ch = fc + j++;
-            nb[ch] = lo;
-            nc[ch] = hi - lo;
-            meta[ch] = (depth + 1u) | (o << 8) | (j == c ? 1u << 17 : 0u);
-            const double chh = 0.5 * g.w;  // tree_gravity.cpp:1180-1184
-            double4 cg;
-            cg.x = g.x + ((o & 4u) ? chh : -chh);
-            cg.y = g.y + ((o & 2u) ? chh : -chh);
-            cg.z = g.z + ((o & 1u) ? chh : -chh);
-            cg.w = chh;
-            geo[ch] = cg;
-          }
+    uint32_t rank = 0;
+    const uint32_t steps = wave_max_u32(small ? c : 0u);
+    for (uint32_t k = 0; k < steps; ++k) {
+      const int src = sub * G + static_cast<int>(k);
+      const uint64_t ok = __shfl(mk, src, kWave);
+      const uint32_t orow = __shfl(row, src, kWave);
+      if (k < c && (ok < mk || (ok == mk && orow < row))) ++rank;
+    }
+    // lanes beyond the leaf keep their place, so this is a permutation of the group
+    const int to = 4 * (sub * G + (on ? static_cast<int>(rank) : l));
+    row = static_cast<uint32_t>(__builtin_amdgcn_ds_permute(to, static_cast<int>(row)));
+    q.x = permute_f64(to, q.x);
+    q.y = permute_f64(to, q.y);
+    q.z = permute_f64(to, q.z);
+    q.w = permute_f64(to, q.w);
+    if (on) {
+      order_out[b + l] = row;
+      pk[b + l] = q;
+    }
+    leaf_moments<G>(mo, o, terms[threadIdx.x / kWave], node, leaf && small, c > 0u, on, steps, q.w, unwrap_canonical(q.x, u.anchor[0], u.L[0]),
+                    unwrap_canonical(q.y, u.anchor[1], u.L[1]), unwrap_canonical(q.z, u.anchor[2], u.L[2]));
+    unsigned long long big = __ballot(!small && l == 0);
+    while (big) {
+      const int s = __ffsll(static_cast<long long>(big)) - 1;
+      big &= big - 1ull;
+      const uint32_t bb = readlane_u32(b, s), bc = readlane_u32(c, s);
+      for (uint32_t e = lane; e < bc; e += kWave) {
+        const uint32_t er = order_in[bb + e];
+        const double4 eq = packed[er];
+        const uint64_t ek = key_of(eq);
+        uint32_t r = 0;
+        for (uint32_t k = 0; k < bc; ++k) {
+          const uint32_t orow = order_in[bb + k];
+          const uint64_t ok = key_of(packed[orow]);
+          if (ok < ek || (ok == ek && orow < er)) ++r;
         }
+        order_out[bb + r] = er;
+        pk[bb + r] = eq;
       }
     }
-    run += tot;
   }
 }
 
-__global__ void level_dev_init_kernel(uint32_t* lv) {
-  const int i = threadIdx.x;
-  if (i < kLvWords) lv[i] = i == 1 ? 1u : 0u;
-}
-
-__global__ void root_init_kernel(uint32_t* nb, uint32_t* nc, uint32_t* meta, double4* geo, uint32_t n, double cx,
-                                 double cy, double cz, double h, const Frame* __restrict__ fr) {
-  nb[0] = 0;
-  nc[0] = n;
-  meta[0] = 1u << 17;
-  geo[0] = fr ? make_double4(fr->centre[0], fr->centre[1], fr->centre[2], fr->half) : make_double4(cx, cy, cz, h);
-}
-
-// A level's node range: [lb, lb + cnt) from the host, or [lv[d], lv[d + 1])
-// from the device when lv is given.
-struct LevelRange {
-  uint32_t lb, cnt;
-  const uint32_t* lv;
-  int d;
-};
-__device__ __forceinline__ void level_range(const LevelRange& r, uint32_t& lb, uint32_t& cnt) {
-  if (r.lv) {
-    lb = r.lv[r.d];
-    cnt = r.lv[r.d + 1] - lb;
-  } else {
-    lb = r.lb;
-    cnt = r.cnt;
-  }
-}
-
-// Bottom-up subtree sizes (in nodes), one level per launch.
-__global__ __launch_bounds__(256) void subtree_kernel(LevelRange r, const uint32_t* __restrict__ nchild,
-                                                      const uint32_t* __restrict__ first_child,
-                                                      uint32_t* __restrict__ subtree) {
-  uint32_t lb, cnt;
-  level_range(r, lb, cnt);
-  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < cnt; k += gridDim.x * blockDim.x) {
-    const uint32_t node = lb + k;
-    uint32_t s = 1;
-    const uint32_t c = nchild[node];
-    for (uint32_t j = 0; j < c; ++j) s += subtree[first_child[node] + j];
-    subtree[node] = s;
-  }
-}
-
-// Top-down preorder indices, one level per launch.
-__global__ __launch_bounds__(256) void preorder_kernel(LevelRange r, const uint32_t* __restrict__ nchild,
-                                                       const uint32_t* __restrict__ first_child,
-                                                       const uint32_t* __restrict__ subtree,
-                                                       uint32_t* __restrict__ pre) {
-  uint32_t lb, cnt;
-  level_range(r, lb, cnt);
-  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < cnt; k += gridDim.x * blockDim.x) {
-    const uint32_t node = lb + k;
-    uint32_t run = pre[node] + 1;
-    const uint32_t c = nchild[node];
-    for (uint32_t j = 0; j < c; ++j) {
-      const uint32_t ch = first_child[node] + j;
-      pre[ch] = run;
-      run += subtree[ch];
-    }
-  }
-}
-
-// In-leaf Morton order: insertion sort of (morton key, source row) pairs.
-__device__ __forceinline__ void leaf_sort_node(uint32_t node, const uint32_t* __restrict__ nb,
-                                               const uint32_t* __restrict__ nc, uint64_t* __restrict__ mk,
-                                               uint32_t* __restrict__ order, uint32_t* __restrict__ from,
-                                               double4* __restrict__ pk) {
-  const uint32_t b = nb[node], e = b + nc[node];
-  for (uint32_t i = b; i < e; ++i) from[i] = i;
-  for (uint32_t i = b + 1; i < e; ++i) {
-    const uint64_t kk = mk[i];
-    const uint32_t kv = order[i];
-    const uint32_t kf = from[i];
-    uint32_t j = i;
-    while (j > b && (mk[j - 1] > kk || (mk[j - 1] == kk && order[j - 1] > kv))) {
-      mk[j] = mk[j - 1];
-      order[j] = order[j - 1];
-      from[j] = from[j - 1];
-      --j;
-    }
-    mk[j] = kk;
-    order[j] = kv;
-    from[j] = kf;
-  }
-  // Apply the leaf's permutation to the source copy in place, one cycle at a
-  // time: position j takes the record that was at from[j]; a written position
-  // is marked by from[j] = j, like a fixed point.
-  for (uint32_t c = b; c < e; ++c) {
-    if (from[c] == c) continue;
-    const double4 first = pk[c];
-    uint32_t j = c;
-    for (;;) {
-      const uint32_t k = from[j];
-      from[j] = j;
-      if (k == c) {
-        pk[j] = first;
-        break;
-      }
-      pk[j] = pk[k];
-      j = k;
-    }
-  }
-}
-
-// total_dev (when given) holds the node count of a capture-safe build.
-__global__ __launch_bounds__(256) void leaf_sort_kernel(uint32_t total_nodes, const uint32_t* __restrict__ total_dev,
-                                                        const uint32_t* __restrict__ nchild,
-                                                        const uint32_t* __restrict__ nb, const uint32_t* __restrict__ nc,
-                                                        uint64_t* __restrict__ mk, uint32_t* __restrict__ order,
-                                                        uint32_t* __restrict__ from, double4* __restrict__ pk) {
-  const uint32_t total = total_dev ? *total_dev : total_nodes;
-  for (uint32_t node = blockIdx.x * blockDim.x + threadIdx.x; node < total; node += gridDim.x * blockDim.x)
-    if (nchild[node] == 0) leaf_sort_node(node, nb, nc, mk, order, from, pk);
-}
-
-// Multipoles, one BFS level per launch from the deepest level up
-// (tree_gravity.cpp:1208-1380, same operation order).
-struct MomArgs {
-  UnwrapArgs u;
-  LevelRange r;
-  int quad;
-};
-
-__device__ __forceinline__ void multipole_node(uint32_t node, const MomArgs& a, const double4* __restrict__ pk,
-                                               const uint32_t* __restrict__ nb, const uint32_t* __restrict__ nc,
-                                               const uint32_t* __restrict__ nchild,
-                                               const uint32_t* __restrict__ first_child,
-                                               const double4* __restrict__ geo, double4* __restrict__ mom,
-                                               double* __restrict__ quad, double* __restrict__ box) {
-  const double4 g = geo[node];
-  double* q = quad + 8ull * node;
-  const uint32_t c = nchild[node];
-  // tight bounding box of the node's particles (unwrapped): lo[3], hi[3]
-  double lo[3] = {g.x, g.y, g.z}, hi[3] = {g.x, g.y, g.z};
-  if (c == 0) {
-    const uint32_t b = nb[node], e = b + nc[node];
-    double tm = 0.0, wx = 0.0, wy = 0.0, wz = 0.0;
-    if (e > b) {
-      for (int ax = 0; ax < 3; ++ax) {
-        lo[ax] = INFINITY;
-        hi[ax] = -INFINITY;
-      }
-    }
-    for (uint32_t i = b; i < e; ++i) {
-      const double4 q = pk[i];
-      const double mm = q.w;
-      const double ux = unwrap_canonical(q.x, a.u.anchor[0], a.u.L[0]);
-      const double uy = unwrap_canonical(q.y, a.u.anchor[1], a.u.L[1]);
-      const double uz = unwrap_canonical(q.z, a.u.anchor[2], a.u.L[2]);
-      tm += mm;
-      wx += mm * ux;
-      wy += mm * uy;
-      wz += mm * uz;
-      lo[0] = fmin(lo[0], ux);
-      lo[1] = fmin(lo[1], uy);
-      lo[2] = fmin(lo[2], uz);
-      hi[0] = fmax(hi[0], ux);
-      hi[1] = fmax(hi[1], uy);
-      hi[2] = fmax(hi[2], uz);
-    }
-    if (box) {
-      for (int ax = 0; ax < 3; ++ax) {
-        box[6ull * node + ax] = lo[ax];
-        box[6ull * node + 3 + ax] = hi[ax];
-      }
-    }
-    double4 M = make_double4(g.x, g.y, g.z, tm);
-    if (tm > 0.0) {
-      M.x = wx / tm;
-      M.y = wy / tm;
-      M.z = wz / tm;
-    }
-    mom[node] = M;
-    double ixx = 0, ixy = 0, ixz = 0, iyy = 0, iyz = 0, izz = 0;
-    if (a.quad && tm > 0.0) {
-      for (uint32_t i = b; i < e; ++i) {
-        const double4 q = pk[i];
-        const double mm = q.w;
-        const double rx = unwrap_canonical(q.x, a.u.anchor[0], a.u.L[0]) - M.x;
-        const double ry = unwrap_canonical(q.y, a.u.anchor[1], a.u.L[1]) - M.y;
-        const double rz = unwrap_canonical(q.z, a.u.anchor[2], a.u.L[2]) - M.z;
-        ixx += mm * rx * rx;
-        ixy += mm * rx * ry;
-        ixz += mm * rx * rz;
-        iyy += mm * ry * ry;
-        iyz += mm * ry * rz;
-        izz += mm * rz * rz;
-      }
-      const double tr = ixx + iyy + izz;
-      q[0] = 3.0 * ixx - tr;
-      q[1] = 3.0 * ixy;
-      q[2] = 3.0 * ixz;
-      q[3] = 3.0 * iyy - tr;
-      q[4] = 3.0 * iyz;
-      q[5] = 3.0 * izz - tr;
-      q[6] = tr;
-    } else {
-      for (int j = 0; j < 7; ++j) q[j] = 0.0;
-    }
-    const double ox = g.x - M.x, oy = g.y - M.y, oz = g.z - M.z;
-    q[7] = sqrt(ox * ox + oy * oy + oz * oz);
-    return;
-  }
-  const uint32_t fc = first_child[node];
-  double tm = 0.0, wx = 0.0, wy = 0.0, wz = 0.0;
-  for (uint32_t j = 0; j < c; ++j) {
-    const double4 cm = mom[fc + j];
-    tm += cm.w;
-    wx += cm.w * cm.x;
-    wy += cm.w * cm.y;
-    wz += cm.w * cm.z;
-  }
-  if (box) {
-    for (int ax = 0; ax < 3; ++ax) {
-      lo[ax] = INFINITY;
-      hi[ax] = -INFINITY;
-    }
-    for (uint32_t j = 0; j < c; ++j) {
-      const double* cb = box + 6ull * (fc + j);
-      for (int ax = 0; ax < 3; ++ax) {
-        lo[ax] = fmin(lo[ax], cb[ax]);
-        hi[ax] = fmax(hi[ax], cb[3 + ax]);
-      }
-    }
-    for (int ax = 0; ax < 3; ++ax) {
-      box[6ull * node + ax] = lo[ax];
-      box[6ull * node + 3 + ax] = hi[ax];
-    }
-  }
-  double4 M = make_double4(g.x, g.y, g.z, tm);
-  if (tm > 0.0) {
-    M.x = wx / tm;
-    M.y = wy / tm;
-    M.z = wz / tm;
-  }
-  mom[node] = M;
-  if (a.quad && tm > 0.0) {
-    double qxx = 0, qxy = 0, qxz = 0, qyy = 0, qyz = 0, qzz = 0, tr = 0;
-    for (uint32_t j = 0; j < c; ++j) {
-      const double4 cm = mom[fc + j];
-      const double* cq = quad + 8ull * (fc + j);
-      const double dx = cm.x - M.x, dy = cm.y - M.y, dz = cm.z - M.z;
-      const double mm = cm.w;
-      const double d2 = dx * dx + dy * dy + dz * dz;
-      qxx += cq[0] + mm * (3.0 * dx * dx - d2);
-      qxy += cq[1] + mm * (3.0 * dx * dy);
-      qxz += cq[2] + mm * (3.0 * dx * dz);
-      qyy += cq[3] + mm * (3.0 * dy * dy - d2);
-      qyz += cq[4] + mm * (3.0 * dy * dz);
-      qzz += cq[5] + mm * (3.0 * dz * dz - d2);
-      tr += cq[6] + mm * d2;
-    }
-    q[0] = qxx; q[1] = qxy; q[2] = qxz; q[3] = qyy; q[4] = qyz; q[5] = qzz; q[6] = tr;
-  } else {
-    for (int j = 0; j < 7; ++j) q[j] = 0.0;
-  }
-  const double ox = g.x - M.x, oy = g.y - M.y, oz = g.z - M.z;
-  q[7] = sqrt(ox * ox + oy * oy + oz * oz);
-}
-
-__global__ __launch_bounds__(128) void multipole_kernel(MomArgs a, const double4* __restrict__ pk,
-                                                        const uint32_t* __restrict__ nb,
-                                                        const uint32_t* __restrict__ nc,
-                                                        const uint32_t* __restrict__ nchild,
-                                                        const uint32_t* __restrict__ first_child,
-                                                        const double4* __restrict__ geo, double4* __restrict__ mom,
-                                                        double* __restrict__ quad /* 8 per node */,
-                                                        double* __restrict__ box /* 6 per node or null */,
-                                                        const Frame* __restrict__ fr) {
+// Moments of one subtree per block, all its levels in one launch: a subtree's
+// nodes of each depth are consecutive, from the first child of the first split
+// node of the depth above to the last child of the last.
+__global__ __launch_bounds__(256) void moment_subtree_kernel(MomArgs a, MomArrays o, const uint32_t* __restrict__ lv,
+                                                             const uint32_t* __restrict__ subs,
+                                                             const Frame* __restrict__ fr) {
+  __shared__ uint32_t lo[kMaxLevels + 1], hi[kMaxLevels + 1];
+  __shared__ WaveTerms terms[256 / kWave];
   if (fr)
     for (int ax = 0; ax < 3; ++ax) a.u.anchor[ax] = fr->anchor[ax];
-  uint32_t lb, cnt;
-  level_range(a.r, lb, cnt);
-  for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < cnt; k += gridDim.x * blockDim.x)
-    multipole_node(lb + k, a, pk, nb, nc, nchild, first_child, geo, mom, quad, box);
+  const uint32_t nsub = lv[kLvTotal] ? lv[kLvSubs] : 0u;
+  for (uint32_t s = blockIdx.x; s < nsub; s += gridDim.x) {
+    __syncthreads();  // the last subtree's levels are done with lo, hi
+    if (threadIdx.x <= kMaxLevels) {
+      const uint32_t root = subs[s];
+      lo[threadIdx.x] = threadIdx.x == 0 ? root : kInvalidIndex;
+      hi[threadIdx.x] = threadIdx.x == 0 ? root + 1u : 0u;
+    }
+    __syncthreads();
+    int levels = 0;
+    for (;;) {
+      const uint32_t l0 = lo[levels], l1 = hi[levels];
+      ++levels;
+      if (levels > kMaxLevels) break;
+      uint32_t mn = kInvalidIndex, mx = 0;
+      for (uint32_t b = l0 + threadIdx.x; b < l1; b += blockDim.x) {
+        const uint32_t c = o.nchild[b];
+        if (c) {
+          const uint32_t f = o.first_child[b];
+          mn = f < mn ? f : mn;
+          mx = f + c > mx ? f + c : mx;
+        }
+      }
+      if (mx) {
+        atomicMin(&lo[levels], mn);
+        atomicMax(&hi[levels], mx);
+      }
+      __syncthreads();
+      if (hi[levels] == 0u) break;  // block-uniform
+    }
+    for (int d = levels - 1; d >= 0; --d) {
+      for (uint32_t b = lo[d] + threadIdx.x / kWave * 8u; b < hi[d]; b += blockDim.x / 8u)  // wave-uniform
+        node_moments(a, o, terms[threadIdx.x / kWave], b + lane_id() / 8u, b + lane_id() / 8u < hi[d]);
+      __syncthreads();
+    }
+  }
+}
+
+// The nodes above the subtrees, deepest level first (one block: about n / cut
+// of them per level).
+__global__ __launch_bounds__(1024) void moment_top_kernel(MomArgs a, MomArrays o, const uint32_t* __restrict__ lv,
+                                                          const uint32_t* __restrict__ tops, uint32_t max_top) {
+  __shared__ WaveTerms terms[1024 / kWave];
+  if (lv[kLvTotal] == 0) return;
+  for (int d = kPathLevels; d >= 0; --d) {
+    const uint32_t n = lv[kLvTops + d];
+    for (uint32_t k0 = threadIdx.x / kWave * 8u; k0 < n; k0 += blockDim.x / 8u) {  // wave-uniform
+      const uint32_t k = k0 + lane_id() / 8u;
+      node_moments(a, o, terms[threadIdx.x / kWave], k < n ? tops[static_cast<std::size_t>(d) * max_top + k] : 0u, k < n);
+    }
+    __syncthreads();
+  }
 }
 
 __device__ __forceinline__ uint32_t to_fixed(double c, double scale) {
@@ -1294,7 +1519,7 @@ __global__ void frame_stats_kernel(const SourceStats* __restrict__ st, const dou
     fr->canonical[a] = (lo >= 0.0 && hi < c.L[a]) ? 1 : 0;
   }
   fr->pad = 0;
-  if (f) atomicOr(fault, f);
+  if (f && fault) atomicOr(fault, f);
 }
 
 // Root cube (tree_gravity.cpp:443-452) and the in-leaf Morton frame
@@ -1317,43 +1542,11 @@ __global__ void frame_root_kernel(const UnwrapResult* __restrict__ res, Frame* _
   fr->mext = ext < 1.0e-12 ? 1.0e-12 : ext;
 }
 
-// After a capture-safe level discovery of `issued` levels: the node count,
-// and fault bits for a node capacity or depth beyond the prepared build or a
-// tree deeper than 21 levels.
-__global__ void level_check_kernel(uint32_t* __restrict__ lv, int issued, unsigned long long* __restrict__ fault) {
-  if (threadIdx.x != 0) return;
-  unsigned long long f = 0;
-  if (lv[kLvOverflow]) f |= kFaultPrepared;
-  if (lv[kLvTooDeep]) f |= kFaultTooDeep;
-  if (issued < kMaxLevels && lv[issued + 1] > lv[issued]) f |= kFaultPrepared;
-  if (f) {
-    // The tree is incomplete (children counted but not emitted, or levels left
-    // out): every level and the node count become empty, so the passes after
-    // this one, the deposit and the walk do nothing; the fault word reports it.
-    for (int d = 0; d < kLvTooDeep; ++d) lv[d] = 0;
-    lv[kLvTotal] = 0;
-    atomicOr(fault, f);
-  } else {
-    lv[kLvTotal] = lv[issued];
-  }
-}
-
 // p[0, *count) = v, the count read on the device.
 template <class T>
 __global__ __launch_bounds__(256) void fill_count_kernel(T* __restrict__ p, T v, const uint32_t* __restrict__ count) {
   const uint32_t n = *count;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
-}
-
-template <class T>
-void grow_copy(DeviceBuffer& b, std::size_t old_count, std::size_t new_count, hipStream_t s) {
-  if (new_count * sizeof(T) <= b.bytes) return;
-  DeviceBuffer nb;
-  nb.reserve(new_count * sizeof(T));
-  if (old_count) CHUI_HIP(hipMemcpyAsync(nb.ptr, b.ptr, old_count * sizeof(T), hipMemcpyDeviceToDevice, s));
-  std::swap(b.ptr, nb.ptr);
-  std::swap(b.bytes, nb.bytes);
-  CHUI_HIP(hipStreamSynchronize(s));  // old buffer freed by nb's destructor after the copy
 }
 
 // Source statistics -> host.
@@ -1552,51 +1745,55 @@ void build_tree(Tree& t, const double* x, const double* y, const double* z, cons
   t.node_count = 0;
   t.leaf_count = 0;
   t.counts_on_device = false;
-  if (!safe) {
-    t.max_depth = 0;
-    t.level_start.clear();
-  }
+  if (!safe) t.max_depth = 0;
   Axes3 p{{x, y, z}};
   Frame* fr = nullptr;
   UnwrapArgs ua{};
   for (int a = 0; a < 3; ++a) ua.L[a] = P.L[a];
-  if (safe) {
-    // statistics -> canonical flags and checks on the device
+  SourceStats* st_dev = nullptr;
+  UnwrapResult* unwrap_dev = nullptr;
+  // The canonical flags, anchors and root cube stay on the device (Frame) in a
+  // capture-safe build and for up to kFrameMax sources: an ordinary build then
+  // reads back once, after its nodes are counted, instead of four times (each
+  // read-back idles the GPU for about 30 us: 32^3 builds took 0.55 ms so).
+  // Above it the waits are below 1% of a solve, and the unwrap's min/max
+  // buffers (bounded by n per axis without a read-back) matter more.
+  if (n > 0 && (safe || n <= kFrameMax)) {
     t.frame.reserve(sizeof(Frame));
     fr = t.frame.as<Frame>();
     const unsigned nb = std::min<unsigned>(grid_for(n, 256), 1024u);
     t.bounds.reserve((1 + nb) * sizeof(SourceStats));
-    SourceStats* st = t.bounds.as<SourceStats>();
-    source_stats_kernel<<<nb, 256, 0, s>>>(p, m, n, st + 1);
+    st_dev = t.bounds.as<SourceStats>();
+    source_stats_kernel<<<nb, 256, 0, s>>>(p, m, n, st_dev + 1);
     CHUI_LAUNCH_CHECK("source_stats_kernel");
-    stats_final_kernel<<<1, 256, 0, s>>>(st + 1, nb, m, st);
+    stats_final_kernel<<<1, 256, 0, s>>>(st_dev + 1, nb, m, st_dev);
     CHUI_LAUNCH_CHECK("stats_final_kernel");
     FrameCheck fc{};
     for (int a = 0; a < 3; ++a) fc.L[a] = P.L[a];
     fc.expect_uniform = t.mass_uniform ? 1 : 0;
     fc.expect_mass = t.uniform_mass;
-    frame_stats_kernel<<<1, 64, 0, s>>>(st, m, fc, fr, P.fault);
+    frame_stats_kernel<<<1, 64, 0, s>>>(st_dev, m, fc, fr, safe ? P.fault : nullptr);
     CHUI_LAUNCH_CHECK("frame_stats_kernel");
     int unused[3] = {0, 0, 0};
-    UnwrapResult* dres = unwrap_axes(t, p, 3, n, P.L, unused, t.unwrap, s, fr);
-    frame_root_kernel<<<1, 64, 0, s>>>(dres, fr);
+    unwrap_dev = unwrap_axes(t, p, 3, n, P.L, unused, t.unwrap, s, fr);
+    frame_root_kernel<<<1, 64, 0, s>>>(unwrap_dev, fr);
     CHUI_LAUNCH_CHECK("frame_root_kernel");
-  } else {
-    const SourceStats st = compute_stats(t, p, m, n, s);
+  }
+  // Source checks, canonical flags and root cube on the host (from a read-back).
+  auto take_stats = [&](const SourceStats& st) {
     if (st.bad_coord) throw std::invalid_argument("Periodic TreePM tree geometry requires finite source coordinates");
     if (st.bad_mass)
       throw std::invalid_argument("Tree gravity requires finite coordinates and finite non-negative masses");
     if (n == 0) return;
     t.mass_uniform = st.mass_nonuniform == 0;
     t.uniform_mass = st.mass0;
-    int canonical[3];
     for (int a = 0; a < 3; ++a) {
       const double lo = host_order_key_inv(st.lo[a]);
       const double hi = host_order_key_inv(st.hi[a]);
-      canonical[a] = (lo >= 0.0 && hi < P.L[a]) ? 1 : 0;  // tree_pm_coupling.cpp:3185-3195
+      t.unwrap.canonical[a] = (lo >= 0.0 && hi < P.L[a]) ? 1 : 0;  // tree_pm_coupling.cpp:3185-3195
     }
-    unwrap_axes(t, p, 3, n, P.L, canonical, t.unwrap, s, nullptr, P.size_for_capture);
-    if (P.size_for_capture) t.frame.reserve(sizeof(Frame));
+  };
+  auto take_unwrap = [&]() {
     const UnwrapResult& U = t.unwrap;
     // Root cube (tree_gravity.cpp:443-452) from the unwrapped bounds.
     double ext = 0.0;
@@ -1608,12 +1805,22 @@ void build_tree(Tree& t, const double* x, const double* y, const double* z, cons
       ua.canonical[a] = U.canonical[a];
       ua.anchor[a] = U.anchor[a];
     }
+  };
+  if (!fr) {
+    take_stats(compute_stats(t, p, m, n, s));
+    if (n == 0) return;
+    int canonical[3];
+    for (int a = 0; a < 3; ++a) canonical[a] = t.unwrap.canonical[a];
+    unwrap_axes(t, p, 3, n, P.L, canonical, t.unwrap, s, nullptr, P.size_for_capture);
+    take_unwrap();
+    if (P.size_for_capture) t.frame.reserve(sizeof(Frame));
   }
 
   // Path keys + stable sort.
   t.keys.reserve(n * sizeof(uint64_t));
   t.keys_alt.reserve(n * sizeof(uint64_t));
   t.order.reserve(n * sizeof(uint32_t));
+  t.sort_vals.reserve(n * sizeof(uint32_t));
   t.vals_alt.reserve(n * sizeof(uint32_t));
   t.sort_scratch.reserve(radix_sort_scratch_bytes(n));
   PathArgs pa{};
@@ -1621,128 +1828,101 @@ void build_tree(Tree& t, const double* x, const double* y, const double* z, cons
   for (int a = 0; a < 3; ++a) pa.c0[a] = t.root_centre[a];
   pa.h0 = t.root_half;
   uint64_t* keys = t.keys.as<uint64_t>();
-  uint32_t* order = t.order.as<uint32_t>();
+  uint32_t* vals = t.sort_vals.as<uint32_t>();
   t.pk.reserve(n * sizeof(double4));
   t.pk_in.reserve(n * sizeof(double4));
-  path_key_kernel<<<grid_for(n, 256), 256, 0, s>>>(p, m, n, pa, keys, order, t.pk_in.as<double4>(), fr);
+  path_key_kernel<<<grid_for(n, 256), 256, 0, s>>>(p, m, n, pa, keys, vals, t.pk_in.as<double4>(), fr);
   CHUI_LAUNCH_CHECK("path_key_kernel");
-  // Sort by the bits of levels 1..16 only (6 digit passes instead of 8). This
-  // is the reference's partition order for every node up to depth 16, and the
-  // order inside a leaf is rebuilt below by (Morton key, row), so it suffices
-  // unless some depth-16 node still splits; the discovery then restarts after
-  // sorting by all 21 levels. A capture-safe build cannot restart: it sorts by
-  // all 21 levels at once (the same partition, and the same order after the
-  // in-leaf sort).
-  constexpr int kPartialSortLevels = 16;
-  constexpr int kPartialSortLow = 3 * (kPathLevels - kPartialSortLevels);
-  bool partial = !safe;
-  radix_sort_pairs(keys, order, t.keys_alt.as<uint64_t>(), t.vals_alt.as<uint32_t>(), n,
-                   partial ? kPartialSortLow : 0, 3 * kPathLevels, t.sort_scratch.ptr, s);
+  // Sort by the digits of the last build's depth + 2 levels (16 in the first
+  // build): the reference's partition order for every node up to that depth,
+  // and the order inside a leaf is rebuilt below by (Morton key, row). If a
+  // node of the last sorted level still splits, the keys are sorted on by all
+  // 21 levels and the nodes counted again. A capture-safe build cannot: it
+  // sorts by the prepared depth + 5 levels, and a deeper tree sets a fault bit.
+  int levels = safe ? t.safe_levels : (t.level_hint > 0 ? t.level_hint : 16);
+  auto sort_keys = [&](int from_level) {
+    uint64_t* alt = keys == t.keys.as<uint64_t>() ? t.keys_alt.as<uint64_t>() : t.keys.as<uint64_t>();
+    uint32_t* valt = vals == t.sort_vals.as<uint32_t>() ? t.vals_alt.as<uint32_t>() : t.sort_vals.as<uint32_t>();
+    if (radix_sort_pairs_swap(keys, vals, alt, valt, n, 3 * (kPathLevels - from_level), 3 * kPathLevels,
+                              t.sort_scratch.ptr, s)) {
+      std::swap(keys, alt);
+      std::swap(vals, valt);
+    }
+  };
+  sort_keys(levels);
 
-  // Level-synchronous discovery. Every level is issued from the host without a
-  // read-back (the kernels read each level's range from lv); the level starts
-  // and flags come back once. A node capacity too small for the tree, or a
-  // depth-16 node that splits while only levels 1..16 are sorted, restarts it.
-  // A capture-safe build issues the prepared depth + 4 levels into the
-  // prepared capacity and reads nothing back; a tree that does not fit sets a
-  // fault bit.
   const std::size_t initial_cap = std::max<std::size_t>(1024, n / 4 + 64);
-  auto ensure = [&](std::size_t need, std::size_t used) {
+  auto ensure = [&](std::size_t need) {
     if (need <= t.bfs_capacity && t.bfs_begin.ptr) return;
-    std::size_t nc = std::max({need, 2 * t.bfs_capacity, initial_cap});
-    grow_copy<uint32_t>(t.bfs_begin, used, nc, s);
-    grow_copy<uint32_t>(t.bfs_count, used, nc, s);
-    grow_copy<uint32_t>(t.bfs_first_child, used, nc, s);
-    grow_copy<uint32_t>(t.bfs_nchild, used, nc, s);
-    grow_copy<uint32_t>(t.bfs_meta, used, nc, s);
-    grow_copy<double4>(t.bfs_geo, used, nc, s);
+    const std::size_t nc = std::max({need, 2 * t.bfs_capacity, initial_cap});
+    for (DeviceBuffer* b : {&t.bfs_begin, &t.bfs_count, &t.bfs_first_child, &t.bfs_nchild, &t.bfs_meta, &t.bfs_subtree,
+                            &t.bfs_pre, &t.node_subs})
+      b->reserve(nc * sizeof(uint32_t));
+    t.bfs_geo.reserve(nc * sizeof(double4));
     t.bfs_capacity = nc;
   };
-  if (!safe) ensure(initial_cap, 0);
-  t.level_dev.reserve(kLvWords * sizeof(uint32_t));
-  t.level_scratch.reserve(kLevelBlocks * sizeof(uint32_t));
-  uint32_t* lv = t.level_dev.as<uint32_t>();
-  uint32_t* bsum = t.level_scratch.as<uint32_t>();
-  int nlevels = 0;       // BFS levels to run the per-level passes over
-  std::size_t total = 0; // node count, or the capacity for a capture-safe build
+  if (!safe) ensure(initial_cap);
+  NodeArgs na{};
+  na.n = static_cast<uint32_t>(n);
+  na.leaf_size = P.leaf_size;
+  na.nblk = static_cast<uint32_t>((n + kNodeThreads - 1) / kNodeThreads);
+  for (int a = 0; a < 3; ++a) na.c0[a] = t.root_centre[a];
+  na.h0 = t.root_half;
+  na.cut = static_cast<uint32_t>(std::max<std::size_t>(512, n / 1024));
+  na.max_top = static_cast<uint32_t>(n / na.cut + 1);
+  t.node_cld.reserve(n * sizeof(uint16_t));
+  t.node_pbase.reserve(n * sizeof(uint32_t));
+  t.node_cnt.reserve((static_cast<std::size_t>(na.nblk) + 1) * kNodeRows * sizeof(uint32_t));
+  t.node_tops.reserve(static_cast<std::size_t>(na.max_top) * kMaxLevels * sizeof(uint32_t));
+  t.level_dev.reserve(sizeof(BuildReport));
+  BuildReport* rep = t.level_dev.as<BuildReport>();
+  uint32_t* lv = rep->lv;
+  uint32_t* cnt = t.node_cnt.as<uint32_t>();
+  uint32_t* totals = cnt + static_cast<std::size_t>(na.nblk) * kNodeRows;
+  std::size_t total = 0;  // node count, or the capacity for a capture-safe build
   for (;;) {
-    const std::size_t cap = std::min<std::size_t>(t.bfs_capacity, 0xFFFFFFFFull);
-    t.level_bounds.reserve(8ull * cap * sizeof(uint32_t));
-    root_init_kernel<<<1, 1, 0, s>>>(t.bfs_begin.as<uint32_t>(), t.bfs_count.as<uint32_t>(),
-                                     t.bfs_meta.as<uint32_t>(), t.bfs_geo.as<double4>(), static_cast<uint32_t>(n),
-                                     t.root_centre[0], t.root_centre[1], t.root_centre[2], t.root_half, fr);
-    CHUI_LAUNCH_CHECK("root_init_kernel");
-    level_dev_init_kernel<<<1, 64, 0, s>>>(lv);
-    CHUI_LAUNCH_CHECK("level_dev_init_kernel");
-    auto issue_levels = [&](int d0, int d1) {
-      for (int d = d0; d < d1; ++d) {
-        const LevelDevArgs la{static_cast<uint32_t>(d), P.leaf_size, static_cast<uint32_t>(cap),
-                              static_cast<uint32_t>(partial ? kPartialSortLevels : kMaxLevels), level_blocks(d, n)};
-        level_count_dev_kernel<<<la.nblocks, 256, 0, s>>>(
-            la, lv, t.bfs_begin.as<uint32_t>(), t.bfs_count.as<uint32_t>(), t.bfs_meta.as<uint32_t>(),
-            t.bfs_geo.as<double4>(), keys, t.bfs_nchild.as<uint32_t>(), t.level_bounds.as<uint32_t>(), bsum);
-        CHUI_LAUNCH_CHECK("level_count_dev_kernel");
-        level_offsets_dev_kernel<<<1, kLevelBlocks / 2, 0, s>>>(la, lv, bsum);
-        CHUI_LAUNCH_CHECK("level_offsets_dev_kernel");
-        level_emit_dev_kernel<<<la.nblocks, 256, 0, s>>>(
-            la, lv, t.bfs_begin.as<uint32_t>(), t.bfs_count.as<uint32_t>(), t.bfs_meta.as<uint32_t>(),
-            t.bfs_geo.as<double4>(), t.level_bounds.as<uint32_t>(), t.bfs_nchild.as<uint32_t>(), bsum,
-            t.bfs_first_child.as<uint32_t>());
-        CHUI_LAUNCH_CHECK("level_emit_dev_kernel");
-      }
-    };
+    na.sorted_levels = levels;
+    na.capacity = static_cast<uint32_t>(std::min<std::size_t>(t.bfs_capacity, 0xFFFFFFFFull));
+    fill_u32(lv + kLvTooDeep, 0u, kLvTops - kLvTooDeep, s);
+    node_count_kernel<<<na.nblk, kNodeThreads, 0, s>>>(na, keys, t.node_cld.as<uint16_t>(), cnt, lv, fr);
+    CHUI_LAUNCH_CHECK("node_count_kernel");
+    exclusive_scan_rows(cnt, totals, kNodeRows, na.nblk, s);
+    node_levels_kernel<<<1, 64, 0, s>>>(na, totals, rep, fr ? st_dev : nullptr, fr ? unwrap_dev : nullptr,
+                                        safe ? P.fault : nullptr);
+    CHUI_LAUNCH_CHECK("node_levels_kernel");
     if (safe) {
-      nlevels = std::min(kMaxLevels, t.safe_levels);
-      issue_levels(0, nlevels);
-      level_check_kernel<<<1, 64, 0, s>>>(lv, nlevels, P.fault);
-      CHUI_LAUNCH_CHECK("level_check_kernel");
-      total = cap;
+      total = na.capacity;
       break;
     }
-    // Levels up to the last build's depth + 2 first (an empty level costs
-    // three launches of about 4 us each); the read-back that follows anyway
-    // tells whether the tree went deeper, and only then are the rest issued.
-    int issued = t.level_hint > 0 ? std::min(kMaxLevels, t.level_hint) : kMaxLevels;
-    issue_levels(0, issued);
-    uint32_t h[kLvWords];
-    for (;;) {
-      t.readback.read(h, lv, sizeof(h), s);
-      // level `issued` is [h[issued], h[issued + 1]), written by the last pass
-      if (issued < kMaxLevels && !h[kLvOverflow] && !(partial && h[kLvDeepSplit]) && h[issued + 1] > h[issued]) {
-        issue_levels(issued, kMaxLevels);
-        issued = kMaxLevels;
-        continue;
+    BuildReport h;
+    t.readback.read(&h, rep, sizeof(h), s);
+    if (fr) {
+      take_stats(h.stats);
+      for (int a = 0; a < 3; ++a) {
+        t.unwrap.anchor[a] = h.unwrap.anchor[a];
+        t.unwrap.umin[a] = h.unwrap.umin[a];
+        t.unwrap.umax[a] = h.unwrap.umax[a];
       }
-      break;
+      take_unwrap();
     }
-    if (partial && h[kLvDeepSplit]) {
-      // A depth-16 node splits (whether it does depends on its count, not on
-      // the unsorted low digits). Sort by every level and start over; the sort
-      // is stable, so equal keys keep their row order.
-      radix_sort_pairs(keys, order, t.keys_alt.as<uint64_t>(), t.vals_alt.as<uint32_t>(), n, 0, 3 * kPathLevels,
-                       t.sort_scratch.ptr, s);
-      partial = false;
+    if (h.lv[kLvDeepSplit]) {
+      levels = kPathLevels;
+      sort_keys(levels);
       continue;
     }
-    if (h[kLvOverflow]) {
-      ensure(2 * t.bfs_capacity, 0);
-      continue;
-    }
-    if (h[kLvTooDeep]) {
+    if (h.lv[kLvTooDeep])
       throw UnsupportedError(
           "octree deeper than 21 levels (more than max_leaf_size coincident or near-coincident particles) "
           "is not built by the GPU path yet");
-    }
-    t.level_start = {h[0], h[1]};
-    for (int d = 0; d + 1 < kMaxLevels && h[d + 2] > h[d + 1]; ++d) t.level_start.push_back(h[d + 2]);
-    t.max_depth = static_cast<uint32_t>(t.level_start.size() - 2);
-    t.leaf_count = h[kLvLeaves];
-    t.level_hint = static_cast<int>(t.max_depth) + 3;
-    t.safe_levels = std::min(kMaxLevels, static_cast<int>(t.max_depth) + 5);
+    total = h.lv[kLvTotal];
+    ensure(total);
+    na.capacity = static_cast<uint32_t>(std::min<std::size_t>(t.bfs_capacity, 0xFFFFFFFFull));
+    t.max_depth = h.lv[kLvDepth];
+    t.leaf_count = h.lv[kLvLeaves];
+    t.level_hint = std::min(kPathLevels, static_cast<int>(t.max_depth) + 2);
+    t.safe_levels = std::min(kPathLevels, static_cast<int>(t.max_depth) + 5);
     t.prepared_n = n;
     t.sized_for_capture = P.size_for_capture;
-    nlevels = static_cast<int>(t.level_start.size()) - 1;
-    total = t.level_start.back();
     break;
   }
   t.node_count = total;
@@ -1750,42 +1930,20 @@ void build_tree(Tree& t, const double* x, const double* y, const double* z, cons
   const uint32_t* total_dev = device_node_count(t);
   // node arrays: the node count, or the capacity when capture-safe builds follow
   const std::size_t nsz = P.size_for_capture ? std::max(total, t.bfs_capacity) : total;
-  // per-level passes: one launch per level; a capture-safe build reads each
-  // level's range on the device and strides a fixed grid over it
-  auto range_of = [&](int d) {
-    LevelRange r{};
-    if (safe) {
-      r.lv = lv;
-      r.d = d;
-    } else {
-      r.lb = static_cast<uint32_t>(t.level_start[d]);
-      r.cnt = static_cast<uint32_t>(t.level_start[d + 1] - t.level_start[d]);
-    }
-    return r;
-  };
-  auto level_grid = [&](int d, unsigned block) {
-    if (safe) return std::min<unsigned>(grid_for(total, block), 1024u);
-    return grid_for(t.level_start[d + 1] - t.level_start[d], block);
-  };
-  t.bfs_subtree.reserve(nsz * sizeof(uint32_t));
-  t.bfs_pre.reserve(nsz * sizeof(uint32_t));
-  t.bfs_mom.reserve(nsz * sizeof(double4));
-  t.bfs_quad.reserve(nsz * 8 * sizeof(double));
-  uint32_t* nchild = t.bfs_nchild.as<uint32_t>();
-  uint32_t* fchild = t.bfs_first_child.as<uint32_t>();
-  for (int d = nlevels - 1; d >= 0; --d) {
-    subtree_kernel<<<level_grid(d, 256), 256, 0, s>>>(range_of(d), nchild, fchild, t.bfs_subtree.as<uint32_t>());
-    CHUI_LAUNCH_CHECK("subtree_kernel");
-  }
-  fill_u32(t.bfs_pre.as<uint32_t>(), 0u, 1, s);
-  for (int d = 0; d < nlevels; ++d) {
-    preorder_kernel<<<level_grid(d, 256), 256, 0, s>>>(range_of(d), nchild, fchild, t.bfs_subtree.as<uint32_t>(),
-                                                       t.bfs_pre.as<uint32_t>());
-    CHUI_LAUNCH_CHECK("preorder_kernel");
-  }
-  // In-leaf Morton order (tree_ordering.cpp:151 extent with the 1e-12 floor).
+  const NodeArrays nodes{t.bfs_begin.as<uint32_t>(),  t.bfs_count.as<uint32_t>(), t.bfs_first_child.as<uint32_t>(),
+                         t.bfs_nchild.as<uint32_t>(), t.bfs_meta.as<uint32_t>(),  t.bfs_pre.as<uint32_t>(),
+                         t.bfs_subtree.as<uint32_t>(), t.bfs_geo.as<double4>()};
+  node_emit_kernel<<<na.nblk, kNodeThreads, 0, s>>>(na, keys, t.node_cld.as<uint16_t>(), cnt, lv, nodes,
+                                                    t.node_pbase.as<uint32_t>(), fr);
+  CHUI_LAUNCH_CHECK("node_emit_kernel");
+  const unsigned node_grid = std::min<unsigned>(grid_for(total, 256), 65536u);
+  node_links_kernel<<<node_grid, 256, 0, s>>>(na, keys, lv, nodes, t.node_pbase.as<uint32_t>(),
+                                              t.node_subs.as<uint32_t>(), t.node_tops.as<uint32_t>());
+  CHUI_LAUNCH_CHECK("node_links_kernel");
+  // In-leaf Morton order (tree_ordering.cpp:151 extent with the 1e-12 floor)
+  // and the tree-order copy of the sources.
   MortonArgs ma{};
-  if (!safe) {
+  if (!fr) {
     const UnwrapResult& U = t.unwrap;
     double mext = 0.0;
     for (int a = 0; a < 3; ++a) {
@@ -1794,28 +1952,30 @@ void build_tree(Tree& t, const double* x, const double* y, const double* z, cons
     }
     ma.extent = std::max(mext, 1.0e-12);
   }
-  uint64_t* mk = t.keys_alt.as<uint64_t>();
   double4* pk = t.pk.as<double4>();
-  gather_sources_kernel<<<grid_for(n, 256), 256, 0, s>>>(t.pk_in.as<double4>(), n, order, pk);
-  CHUI_LAUNCH_CHECK("gather_sources_kernel");
-  leaf_morton_kernel<<<grid_for(n, 256), 256, 0, s>>>(pk, n, ua, ma, mk, fr);
-  CHUI_LAUNCH_CHECK("leaf_morton_kernel");
-  leaf_sort_kernel<<<grid_for(total, 256), 256, 0, s>>>(static_cast<uint32_t>(total), total_dev, nchild,
-                                                        t.bfs_begin.as<uint32_t>(), t.bfs_count.as<uint32_t>(), mk,
-                                                        order, t.vals_alt.as<uint32_t>(), pk);
-  CHUI_LAUNCH_CHECK("leaf_sort_kernel");
-  // Multipoles and tight particle boxes bottom-up.
+  // Multipoles and tight particle boxes, the leaves' with their order, then bottom-up.
+  t.bfs_mom.reserve(nsz * sizeof(double4));
+  t.bfs_quad.reserve(nsz * 8 * sizeof(double));
   t.bfs_box.reserve(nsz * 6 * sizeof(double));
-  for (int d = nlevels - 1; d >= 0; --d) {
-    MomArgs ma2{};
-    ma2.u = ua;
-    ma2.r = range_of(d);
-    ma2.quad = P.quadrupole ? 1 : 0;
-    multipole_kernel<<<level_grid(d, 128), 128, 0, s>>>(
-        ma2, pk, t.bfs_begin.as<uint32_t>(), t.bfs_count.as<uint32_t>(), nchild, fchild,
-        t.bfs_geo.as<double4>(), t.bfs_mom.as<double4>(), t.bfs_quad.as<double>(), t.bfs_box.as<double>(), fr);
-    CHUI_LAUNCH_CHECK("multipole_kernel");
-  }
+  MomArgs mo{};
+  mo.u = ua;
+  mo.quad = P.quadrupole ? 1 : 0;
+  mo.done = P.leaf_size <= 16 ? 16u : P.leaf_size <= 32 ? 32u : 64u;  // lanes per leaf below
+  const MomArrays mv{pk, nodes.begin, nodes.count, nodes.nchild, nodes.first_child, nodes.geo,
+                     t.bfs_mom.as<double4>(), t.bfs_quad.as<double>(), t.bfs_box.as<double>()};
+  auto order_leaves = [&](auto kernel, int lanes) {
+    const unsigned grid = std::min<unsigned>(grid_for(total * lanes, 256), 65536u);
+    kernel<<<grid, 256, 0, s>>>(static_cast<uint32_t>(total), total_dev, mo, mv, ma, t.pk_in.as<double4>(), vals,
+                                t.order.as<uint32_t>(), pk, fr);
+    CHUI_LAUNCH_CHECK("leaf_order_kernel");
+  };
+  if (mo.done == 16u) order_leaves(leaf_order_kernel<16>, 16);
+  else if (mo.done == 32u) order_leaves(leaf_order_kernel<32>, 32);
+  else order_leaves(leaf_order_kernel<64>, 64);
+  moment_subtree_kernel<<<2048, 256, 0, s>>>(mo, mv, lv, t.node_subs.as<uint32_t>(), fr);
+  CHUI_LAUNCH_CHECK("moment_subtree_kernel");
+  moment_top_kernel<<<1, 1024, 0, s>>>(mo, mv, lv, t.node_tops.as<uint32_t>(), na.max_top);
+  CHUI_LAUNCH_CHECK("moment_top_kernel");
   // Preorder records: links and, for mixed builds, the fixed-point records;
   // the FP64 records for FP64 builds (or later, on demand).
   t.link.reserve(nsz * sizeof(NodeLink));
@@ -1917,6 +2077,9 @@ DepositUnits build_deposit_units(Tree& t, const DepositTiling& d, hipStream_t s)
   uint32_t* flag = t.dep_flag.as<uint32_t>();
   uint32_t* totals = t.dep_total.as<uint32_t>();  // [0] units, [1] blocks
   const uint32_t* total_dev = device_node_count(t);
+  // counts left on the device: capture-safe builds, and sources few enough for
+  // the two read-backs to matter (kFrameMax)
+  const bool on_device = total_dev || t.n <= kFrameMax;
   fill_u32(flag, 0u, total, s);
   deposit_flag_kernel<<<grid_for(total, 256), 256, 0, s>>>(static_cast<uint32_t>(total), total_dev,
                                                            t.bfs_nchild.as<uint32_t>(),
@@ -1924,7 +2087,7 @@ DepositUnits build_deposit_units(Tree& t, const DepositTiling& d, hipStream_t s)
                                                            d, flag);
   CHUI_LAUNCH_CHECK("deposit_flag_kernel");
   exclusive_scan_u32(flag, t.dep_index.as<uint32_t>(), total, totals, t.dep_scan.ptr, s);
-  if (total_dev) fill_u32(t.dep_blocks.as<uint32_t>(), 0u, total, s);  // blocks past the last unit stay 0
+  if (on_device) fill_u32(t.dep_blocks.as<uint32_t>(), 0u, total, s);  // blocks past the last unit stay 0
   deposit_emit_kernel<<<grid_for(total, 256), 256, 0, s>>>(
       static_cast<uint32_t>(total), total_dev, flag, t.dep_index.as<uint32_t>(), t.bfs_begin.as<uint32_t>(),
       t.bfs_count.as<uint32_t>(), t.bfs_box.as<double>(), d, t.dep_units.as<DepositUnit>(),
@@ -1932,10 +2095,10 @@ DepositUnits build_deposit_units(Tree& t, const DepositTiling& d, hipStream_t s)
   CHUI_LAUNCH_CHECK("deposit_emit_kernel");
   r.units = t.dep_units.as<DepositUnit>();
   r.first_block = t.dep_blocks.as<uint32_t>();
-  if (total_dev) {
-    // capture-safe: scan the blocks of every capacity slot (zero past the last
-    // unit) and leave both counts on the device; the deposit's grid is a fixed
-    // size that strides over the real block count
+  if (on_device) {
+    // scan the blocks of every node slot (zero past the last unit) and leave
+    // both counts on the device; the deposit's grid is a fixed size that
+    // strides over the real block count
     exclusive_scan_u32(t.dep_blocks.as<uint32_t>(), t.dep_blocks.as<uint32_t>(), total, totals + 1, t.dep_scan.ptr,
                        s);
     r.dev_counts = totals;
@@ -1953,7 +2116,7 @@ DepositUnits build_deposit_units(Tree& t, const DepositTiling& d, hipStream_t s)
 }
 
 const uint32_t* device_node_count(const Tree& t) {
-  return t.counts_on_device ? t.level_dev.as<uint32_t>() + kLvTotal : nullptr;
+  return t.counts_on_device ? t.level_dev.as<BuildReport>()->lv + kLvTotal : nullptr;
 }
 
 void build_pos_of_row(Tree& t, hipStream_t s) {

@@ -50,6 +50,10 @@ struct alignas(16) WalkNode {
 constexpr uint32_t kLastSibling = 0x100u;
 constexpr uint32_t kWalkNodePad = 8;  // records readable past the last node
 
+// Up to this many sources a build keeps its frame and the deposit its counts
+// on the device (one read-back per solve).
+constexpr std::size_t kFrameMax = std::size_t(1) << 21;
+
 struct UnwrapResult {
   double anchor[3];
   double umin[3], umax[3];
@@ -89,10 +93,10 @@ struct Tree {
   std::size_t node_count = 0;
   std::size_t leaf_count = 0;
   uint32_t max_depth = 0;
-  int level_hint = 0;  // levels the next build issues before its first read-back (0: all)
+  int level_hint = 0;  // octant levels the next build sorts by (0: 16)
   // Capture-safe builds: the node capacity (bfs_capacity), the source count,
-  // the mass uniformity and the levels issued (safe_levels, the prepared
-  // depth + 4) come from the last ordinary build; node_count is then the
+  // the mass uniformity and the levels sorted by (safe_levels, the prepared
+  // depth + 5) come from the last ordinary build; node_count is then the
   // capacity and the real count sits on the device (counts_on_device).
   int safe_levels = 0;
   std::size_t prepared_n = 0;
@@ -118,13 +122,13 @@ struct Tree {
   bool cubic = false;      // equal axes: the mixed records' separation unit is fixed point
   double fscale[3] = {0, 0, 0};  // 2^32 / L per axis
   // construction scratch
-  DeviceBuffer keys, keys_alt, vals_alt, sort_scratch;
+  DeviceBuffer keys, keys_alt, sort_vals, vals_alt, sort_scratch;
   DeviceBuffer bucket_min, bucket_max, block_best, block_max, occ_bytes;
   DeviceBuffer bfs_begin, bfs_count, bfs_first_child, bfs_nchild, bfs_meta, bfs_geo, bfs_subtree, bfs_pre,
-      bfs_mom, bfs_quad, bfs_box, bfs_scan, level_scratch, level_bounds, level_dev, flags, bounds;
+      bfs_mom, bfs_quad, bfs_box, bfs_scan, level_dev, bounds;
+  DeviceBuffer node_cld, node_pbase, node_cnt, node_subs, node_tops;
   DeviceBuffer dep_flag, dep_index, dep_units, dep_blocks, dep_scan, dep_total;
   std::size_t bfs_capacity = 0;
-  std::vector<std::size_t> level_start;  // BFS level ranges (host copy)
   PinnedReadback readback;               // counts and flags read back during a build
 };
 
