@@ -441,6 +441,9 @@ chui::WalkParams base_walk_params(const Ctx* c, const chui_treepm_options* o, co
   }
   wp.box_max64 = 2.0 * sp.rcut;
   wp.box_single = std::min({wp.fast_half_extent[0], wp.fast_half_extent[1], wp.fast_half_extent[2]}) >= 2u ? 1 : 0;
+  // up to 2^20 sources a pair on the other side of r_cut shows in the force
+  // field's relative L2 (walkmix_box_kernel)
+  wp.shared_origin = c->tree.n <= (1u << 20) ? 1 : 0;
   wp.node_count = static_cast<uint32_t>(c->tree.node_count);
   wp.mesh_row = mesh_row;
   return wp;
@@ -925,15 +928,6 @@ void solve_device_impl(Ctx* c, const double* x, const double* y, const double* z
           wp.rcut2_tab = static_cast<float>(wp.rcut2 * scale);
           wp.eps2_tab = static_cast<float>(wp.eps * wp.eps * scale);
           wp.force_scale = static_cast<float>(wp.G * scale * (uniform ? um : 1.0));
-          // FP64 cutoff decisions up to 2^18 sources, where a pair on the wrong
-          // side of r_cut shows in the force field's relative L2 (see
-          // walkmix_box_kernel)
-          wp.exact_pairs = n <= 262144 ? 1 : 0;
-          const double unit = wp.cubic ? o->box_size[0] / 4294967296.0 : 1.0;
-          for (int a = 0; a < 3; ++a) wp.fx_to_len64[a] = o->box_size[a] / 4294967296.0;
-          wp.sep2_to_tab = scale * unit * unit;
-          wp.eps2_tab64 = wp.eps * wp.eps * scale;
-          wp.rcut2_sep64 = wp.rcut2 / (unit * unit);
           wp.log_cells = c->ltab_cells;
           wp.log_base = static_cast<uint32_t>(c->ltab_first_octave + 127) << chui::kLogCellBits;
         }

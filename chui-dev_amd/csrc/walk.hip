@@ -2206,14 +2206,17 @@ __device__ __forceinline__ uint32_t box_segment(uint32_t seg, uint32_t per_wave,
 // second half of the window takes a batch's overflow and stages the leaves of
 // the lane-by-lane walks.
 //
-// EXACT (few sources): the pairs keep the sources' and targets' fixed-point
-// coordinates, and r^2 and its cutoff are evaluated in FP64. In FP32 a pair
+// The pairs' separations are the counting walk's: FP32 differences of offsets
+// from one origin, the centre of the 64 targets that share one of its waves,
+// or fixed-point differences where those span too much for it (SHARED). In FP32 a pair
 // within about 1e-7 of r_cut may fall on either side of it, and the residual
 // is still 1.8e-2 of Newtonian there: about one pair in 2.6e7 does, one per
-// 64^3 box, which moves a 32^3 box's force field by 2e-6 in relative L2 (2.5e-7
-// otherwise) when it happens. The FP64 form takes 27 VALU instructions per
-// pair against 16.
-template <int SCHEME, bool CUBIC, bool LOG, int WAVES, bool FRAME, bool EXACT>
+// 64^3 box, which moves a 32^3 box's force field by 2e-6 in relative L2 (1e-7
+// otherwise). So up to 2^20 sources both walks decide each pair alike; beyond,
+// where single pairs do not show, the origin is the segment's centre, which the
+// box test can share (256^3: 4 % of the solve). FP64 decisions took 27 VALU
+// instructions per pair against 16.
+template <int SCHEME, bool CUBIC, bool LOG, int WAVES, bool FRAME, bool SHARED>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(5)))
 void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long long* __restrict__ counters,
                         const NodeLink* __restrict__ node_link, const NodeGeo32* __restrict__ node_geo,
@@ -2255,6 +2258,33 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
   const float4* const lcell = ltab - P.log_base;
   const uint32_t lbase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_f32x4*)ltab - P.log_base));
 
+  const float far = 64.0f * sqrtf(rc2);
+  // --- the counting walk's origin (SHARED), else the segment's ---
+  uint32_t wox = 0, woy = 0, woz = 0;
+  bool wave_origin = false;
+  if constexpr (!SHARED) {
+    wave_origin = FRAME;
+  } else {
+    const uint32_t i = (k0 & ~(static_cast<uint32_t>(kWave) - 1u)) + lane;
+    const bool in = i < P.n_targets;
+    const uint32_t v = in ? i : k0;
+    const uint4 t = D.src32[P.identity_targets ? v : D.tpos[v]];
+    const uint32_t pp[3] = {t.x, t.y, t.z};
+    uint32_t o[3];
+    wave_origin = true;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const uint32_t o0 = readlane_u32(pp[a], 0);
+      const uint32_t off = in ? (pp[a] - o0) ^ 0x80000000u : 0x80000000u;  // ordered as unsigned
+      const int32_t lo = static_cast<int32_t>(wave_min_u32(off) ^ 0x80000000u);
+      const int32_t hi = static_cast<int32_t>(wave_max_u32(off) ^ 0x80000000u);
+      const int64_t mid = (static_cast<int64_t>(lo) + static_cast<int64_t>(hi)) / 2;
+      o[a] = o0 + static_cast<uint32_t>(static_cast<int32_t>(mid));
+      const int64_t half = (static_cast<int64_t>(hi) - static_cast<int64_t>(lo)) / 2 + 1;
+      wave_origin = wave_origin && half <= static_cast<int64_t>(P.fast_half_extent[a]);
+    }
+    wox = o[0]; woy = o[1]; woz = o[2];
+  }
   for (uint32_t seg = 0; seg < here;) {
     // --- the segment and its box ---
     uint32_t px, py, pz;
@@ -2309,7 +2339,12 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
       py = t.y;
       pz = t.z;
     }
-    const float tx = fx_delta(px, ox, u0), ty = fx_delta(py, oy, u1), tz = fx_delta(pz, oz, u2);
+    if constexpr (!SHARED) {
+      wox = ox;
+      woy = oy;
+      woz = oz;
+    }
+    const float tx = fx_delta(px, wox, u0), ty = fx_delta(py, woy, u1), tz = fx_delta(pz, woz, u2);
     float sum[3] = {0.0f, 0.0f, 0.0f}, comp[3] = {0.0f, 0.0f, 0.0f};  // Kahan totals of this lane's slice
     auto accumulate = [&](float vx, float vy, float vz) {
       kahan_add(sum[0], comp[0], vx);
@@ -2325,31 +2360,17 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
       pend = 0;
     };
     auto stage_record = [&]<bool NEAR>(const uint4& sv, float mj) -> float4 {
-      if constexpr (NEAR && !EXACT)
-        return make_float4(fx_delta(sv.x, ox, u0), fx_delta(sv.y, oy, u1), fx_delta(sv.z, oz, u2), mj);
+      if constexpr (NEAR)
+        return make_float4(fx_delta(sv.x, wox, u0), fx_delta(sv.y, woy, u1), fx_delta(sv.z, woz, u2), mj);
       else
         return make_float4(__uint_as_float(sv.x), __uint_as_float(sv.y), __uint_as_float(sv.z), mj);
     };
-    // EXACT: s of a fixed-point record, 1 beyond r_cut and below 1 inside it
-    auto exact_s = [&](const float4& sj) -> float {
-      double dx = static_cast<double>(static_cast<int32_t>(__float_as_uint(sj.x) - px));
-      double dy = static_cast<double>(static_cast<int32_t>(__float_as_uint(sj.y) - py));
-      double dz = static_cast<double>(static_cast<int32_t>(__float_as_uint(sj.z) - pz));
-      if constexpr (!CUBIC) {
-        dx *= P.fx_to_len64[0];
-        dy *= P.fx_to_len64[1];
-        dz *= P.fx_to_len64[2];
-      }
-      const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
-      const float sv = fminf(static_cast<float>(fma(r2, P.sep2_to_tab, P.eps2_tab64)), 0.99999994f);
-      return r2 <= P.rcut2_sep64 ? sv : 1.0f;
-    };
-    // One pair term; NEAR: offsets from the box centre, else fixed point.
+    // One pair term; NEAR: offsets from the origin, else fixed point.
     // UMASS: the force scale carries the mass. SEL: lanes with a negative
     // cutoff drop the term.
     auto pair = [&]<bool NEAR, bool UMASS, bool SEL>(const float4& sj, float lim, float& lx, float& ly, float& lz) {
       float dx, dy, dz;
-      if constexpr (NEAR && !EXACT) {
+      if constexpr (NEAR) {
         dx = sj.x - tx;
         dy = sj.y - ty;
         dz = sj.z - tz;
@@ -2363,7 +2384,6 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
         // s = r^2 + eps^2 clamped to [0, 1]: s >= eps^2 >= 2^first_octave, and
         // s = 1 (r_cut and beyond) is the zero cell
         float sc = __builtin_amdgcn_fmed3f(fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, eps2))), 0.0f, 1.0f);
-        if constexpr (EXACT) sc = exact_s(sj);
         const uint32_t bits = __float_as_uint(sc);
         const float4 c = lcell[bits >> kLogMantissaShift];
         const float u = static_cast<float>(bits & ((1u << kLogMantissaShift) - 1u));
@@ -2471,7 +2491,7 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
       uint32_t wn = 0;  // records in the window, below kWindow between batches
       const float4* const mine = win + slice * (TL + 1u);
       // iters records of every slice (a multiple of 4)
-      auto window_pairs = [&]<bool UMASS>(uint32_t iters) {
+      auto window_pairs = [&]<bool NEAR, bool UMASS>(uint32_t iters) {
         float lx = 0.0f, ly = 0.0f, lz = 0.0f;
         if constexpr (LOG) {
           // two table reads in flight before their polynomials are evaluated
@@ -2485,16 +2505,9 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
               for (int q = 0; q < kPairGroup; ++q) {
                 const float4 sj = mine[i0 + h + q];
                 mj[q] = sj.w;
-                if constexpr (EXACT) {
-                  dx[q] = fx_delta(__float_as_uint(sj.x), px, u0);
-                  dy[q] = fx_delta(__float_as_uint(sj.y), py, u1);
-                  dz[q] = fx_delta(__float_as_uint(sj.z), pz, u2);
-                  bits[q] = __float_as_uint(exact_s(sj));
-                  continue;
-                }
-                dx[q] = sj.x - tx;
-                dy[q] = sj.y - ty;
-                dz[q] = sj.z - tz;
+                dx[q] = NEAR ? sj.x - tx : fx_delta(__float_as_uint(sj.x), px, u0);
+                dy[q] = NEAR ? sj.y - ty : fx_delta(__float_as_uint(sj.y), py, u1);
+                dz[q] = NEAR ? sj.z - tz : fx_delta(__float_as_uint(sj.z), pz, u2);
                 bits[q] = __float_as_uint(__builtin_amdgcn_fmed3f(
                     fmaf(dx[q], dx[q], fmaf(dy[q], dy[q], fmaf(dz[q], dz[q], eps2))), 0.0f, 1.0f));
               }
@@ -2514,7 +2527,7 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
         } else {
 #pragma unroll 4
           for (uint32_t i0 = 0; i0 < iters; ++i0)
-            pair.template operator()<true, UMASS, false>(mine[i0], rc2, lx, ly, lz);
+            pair.template operator()<NEAR, UMASS, false>(mine[i0], rc2, lx, ly, lz);
         }
         psx += lx;
         psy += ly;
@@ -2527,8 +2540,14 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
         const uint32_t iters = (((cn + (1u << lgS) - 1u) >> lgS) + 3u) & ~3u;
         if (pend + iters > static_cast<uint32_t>(kWindow)) fold();
         pend += iters;
-        if (D.uniform_mass) window_pairs.template operator()<true>(iters);
-        else window_pairs.template operator()<false>(iters);
+        if (!SHARED || wave_origin) {
+          if (D.uniform_mass) window_pairs.template operator()<true, true>(iters);
+          else window_pairs.template operator()<true, false>(iters);
+        } else if (D.uniform_mass) {
+          window_pairs.template operator()<false, true>(iters);
+        } else {
+          window_pairs.template operator()<false, false>(iters);
+        }
         __builtin_amdgcn_wave_barrier();
       };
       auto slot_of = [&](uint32_t r) -> uint32_t {
@@ -2540,10 +2559,11 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
           wnode, lds, lane, frame, [&](uint32_t j) -> uint4 { return D.src32[j]; },
           [&](const uint4& sv, bool on, bool last) {
             const float mj = D.uniform_mass ? 1.0f : __uint_as_float(sv.w);
-            const float4 rec = stage_record.template operator()<true>(sv, mj);
-            const float ex = fmaxf(fabsf(EXACT ? fx_delta(sv.x, ox, u0) : rec.x) - bt0, 0.0f);
-            const float ey = fmaxf(fabsf(EXACT ? fx_delta(sv.y, oy, u1) : rec.y) - bt1, 0.0f);
-            const float ez = fmaxf(fabsf(EXACT ? fx_delta(sv.z, oz, u2) : rec.z) - bt2, 0.0f);
+            const float4 rec = !SHARED || wave_origin ? stage_record.template operator()<true>(sv, mj)
+                                           : stage_record.template operator()<false>(sv, mj);
+            const float ex = fmaxf(fabsf(SHARED ? fx_delta(sv.x, ox, u0) : rec.x) - bt0, 0.0f);
+            const float ey = fmaxf(fabsf(SHARED ? fx_delta(sv.y, oy, u1) : rec.y) - bt1, 0.0f);
+            const float ez = fmaxf(fabsf(SHARED ? fx_delta(sv.z, oz, u2) : rec.z) - bt2, 0.0f);
             const bool keep = on && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > cull2);
             const unsigned long long km = __ballot(keep);
             __builtin_amdgcn_wave_barrier();
@@ -2552,13 +2572,12 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
             while (wn >= static_cast<uint32_t>(kWindow) || (last && wn)) {
               const uint32_t cn = wn < static_cast<uint32_t>(kWindow) ? wn : static_cast<uint32_t>(kWindow);
               if (static_cast<uint32_t>(lane) >= cn) {
-                // dummies beyond r_cut of everything fill the last window
-                // (EXACT: half a period from the box centre per axis)
-                const float far = 64.0f * sqrtf(rc2);
-                win[slot_of(lane)] = EXACT ? make_float4(__uint_as_float(ox ^ 0x80000000u),
-                                                         __uint_as_float(oy ^ 0x80000000u),
-                                                         __uint_as_float(oz ^ 0x80000000u), 0.0f)
-                                           : make_float4(far, far, far, 0.0f);
+                // dummies beyond r_cut of everything fill the last window (in
+                // fixed point half a period from the box centre per axis)
+                win[slot_of(lane)] = !SHARED || wave_origin ? make_float4(far, far, far, 0.0f)
+                                                 : make_float4(__uint_as_float(ox ^ 0x80000000u),
+                                                               __uint_as_float(oy ^ 0x80000000u),
+                                                               __uint_as_float(oz ^ 0x80000000u), 0.0f);
               }
               evaluate(cn);
               wn -= cn;
@@ -2571,7 +2590,8 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
             float mx, my, mz;
             if (!__ballot(owner && accepts(pre, node_geo[pre], mx, my, mz))) return true;
             nxt = owner ? pre : end;
-            walk.template operator()<true>(end);
+            if (!SHARED || wave_origin) walk.template operator()<true>(end);
+            else walk.template operator()<false>(end);
             return false;
           });
     } else {
@@ -3524,15 +3544,13 @@ void launch_box(const WalkParams& p, const WalkData& d, const WalkOutputs& out, 
                 hipStream_t s) {
   const WalkParams q = box_params(p);
   const std::size_t lds = LOG ? p.log_cells * sizeof(float4) : 0;
-  if (LOG && q.box_single && q.exact_pairs)
-    walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, true, LOG><<<box_blocks(q, WAVES), WAVES * kWave, lds, s>>>(
-        q, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32, d.wnode);
-  else if (q.box_single)
-    walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, true, false><<<box_blocks(q, WAVES), WAVES * kWave, lds, s>>>(
-        q, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32, d.wnode);
-  else
-    walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, false, false><<<box_blocks(q, WAVES), WAVES * kWave, lds, s>>>(
-        q, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32, d.wnode);
+  const unsigned grid = box_blocks(q, WAVES);
+  const auto go = [&](auto kernel) {
+    kernel<<<grid, WAVES * kWave, lds, s>>>(q, d, out, counters, d.link, d.geo32, d.mom32, d.quad32, d.box32, d.wnode);
+  };
+  if (q.box_single && q.shared_origin) go(walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, true, true>);
+  else if (q.box_single) go(walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, true, false>);
+  else go(walkmix_box_kernel<SCHEME, CUBIC, LOG, WAVES, false, false>);
   CHUI_LAUNCH_CHECK("walkmix_box_kernel");
 }
 

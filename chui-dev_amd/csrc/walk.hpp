@@ -62,18 +62,14 @@ struct WalkParams {
   double box_max64;      // the same for the FP64 walk (length)
   int box_single;        // a single target always has a box frame (r_cut clear of L/2)
   uint32_t targets_per_wave;  // box walks: consecutive targets of a wave (8..64, a power of two)
-  // FP64 box-classified walk (solves without counters or nearest-pair lane):
-  // degree-5 cells of -H / 8 a^3 on [0, t_max] (centres 0..h64_cells, t = r^2 /
-  // 4a^2), r^2 -> cell coordinate and eps^2 (at least 1e-36).
   // Mixed timed walk with the residual table indexed by the float bits of
   // s = r^2 + eps^2 (log_cells > 0): cells (the last one, at s = 1, is zero)
   // and the (exponent, top-5-mantissa) field of the first cell.
   uint32_t log_cells, log_base;
-  // the same walk with r^2 and the cutoff in FP64 (few sources): lengths per
-  // fixed-point unit, separation unit^2 -> table units, eps^2 there, r_cut^2 in
-  // separation units
-  int exact_pairs;
-  double fx_to_len64[3], sep2_to_tab, eps2_tab64, rcut2_sep64;
+  int shared_origin;  // mixed box walk: decides each pair as the counting walk does (few sources)
+  // FP64 box-classified walk (solves without counters or nearest-pair lane):
+  // degree-5 cells of -H / 8 a^3 on [0, t_max] (centres 0..h64_cells, t = r^2 /
+  // 4a^2), r^2 -> cell coordinate and eps^2 (at least 1e-36).
   int box64;
   int h64_cells;
   double h64_scale;
