@@ -748,6 +748,7 @@ struct WalkData {
   const NodeGeo64* geo64;
   const NodeMom64* mom64;
   const NodeQuad64* quad64;
+  const uint32_t* child_index;  // group walks
   const NodeGeo32* geo32;
   const NodeMom32* mom32;
   const NodeQuad32* quad32;
@@ -1017,21 +1018,27 @@ __global__ __launch_bounds__(kWalkThreads) void walk64_kernel(WalkParams P, Walk
 //   1. checks every target's history and bounded metric; a failing group is
 //      appended to the per-target fallback list (tree_pm_coupling.cpp:4341-4370);
 //   2. walks the tree once for the group box (buildTreePmGroupInteractionList,
-//      tree_pm_group_walk.hpp:78-163). The walk is the stackless preorder walk
-//      of the per-target kernel made wave-cooperative: the 64 lanes decide 64
-//      consecutive preorder nodes at once, and the nodes actually visited are
-//      the chain p -> next(p) -> ... through them (next = q + 1 to open, q + skip
-//      otherwise). Listed leaves and accepted nodes are appended in preorder to
-//      an LDS buffer;
-//   3. whenever the buffer fills (and at the end) every target evaluates the
-//      buffered list (accumulateTreePmGroupCulledLeaves, :290-341, and the
-//      accepted-node expansion): a group of T targets gives each target S lanes
-//      (the largest power of two with S T <= 64). The listed leaves' sources
-//      are staged in LDS 64 at a time, each lane taking every S-th staged
-//      source and every S-th accepted node; the lanes' sums are added at the
-//      end. The per-target leaf cull is evaluated for its counters only: a
-//      culled leaf lies beyond r_cut of the target, so its pairs are zero, and
-//      evaluating every listed source keeps all S lanes of a target busy.
+//      tree_pm_group_walk.hpp:78-163): eight opened nodes are popped from an
+//      LDS stack and the lanes decide their children, so every lane's node is
+//      one the walk visits. (Deciding 64 consecutive preorder nodes and
+//      following the visited chain through them left most of each window
+//      unused and was half of the kernel's time.) Listed leaves and accepted
+//      nodes are appended to LDS lists;
+//   3. whenever a list fills (and at the end) the listed leaves' sources are
+//      taken 64 at a time; those beyond r_cut of the group box (beyond it of
+//      every target, so their pairs are zero) are dropped, the rest compacted
+//      into an LDS window, and every full window of 64 is evaluated by all
+//      targets: a group of T targets gives each target S lanes (the largest
+//      power of two with S T <= 64), each taking every S-th source and every
+//      S-th accepted node (accumulateTreePmGroupCulledLeaves, :290-341); the
+//      lanes' sums are added at the end. The per-target leaf cull is evaluated
+//      only for its counters, when they are read.
+// Four waves share a block for the FP64 pair table's cells up to r_cut: 12 KB
+// of LDS instead of gathers from a 128 KB table in memory. What bounds it is
+// the latency of the walk's dependent loads at 2 to 3 waves per SIMD, then FP64
+// issue in the pairs. Kernel time, 128^3 bodies and a 256^3 mesh in FP64: 23.1
+// ms, with the window and the table in LDS 21, with the stack 12.2; 1500001
+// bodies mixed: 15.0 to 10.8 ms.
 // Groups above 64 targets are evaluated 64 targets at a time, repeating the
 // (identical) tree walk for each.
 //
@@ -1047,7 +1054,13 @@ __global__ __launch_bounds__(kWalkThreads) void walk64_kernel(WalkParams P, Walk
 // interpolation reads the FP32 force meshes at the fixed-point position.
 constexpr int kGroupLeafCap = 192;
 constexpr int kGroupNodeCap = 128;
-constexpr int kGroupStage = 64;  // listed sources staged in LDS per evaluation pass
+constexpr int kGroupStage = 64;  // sources evaluated in a pass
+// Open nodes of the tree walk: eight are expanded at a time, one at a time from
+// kGroupWide on, so that a depth of 21 levels cannot overflow the stack.
+constexpr uint32_t kNoNode = 0xFFFFFFFFu;  // child_index without a child
+constexpr uint32_t kGroupWide = 96;
+constexpr uint32_t kGroupStack = kGroupWide + 56 + 7 * 21 + 13;
+constexpr int kGroupCells = 384;  // FP64 pair table cells held in LDS (12 KB; r_cut = 4.5 a needs 326)
 
 struct GroupLeaf {
   double ox, oy, oz, h;  // cell centre relative to the group centre, cell half size
@@ -1081,29 +1094,69 @@ template <class T> __device__ __forceinline__ T scan_max(T v, int lane) {
   return v;
 }
 
-template <int SCHEME, bool MIX, bool NODE32>
+// inclusive maximum over the lanes up to this one (all 64 active)
+__device__ __forceinline__ uint32_t group_scan_max(uint32_t v) {
+  v = dpp_max_step(v, CHUI_DPP(v, 0x111, 0xf, 0u));  // row_shr:1
+  v = dpp_max_step(v, CHUI_DPP(v, 0x112, 0xf, 0u));  // row_shr:2
+  v = dpp_max_step(v, CHUI_DPP(v, 0x114, 0xf, 0u));  // row_shr:4
+  v = dpp_max_step(v, CHUI_DPP(v, 0x118, 0xf, 0u));  // row_shr:8
+  v = dpp_max_step(v, CHUI_DPP(v, 0x142, 0xa, 0u));  // row_bcast:15
+  v = dpp_max_step(v, CHUI_DPP(v, 0x143, 0xc, 0u));  // row_bcast:31
+  return v;
+}
+// LDS written by some lanes of the wave is read by others after this
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// One wave's lists and window.
+template <bool MIX>
+struct GroupLds {
+  GroupLeaf leaves[kGroupLeafCap];
+  uint32_t nodes[kGroupNodeCap];
+  uint32_t leaf_pre[kGroupLeafCap + 1];
+  uint32_t open[kGroupStack];
+  uint32_t mark[kWave];
+  std::conditional_t<MIX, uint4, double4> stage[2 * kGroupStage];
+  uint32_t stage_j[2 * kGroupStage];
+};
+
+// TAB: the FP64 pair table's cells up to r_cut lie in LDS.
+template <int SCHEME, bool MIX, bool NODE32, bool TAB>
 __device__ __forceinline__ void group_walk_body(const WalkParams& P, const GroupParams& G, const WalkData& D,
                                                 const uint32_t* __restrict__ leaf_of_pos, const WalkOutputs& out,
                                                 uint32_t* __restrict__ fb_pos, uint32_t* __restrict__ fb_slot,
                                                 uint32_t* __restrict__ fb_count,
                                                 unsigned long long* __restrict__ counters) {
-  __shared__ GroupLeaf leaves[kGroupLeafCap];
-  __shared__ uint32_t nodes[kGroupNodeCap];
-  __shared__ uint32_t leaf_pre[kGroupLeafCap + 1];
-  __shared__ double4 stage[MIX ? 1 : kGroupStage];
-  __shared__ uint4 stage32[MIX ? kGroupStage : 1];
+  __shared__ GroupLds<MIX> lds_all[kWalkWaves];
   __shared__ float4 htab[MIX ? kHTableCells : 1];
-  __shared__ uint32_t stage_j[kGroupStage];
-  const int lane = threadIdx.x;
+  __shared__ double4 gtab[TAB ? kGroupCells : 1];
+  const int w = static_cast<int>(readlane_u32(threadIdx.x / kWave, 0));
+  const int lane = threadIdx.x % kWave;
   if constexpr (MIX) {
-    for (int i = lane; i < kHTableCells; i += kWave) htab[i] = D.htab[i];
-    __syncthreads();
+    for (int i = threadIdx.x; i < kHTableCells; i += kWalkThreads) htab[i] = D.htab[i];
   }
-  const uint32_t bb = blockIdx.x * G.block;
+  if constexpr (TAB) {
+    for (int i = threadIdx.x; i < static_cast<int>(G.table_cells); i += kWalkThreads) gtab[i] = D.gcoef[i];
+  }
+  if constexpr (MIX || TAB) __syncthreads();
+  GroupLeaf* const leaves = lds_all[w].leaves;
+  uint32_t* const nodes = lds_all[w].nodes;
+  uint32_t* const leaf_pre = lds_all[w].leaf_pre;
+  uint32_t* const mark = lds_all[w].mark;
+  uint32_t* const open = lds_all[w].open;
+  auto* const stage = lds_all[w].stage;
+  uint32_t* const stage_j = lds_all[w].stage_j;
+  const uint64_t bb64 = (static_cast<uint64_t>(xcd_logical_block()) * kWalkWaves + w) * G.block;
+  if (bb64 >= P.n_targets) return;
+  const uint32_t bb = static_cast<uint32_t>(bb64);
   const uint32_t be = min(bb + G.block, P.n_targets);
   const double L0 = P.L[0], L1 = P.L[1], L2 = P.L[2];
   const double cull2 = P.rcut2 * (1.0 + 1.0e-9);
-  const double tlim = 0x1.fffffffffffffp+5;  // largest double below 64
+  // table coordinates end below 64, or within the cells held in LDS (every
+  // pair inside r_cut lies below)
+  const double tlim = TAB ? (G.table_cells - 0.5) / 64.0 : 0x1.fffffffffffffp+5;
   const double iL0 = 1.0 / P.L[0], iL1 = 1.0 / P.L[1], iL2 = 1.0 / P.L[2];
   const double eps2 = P.eps * P.eps;
   uint32_t cnt[kGroupCounters] = {};
@@ -1214,6 +1267,27 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
       cnt[5] += 1;
       cnt[6] += count;
     }
+    // all sources in [0, L] and r_cut around the group inside the box on every
+    // axis: its pairs need no image (a source within r_cut of the group box has
+    // none nearer)
+    const double rcm = P.rcut * (1.0 + 1.0e-9);
+    const auto clear = [&](double c, double hg, double L, int a) {
+      return G.lo[a] >= 0.0 && G.hi[a] <= L && c - hg - rcm > 0.0 && c + hg + rcm < L && 2.0 * hg + rcm < 0.4999 * L;
+    };
+    const bool inner = clear(c0x, hg0, L0, 0) && clear(c0y, hg1, L1, 1) && clear(c0z, hg2, L2, 2);
+    // MIX: the group box in fixed point and table units, widened by the
+    // roundings of its centre and of the offsets
+    uint32_t gcx = 0, gcy = 0, gcz = 0;
+    float gt0 = 0.0f, gt1 = 0.0f, gt2 = 0.0f;
+    if constexpr (MIX) {
+      const double f0 = 4294967296.0 / L0, f1 = 4294967296.0 / L1, f2 = 4294967296.0 / L2;
+      gcx = readlane_u32(static_cast<uint32_t>(static_cast<int64_t>(floor(c0x * f0))), 0);
+      gcy = readlane_u32(static_cast<uint32_t>(static_cast<int64_t>(floor(c0y * f1))), 0);
+      gcz = readlane_u32(static_cast<uint32_t>(static_cast<int64_t>(floor(c0z * f2))), 0);
+      gt0 = static_cast<float>(hg0 * f0 + 4.0) * P.tab_scale[0] * 1.000001f;
+      gt1 = static_cast<float>(hg1 * f1 + 4.0) * P.tab_scale[1] * 1.000001f;
+      gt2 = static_cast<float>(hg2 * f2 + 4.0) * P.tab_scale[2] * 1.000001f;
+    }
     size_max = count > size_max ? count : size_max;
 
     // ---- targets, 64 at a time
@@ -1246,108 +1320,62 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
         oz = nearest_image(pz - c0z, L2);
       }
       double ax = 0.0, ay = 0.0, az = 0.0, nearest = INFINITY;
-      uint32_t listed = 0, nl = 0, nm = 0, p = 0;
+      uint32_t listed = 0, nl = 0, nm = 0;
 
-      auto evaluate = [&]() {
-        __syncthreads();
-        // candidate and culled leaves per target (the counters of
-        // accumulateTreePmGroupCulledLeaves): a culled leaf lies beyond r_cut
-        // of the target, so its sources add nothing to the pair sums below
-        for (uint32_t e = s; e < nl; e += S) {
-          if (!valid) continue;
-          const GroupLeaf Lf = leaves[e];
-          const double gx = fmax(0.0, fabs(wrap_half(Lf.ox - ox, L0)) - Lf.h);
-          const double gy = fmax(0.0, fabs(wrap_half(Lf.oy - oy, L1)) - Lf.h);
-          const double gz = fmax(0.0, fabs(wrap_half(Lf.oz - oz, L2)) - Lf.h);
-          const bool cull = gx * gx + gy * gy + gz * gz > cull2;
-          ++cnt[11];
-          if (cull) ++cnt[12];
-          else cnt[13] += Lf.e - Lf.b;
-        }
-        // exclusive prefix of the listed leaves' source counts
-        uint32_t total = 0;
-        for (uint32_t c = 0; c < nl; c += kWave) {
-          const uint32_t e = c + lane;
-          const uint32_t own = e < nl ? leaves[e].e - leaves[e].b : 0u;
-          uint32_t incl = own;
-          for (int off = 1; off < kWave; off <<= 1) {
-            const uint32_t o = __shfl_up(incl, off, kWave);
-            if (lane >= off) incl += o;
+      uint32_t wn = 0;  // sources in the window, below kGroupStage between batches
+      // the first gn staged sources: each of a target's S lanes takes every
+      // S-th one
+      auto pairs = [&]<bool WRAP>(uint32_t gn) {
+        if (!valid) return;
+        if constexpr (MIX) {
+          // FP32 pairs in H-table units (the mixed strict walk's pair term)
+          const float u0 = P.tab_scale[0], u1 = P.tab_scale[1], u2 = P.tab_scale[2];
+          const float rc2 = P.rcut2_tab, e2 = P.eps2_tab, c8 = P.c8_tab;
+          float lx = 0.0f, ly = 0.0f, lz = 0.0f, near_t = INFINITY;
+          uint32_t inside_n = 0;
+          for (uint32_t q = s; q < gn; q += S) {
+            const uint4 sv = stage[q];
+            const uint32_t j = stage_j[q];
+            const float dx = fx_delta(sv.x, tx, u0), dy = fx_delta(sv.y, ty, u1), dz = fx_delta(sv.z, tz, u2);
+            const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+            const float rinv = __builtin_amdgcn_rsqf(r2 + e2);
+            const float soft = rinv * rinv * rinv;
+            const int ci = static_cast<int>(fminf(r2, static_cast<float>(kHTableCells - 1)));
+            const float fu = __builtin_amdgcn_fractf(r2);
+            const float4 c = htab[ci];
+            const float hcoef = fmaf(fmaf(fmaf(c.w, fu, c.z), fu, c.y), fu, c.x);
+            float fr = fmaf(-hcoef, c8, soft);
+            if (!D.uniform_mass) fr *= __uint_as_float(sv.w);
+            const bool inside = j != tp && r2 <= rc2;
+            const float f = inside ? fr : 0.0f;
+            lx = fmaf(f, dx, lx);
+            ly = fmaf(f, dy, ly);
+            lz = fmaf(f, dz, lz);
+            inside_n += inside ? 1u : 0u;
+            near_t = inside ? fminf(near_t, r2) : near_t;
           }
-          if (e < nl) leaf_pre[e] = total + incl - own;
-          total += readlane_u32(incl, kWave - 1);
-        }
-        if (lane == 0) leaf_pre[nl] = total;
-        // the listed sources, kGroupStage at a time: staged once in LDS and
-        // evaluated by each target's S lanes (lane s takes every S-th source)
-        for (uint32_t g0 = 0; g0 < total; g0 += kGroupStage) {
-          const uint32_t gn = min(total - g0, static_cast<uint32_t>(kGroupStage));
-          __syncthreads();
-          if (static_cast<uint32_t>(lane) < gn) {
-            const uint32_t g = g0 + lane;
-            uint32_t lo = 0, hi = nl;  // the leaf e with leaf_pre[e] <= g < leaf_pre[e + 1]
-            while (hi - lo > 1) {
-              const uint32_t mid = (lo + hi) >> 1;
-              if (leaf_pre[mid] <= g) lo = mid;
-              else hi = mid;
-            }
-            const uint32_t j = leaves[lo].b + (g - leaf_pre[lo]);
-            if constexpr (MIX) stage32[lane] = D.src32[j];
-            else stage[lane] = D.src64[j];
-            stage_j[lane] = j;
-          }
-          __syncthreads();
-          if (!valid) continue;
-          if constexpr (MIX) {
-            // FP32 pairs in H-table units (the mixed strict walk's pair term)
-            const float u0 = P.tab_scale[0], u1 = P.tab_scale[1], u2 = P.tab_scale[2];
-            const float rc2 = P.rcut2_tab, e2 = P.eps2_tab, c8 = P.c8_tab;
-            float lx = 0.0f, ly = 0.0f, lz = 0.0f, near_t = INFINITY;
-            uint32_t inside_n = 0;
-            for (uint32_t q = s; q < gn; q += S) {
-              const uint4 sv = stage32[q];
-              const uint32_t j = stage_j[q];
-              const float dx = fx_delta(sv.x, tx, u0), dy = fx_delta(sv.y, ty, u1), dz = fx_delta(sv.z, tz, u2);
-              const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-              const float rinv = __builtin_amdgcn_rsqf(r2 + e2);
-              const float soft = rinv * rinv * rinv;
-              const int ci = static_cast<int>(fminf(r2, static_cast<float>(kHTableCells - 1)));
-              const float fu = __builtin_amdgcn_fractf(r2);
-              const float4 c = htab[ci];
-              const float hcoef = fmaf(fmaf(fmaf(c.w, fu, c.z), fu, c.y), fu, c.x);
-              float fr = fmaf(-hcoef, c8, soft);
-              if (!D.uniform_mass) fr *= __uint_as_float(sv.w);
-              const bool inside = j != tp && r2 <= rc2;
-              const float f = inside ? fr : 0.0f;
-              lx = fmaf(f, dx, lx);
-              ly = fmaf(f, dy, ly);
-              lz = fmaf(f, dz, lz);
-              inside_n += inside ? 1u : 0u;
-              near_t = inside ? fminf(near_t, r2) : near_t;
-            }
-            const double gm = P.force_scale;
-            ax = fma(gm, static_cast<double>(lx), ax);
-            ay = fma(gm, static_cast<double>(ly), ay);
-            az = fma(gm, static_cast<double>(lz), az);
-            cnt[2] += inside_n;
-            nearest = fmin(nearest, static_cast<double>(near_t) * static_cast<double>(P.tab_to_len2));
-            continue;
-          }
+          const double gm = P.force_scale;
+          ax = fma(gm, static_cast<double>(lx), ax);
+          ay = fma(gm, static_cast<double>(ly), ay);
+          az = fma(gm, static_cast<double>(lz), az);
+          cnt[2] += inside_n;
+          nearest = fmin(nearest, static_cast<double>(near_t) * static_cast<double>(P.tab_to_len2));
+        } else {
           for (uint32_t q = s; q < gn; q += S) {
             const double4 sj = stage[q];
             const uint32_t j = stage_j[q];
             // minimum image by rounding: the same separations as wrap_half
             // wherever |d| <= L/2 or d - L is exact (every pair inside r_cut)
             const double ex = sj.x - px, ey = sj.y - py, ez = sj.z - pz;
-            const double dx = fma(-L0, rint(ex * iL0), ex), dy = fma(-L1, rint(ey * iL1), ey),
-                         dz = fma(-L2, rint(ez * iL2), ez);
+            const double dx = WRAP ? fma(-L0, rint(ex * iL0), ex) : ex, dy = WRAP ? fma(-L1, rint(ey * iL1), ey) : ey,
+                         dz = WRAP ? fma(-L2, rint(ez * iL2), ez) : ez;
             const double r2 = dx * dx + dy * dy + dz * dz;
             const bool inside = j != tp && r2 <= P.rcut2;
             // the Hermite cell as a cubic in u (Horner with fused steps)
             const double cell = fmin(r2 * P.inv2a2, tlim) * 64.0;
             const int ci = static_cast<int>(cell);
             const double u = cell - static_cast<double>(ci);
-            const double4 hc = D.gcoef[ci];
+            const double4 hc = TAB ? gtab[ci] : D.gcoef[ci];
             const double lr = fma(fma(fma(hc.w, u, hc.z), u, hc.y), u, hc.x) * P.inv8a3;
             // (r^2 + eps^2)^(-3/2): hardware reciprocal square root and two
             // Newton steps y <- y + y (1 - dd y^2) / 2 (r2 = 0 is masked below)
@@ -1364,6 +1392,94 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
             cnt[2] += inside ? 1u : 0u;
             nearest = inside ? fmin(nearest, r2) : nearest;
           }
+        }
+      };
+      auto evaluate = [&](bool last) {
+        wave_sync();
+        // candidate and culled leaves per target (the counters of
+        // accumulateTreePmGroupCulledLeaves): a culled leaf lies beyond r_cut
+        // of the target, so its sources add nothing to the pair sums below
+        if (G.count) {
+          for (uint32_t e = s; e < nl; e += S) {
+            if (!valid) continue;
+            const GroupLeaf Lf = leaves[e];
+            const double gx = fmax(0.0, fabs(wrap_half(Lf.ox - ox, L0)) - Lf.h);
+            const double gy = fmax(0.0, fabs(wrap_half(Lf.oy - oy, L1)) - Lf.h);
+            const double gz = fmax(0.0, fabs(wrap_half(Lf.oz - oz, L2)) - Lf.h);
+            const bool cull = gx * gx + gy * gy + gz * gz > cull2;
+            ++cnt[11];
+            if (cull) ++cnt[12];
+            else cnt[13] += Lf.e - Lf.b;
+          }
+        }
+        // exclusive prefix of the listed leaves' source counts
+        uint32_t total = 0;
+        for (uint32_t c = 0; c < nl; c += kWave) {
+          const uint32_t e = c + lane;
+          const uint32_t own = e < nl ? leaves[e].e - leaves[e].b : 0u;
+          uint32_t incl = own;
+          for (int off = 1; off < kWave; off <<= 1) {
+            const uint32_t o = __shfl_up(incl, off, kWave);
+            if (lane >= off) incl += o;
+          }
+          if (e < nl) leaf_pre[e] = total + incl - own;
+          total += readlane_u32(incl, kWave - 1);
+        }
+        wave_sync();
+        // the listed sources, 64 at a time: leaves (none is empty) mark the
+        // lane where they start and a running maximum gives every lane its
+        // leaf; sources beyond r_cut of the group box are dropped
+        uint32_t e0 = 0;  // the leaf of the last batch's last source
+        for (uint32_t g0 = 0;; g0 += kWave) {
+          mark[lane] = 0;
+          wave_sync();
+          const uint32_t e = e0 + 1u + lane;
+          const uint32_t st = e < nl ? leaf_pre[e] - g0 : static_cast<uint32_t>(kWave);
+          if (st < static_cast<uint32_t>(kWave)) mark[st] = lane + 1u;
+          wave_sync();
+          const uint32_t lf = e0 + group_scan_max(mark[lane]);
+          const uint32_t g = g0 + lane;
+          const bool on = g < total;
+          const uint32_t j = on ? leaves[lf].b + (g - leaf_pre[lf]) : 0u;
+          e0 = readlane_u32(lf, kWave - 1);
+          bool keep;
+          std::conditional_t<MIX, uint4, double4> rec;
+          if constexpr (MIX) {
+            rec = D.src32[j];
+            const float ex = fmaxf(fabsf(fx_delta(rec.x, gcx, P.tab_scale[0])) - gt0, 0.0f);
+            const float ey = fmaxf(fabsf(fx_delta(rec.y, gcy, P.tab_scale[1])) - gt1, 0.0f);
+            const float ez = fmaxf(fabsf(fx_delta(rec.z, gcz, P.tab_scale[2])) - gt2, 0.0f);
+            keep = on && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > P.rcut2_tab * 1.00001f);
+          } else {
+            rec = D.src64[j];
+            const double ex = fmax(0.0, fabs(nearest_image_inv(rec.x - c0x, L0, iL0)) - hg0);
+            const double ey = fmax(0.0, fabs(nearest_image_inv(rec.y - c0y, L1, iL1)) - hg1);
+            const double ez = fmax(0.0, fabs(nearest_image_inv(rec.z - c0z, L2, iL2)) - hg2);
+            keep = on && !(ex * ex + ey * ey + ez * ez > cull2);
+          }
+          const unsigned long long km = __ballot(keep);
+          if (keep) {
+            const uint32_t at = wn + static_cast<uint32_t>(__popcll(km & ((1ull << lane) - 1ull)));
+            stage[at] = rec;
+            stage_j[at] = j;
+          }
+          wn += static_cast<uint32_t>(__popcll(km));
+          const bool end = g0 + kWave >= total;
+          while (wn >= static_cast<uint32_t>(kGroupStage) || (last && end && wn)) {
+            const uint32_t gn = wn < static_cast<uint32_t>(kGroupStage) ? wn : static_cast<uint32_t>(kGroupStage);
+            wave_sync();
+            if (MIX || !inner) pairs.template operator()<true>(gn);
+            else pairs.template operator()<false>(gn);
+            wave_sync();
+            wn -= gn;
+            // the records past the window move to its front
+            if (static_cast<uint32_t>(lane) < wn) {
+              stage[lane] = stage[kGroupStage + lane];
+              stage_j[lane] = stage_j[kGroupStage + lane];
+            }
+          }
+          wave_sync();
+          if (end) break;
         }
         for (uint32_t e = s; e < nm; e += S) {
           if (!valid) continue;
@@ -1393,23 +1509,38 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
             else node_accel64(M, D.quad64[nd], dx, dy, dz, P, ax, ay, az);
           }
         }
-        __syncthreads();
+        wave_sync();
         nl = 0;
         nm = 0;
       };
 
+      uint32_t sp = 0;
+      bool root = true;
       while (true) {
-        const bool done = p >= P.node_count;
+        const bool done = !root && sp == 0;
         if (done || nl > static_cast<uint32_t>(kGroupLeafCap - kWave) ||
             nm > static_cast<uint32_t>(kGroupNodeCap - kWave))
-          evaluate();
+          evaluate(done);
         if (done) break;
-        // decide preorder nodes p .. p + 63 for the group box
-        const uint32_t q = p + lane;
-        uint32_t next = q + 1, lb = 0, le = 0;
+        // decide the children of up to eight open nodes (or the root) for the
+        // group box, one to a lane
+        uint32_t q = kNoNode;
+        wave_sync();
+        if (root) {
+          if (lane == 0) q = 0;
+          root = false;
+        } else {
+          const uint32_t m = sp > kGroupWide ? 1u : min(sp, 8u);
+          sp -= m;
+          const uint32_t k = static_cast<uint32_t>(lane) >> 3;
+          if (k < m) q = D.child_index[8ull * open[sp + k] + (lane & 7)];
+        }
+        wave_sync();
+        const bool on = q != kNoNode;
+        uint32_t lb = 0, le = 0;
         int kind = 3;  // 0 pruned, 1 listed leaf, 2 accepted node, 3 opened
         double dc0 = 0.0, dc1 = 0.0, dc2 = 0.0, h = 0.0;
-        if (q < P.node_count) {
+        if (on) {
           const NodeLink lk = D.link[q];
           const NodeGeo64 g = D.geo64[q];
           h = g.half;
@@ -1440,18 +1571,8 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
             }
             kind = acc ? 2 : 3;
           }
-          next = kind == 3 ? q + 1 : q + lk.skip;
         }
-        // the visited chain through the window
-        unsigned long long chain = 0;
-        uint32_t cur = p;
-        while (cur < p + kWave && cur < P.node_count) {
-          const uint32_t l = cur - p;
-          chain |= 1ull << l;
-          cur = readlane_u32(next, l);
-        }
-        p = cur;
-        const bool on = (chain >> lane) & 1ull;
+        const unsigned long long vm = __ballot(on);
         const unsigned long long lm = __ballot(on && kind == 1);
         const unsigned long long mm = __ballot(on && kind == 2);
         const unsigned long long below = (1ull << lane) - 1ull;
@@ -1465,12 +1586,14 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
           Lf.e = le;
         }
         if (on && kind == 2) nodes[nm + __popcll(mm & below)] = q;
-        const unsigned long long pm = __ballot(on && kind == 0);
+        const unsigned long long pm = __ballot(on && kind == 0), om = __ballot(on && kind == 3);
+        if (on && kind == 3) open[sp + __popcll(om & below)] = q;
+        sp += __popcll(om);
         nl += __popcll(lm);
         nm += __popcll(mm);
         listed += __popcll(lm) + __popcll(mm);
         if (first && lane == 0) {
-          cnt[0] += __popcll(chain);
+          cnt[0] += __popcll(vm);
           cnt[1] += __popcll(pm);
           cnt[3] += __popcll(mm);
           cnt[4] += __popcll(lm);
@@ -1542,22 +1665,22 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
 // bytes per lane and ran 2% (FP64) to 29% (mixed) slower at 256^3. The mixed
 // walk with FP32 node expansions (RADIAL false) holds 142 VGPRs and runs 3
 // waves per SIMD (4 waves: 128 VGPRs with spills, 16% slower).
-template <int SCHEME>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(2))) void group_walk64_kernel(
+template <int SCHEME, bool TAB>
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(2))) void group_walk64_kernel(
     WalkParams P, GroupParams G, WalkData D, const uint32_t* __restrict__ leaf_of_pos, WalkOutputs out,
     uint32_t* __restrict__ fb_pos, uint32_t* __restrict__ fb_slot, uint32_t* __restrict__ fb_count,
     unsigned long long* __restrict__ counters) {
-  group_walk_body<SCHEME, false, false>(P, G, D, leaf_of_pos, out, fb_pos, fb_slot, fb_count, counters);
+  group_walk_body<SCHEME, false, false, TAB>(P, G, D, leaf_of_pos, out, fb_pos, fb_slot, fb_count, counters);
 }
 
 // RADIAL: the radial-coefficient node expansion (FP64; the FP32 expansion is
 // the plain monopole + quadrupole one).
 template <int SCHEME, bool RADIAL>
-__global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(RADIAL ? 2 : 3))) void group_walkmix_kernel(
+__global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(RADIAL ? 2 : 3))) void group_walkmix_kernel(
     WalkParams P, GroupParams G, WalkData D, const uint32_t* __restrict__ leaf_of_pos, WalkOutputs out,
     uint32_t* __restrict__ fb_pos, uint32_t* __restrict__ fb_slot, uint32_t* __restrict__ fb_count,
     unsigned long long* __restrict__ counters) {
-  group_walk_body<SCHEME, true, !RADIAL>(P, G, D, leaf_of_pos, out, fb_pos, fb_slot, fb_count, counters);
+  group_walk_body<SCHEME, true, !RADIAL, false>(P, G, D, leaf_of_pos, out, fb_pos, fb_slot, fb_count, counters);
 }
 
 // Mixed adaptive solves: targets the group walk hands back (or every target
@@ -3769,6 +3892,7 @@ void walk_fp64_group(const Tree& t, const WalkParams& p, const GroupParams& g, c
   d.geo64 = t.geo64.as<NodeGeo64>();
   d.mom64 = t.mom64.as<NodeMom64>();
   d.quad64 = t.quad64.as<NodeQuad64>();
+  d.child_index = t.child_index.as<uint32_t>();
   d.order = t.order.as<uint32_t>();
   d.src64 = src;
   d.uniform_mass = uniform_mass;
@@ -3780,13 +3904,22 @@ void walk_fp64_group(const Tree& t, const WalkParams& p, const GroupParams& g, c
   d.gtab = gtab;
   d.gcoef = gcoef;
   d.prev = prev;
-  const unsigned blocks = static_cast<unsigned>((static_cast<std::size_t>(p.n_targets) + g.block - 1) / g.block);
-  if (p.assignment == 0)
-    group_walk64_kernel<0><<<blocks, kWave, 0, s>>>(p, g, d, leaf_of_pos, out, fallback_pos, fallback_slot,
-                                                    fallback_count, counters);
-  else
-    group_walk64_kernel<1><<<blocks, kWave, 0, s>>>(p, g, d, leaf_of_pos, out, fallback_pos, fallback_slot,
-                                                    fallback_count, counters);
+  // the table's cells up to r_cut in LDS when they fit (one more for rounding)
+  GroupParams gp = g;
+  const double cells = std::floor(p.rcut2 * p.inv2a2 * 64.0 * (1.0 + 1.0e-12)) + 2.0;
+  gp.table_cells = cells <= kGroupCells ? static_cast<uint32_t>(cells) : 0u;
+  const unsigned blocks = grid_for((static_cast<std::size_t>(p.n_targets) + g.block - 1) / g.block, kWalkWaves);
+  const auto go = [&](auto kernel) {
+    kernel<<<blocks, kWalkThreads, 0, s>>>(p, gp, d, leaf_of_pos, out, fallback_pos, fallback_slot, fallback_count,
+                                           counters);
+  };
+  if (p.assignment == 0) {
+    if (gp.table_cells) go(group_walk64_kernel<0, true>);
+    else go(group_walk64_kernel<0, false>);
+  } else {
+    if (gp.table_cells) go(group_walk64_kernel<1, true>);
+    else go(group_walk64_kernel<1, false>);
+  }
   CHUI_LAUNCH_CHECK("group_walk64_kernel");
 }
 
@@ -3805,6 +3938,7 @@ void walk_mixed_group(const Tree& t, const WalkParams& p, const GroupParams& g, 
   d.geo64 = t.geo64.as<NodeGeo64>();
   d.mom64 = t.mom64.as<NodeMom64>();
   d.quad64 = t.quad64.as<NodeQuad64>();
+  d.child_index = t.child_index.as<uint32_t>();
   d.order = t.order.as<uint32_t>();
   d.src64 = src64;
   d.src32 = src32;
@@ -3818,10 +3952,11 @@ void walk_mixed_group(const Tree& t, const WalkParams& p, const GroupParams& g, 
   d.f32y = fy;
   d.f32z = fz;
   d.prev = prev;
-  const unsigned blocks = static_cast<unsigned>((static_cast<std::size_t>(p.n_targets) + g.block - 1) / g.block);
+  const unsigned blocks = grid_for((static_cast<std::size_t>(p.n_targets) + g.block - 1) / g.block, kWalkWaves);
   if (!t.mom32.ptr || !t.quad32.ptr) throw std::logic_error("mixed group walk on a tree without FP32 node records");
   auto go = [&](auto kernel) {
-    kernel<<<blocks, kWave, 0, s>>>(p, g, d, leaf_of_pos, out, fallback_pos, fallback_slot, fallback_count, counters);
+    kernel<<<blocks, kWalkThreads, 0, s>>>(p, g, d, leaf_of_pos, out, fallback_pos, fallback_slot, fallback_count,
+                                           counters);
   };
   if (p.assignment == 0) {
     if (p.radial) go(group_walkmix_kernel<0, true>);

@@ -98,6 +98,8 @@ struct GroupParams {
   double amax2;
   int contain;           // kContainNode
   double lo[3], hi[3];
+  int count;             // someone reads the candidate and culled leaf counters
+  uint32_t table_cells;  // FP64 pair table cells up to r_cut (0: too many for LDS)
 };
 
 // Group walk counters on the device (chui_treepm_walk_counters order after
