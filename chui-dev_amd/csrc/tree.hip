@@ -974,8 +974,9 @@ __global__ __launch_bounds__(256) void node_links_kernel(NodeArgs a, const uint6
 // Multipoles, bottom up (tree_gravity.cpp:1208-1380, same operation order). A
 // particle or child has a lane: its terms go to LDS, and one lane per sum adds
 // them in tree order, so a wave's loads are independent and contiguous. One
-// thread per node left a wave to chains of dependent loads (all nodes: 128^3
-// 270 us, 256^3 983 us).
+// thread per node left a wave to chains of dependent loads. Leaf order, subtrees
+// and top, thread per node and now: 128^3 71 + 270 + 84 and 118 + 76 + 39 us,
+// 256^3 594 + 983 + 77 and 995 + 417 + 38 us.
 struct MomArgs {
   UnwrapArgs u;
   int quad;
@@ -1220,14 +1221,6 @@ __device__ __forceinline__ void node_moments(const MomArgs& a, const MomArrays& 
   }
 }
 
-// In-leaf Morton order (tree_ordering.cpp:151): the (Morton key, row) ranks of
-// a leaf's particles by comparison, G lanes per node; leaves of more than G
-// particles are ranked by the whole wave. Reads the sort's order and the
-// input-order records, writes the final order and the tree-order copy of the
-// sources (canonical coordinates and mass), so the gather, the Morton keys and
-// the permutation are one pass (256^3: 0.85 ms in three). The records move to
-// their rank's lane first: the stores are contiguous, and the leaf's moments
-// are summed in tree order while its particles are in registers.
 // v moved to the lane at byte address `to` / 4; all lanes active, `to` a permutation
 __device__ __forceinline__ double permute_f64(int to, double v) {
   const uint64_t b = static_cast<uint64_t>(__double_as_longlong(v));
@@ -1236,6 +1229,14 @@ __device__ __forceinline__ double permute_f64(int to, double v) {
   return __longlong_as_double(static_cast<long long>((static_cast<uint64_t>(hi) << 32) | lo));
 }
 
+// In-leaf Morton order (tree_ordering.cpp:151): the (Morton key, row) ranks of
+// a leaf's particles by comparison, G lanes per node; leaves of more than G
+// particles are ranked by the whole wave. Reads the sort's order and the
+// input-order records, writes the final order and the tree-order copy of the
+// sources (canonical coordinates and mass), so the gather, the Morton keys and
+// the permutation are one pass (256^3: 0.85 ms in three). The records move to
+// their rank's lane first: the stores are contiguous, and the leaf's moments
+// are summed in tree order while its particles are in registers.
 template <int G>
 __global__ __launch_bounds__(256) void leaf_order_kernel(uint32_t total_nodes, const uint32_t* __restrict__ total_dev,
                                                          MomArgs mo, MomArrays o,
@@ -1322,7 +1323,10 @@ __global__ __launch_bounds__(256) void leaf_order_kernel(uint32_t total_nodes, c
   }
 }
 
-// Moments of one subtree per block, all its levels in one launch: a subtree's
+// Moments of one subtree per block, all its levels in one launch (bound by the
+// loads of each level waiting for the level below; a launch per level took 13
+// to 15 launches of 4 to 60 us, hence subtrees of max(512, n / 1024) particles:
+// a thousand or more blocks, and at most a few thousand nodes above them). A subtree's
 // nodes of each depth are consecutive, from the first child of the first split
 // node of the depth above to the last child of the last.
 __global__ __launch_bounds__(256) void moment_subtree_kernel(MomArgs a, MomArrays o, const uint32_t* __restrict__ lv,

@@ -2337,10 +2337,12 @@ __device__ __forceinline__ uint32_t box_segment(uint32_t seg, uint32_t per_wave,
 // 64^3 box, which moves a 32^3 box's force field by 2e-6 in relative L2 (1e-7
 // otherwise). So up to 2^20 sources both walks decide each pair alike; beyond,
 // where single pairs do not show, the origin is the segment's centre, which the
-// box test can share (256^3: 4 % of the solve). FP64 decisions took 27 VALU
-// instructions per pair against 16.
+// box test can share (256^3: 4 % of the solve). SHARED holds both forms of a
+// pair: 4 waves per SIMD without spills instead of 5 with 27 registers spilled
+// (eleven boxes of 32^3 to 96^3: 6.01 to 5.34 ms; one of 100003: 1083 to 1020
+// us). FP64 decisions took 27 VALU instructions per pair against 16.
 template <int SCHEME, bool CUBIC, bool LOG, int WAVES, bool FRAME, bool SHARED>
-__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(5)))
+__global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(SHARED ? 4 : 5)))
 void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long long* __restrict__ counters,
                         const NodeLink* __restrict__ node_link, const NodeGeo32* __restrict__ node_geo,
                         const NodeMom32* __restrict__ node_mom, const NodeQuad32* __restrict__ node_quad,
@@ -2611,6 +2613,18 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
       // every target; the 1e-5 margin covers the rounding of the offsets, so
       // every dropped source is one whose pairs are all zero
       const float cull2 = rc2 * 1.00001f;
+      // SHARED: the box centre in the origin's frame; the offsets there reach
+      // L/16 + r_cut, so their roundings may take 3e-7 of that off the gap
+      float obx = 0.0f, oby = 0.0f, obz = 0.0f;
+      if (SHARED && wave_origin) {
+        obx = fx_delta(ox, wox, u0);
+        oby = fx_delta(oy, woy, u1);
+        obz = fx_delta(oz, woz, u2);
+        const float far_r = sqrtf(rc2);
+        bt0 += 6.0e-7f * (268435456.0f * u0 + far_r);
+        bt1 += 6.0e-7f * (268435456.0f * u1 + far_r);
+        bt2 += 6.0e-7f * (268435456.0f * u2 + far_r);
+      }
       uint32_t wn = 0;  // records in the window, below kWindow between batches
       const float4* const mine = win + slice * (TL + 1u);
       // iters records of every slice (a multiple of 4)
@@ -2684,9 +2698,9 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
             const float mj = D.uniform_mass ? 1.0f : __uint_as_float(sv.w);
             const float4 rec = !SHARED || wave_origin ? stage_record.template operator()<true>(sv, mj)
                                            : stage_record.template operator()<false>(sv, mj);
-            const float ex = fmaxf(fabsf(SHARED ? fx_delta(sv.x, ox, u0) : rec.x) - bt0, 0.0f);
-            const float ey = fmaxf(fabsf(SHARED ? fx_delta(sv.y, oy, u1) : rec.y) - bt1, 0.0f);
-            const float ez = fmaxf(fabsf(SHARED ? fx_delta(sv.z, oz, u2) : rec.z) - bt2, 0.0f);
+            const float ex = fmaxf(fabsf(!SHARED ? rec.x : wave_origin ? rec.x - obx : fx_delta(sv.x, ox, u0)) - bt0, 0.0f);
+            const float ey = fmaxf(fabsf(!SHARED ? rec.y : wave_origin ? rec.y - oby : fx_delta(sv.y, oy, u1)) - bt1, 0.0f);
+            const float ez = fmaxf(fabsf(!SHARED ? rec.z : wave_origin ? rec.z - obz : fx_delta(sv.z, oz, u2)) - bt2, 0.0f);
             const bool keep = on && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > cull2);
             const unsigned long long km = __ballot(keep);
             __builtin_amdgcn_wave_barrier();
