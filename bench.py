@@ -272,7 +272,7 @@ def main():
         "ensemble": ensemble,
         "hierarchical_kdk": hierarchical,
         "stages_ms_mixed": {k: v / max(prof_mixed["solves"], 1) for k, v in prof_mixed.items() if k.endswith("_ms")},
-        "roofline": {"bound": "hbm", "kernel": "walkmix_kernel", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
+        "roofline": {"bound": "hbm", "kernel": "walkmix_box_kernel", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK, "traffic": measured_traffic(w.name),
                      "algorithmic_bytes_per_launch": walk_bytes, "launch_ms": walk_ms,
                      "valu": {"pairs": pairs, "flop_per_pair": FLOP_PER_PAIR,
