@@ -601,6 +601,7 @@ void solve_device_impl(Ctx* c, const double* x, const double* y, const double* z
   const bool safe_mode = c->capture_safe;
   const bool safe = safe_mode && n > 0 && c->tree.prepared_n == n && c->tree.sized_for_capture;
   const bool rec = recording(c);
+  const chui::RecordingScope recording_scope(rec);
   if (rec && !safe)
     throw std::runtime_error(
         "graph capture of a solve on a context not prepared for these sources: run one capture-safe solve of "
@@ -1630,6 +1631,7 @@ void force_vjp_impl(Ctx* c, const double* x, const double* y, const double* z, c
   const bool safe_mode = c->capture_safe;
   const bool safe = safe_mode && c->tree.prepared_n == n && c->tree.sized_for_capture;
   const bool rec = recording(c);
+  const chui::RecordingScope recording_scope(rec);
   if (rec && (!safe || (quad && c->vjp_safe_cap == 0)))
     throw std::runtime_error(
         "graph capture of a force VJP on a context not prepared for these sources: run one capture-safe VJP of "
@@ -1882,6 +1884,7 @@ chui_status chui_treepm_solve(chui_treepm_context* c, const double* x, const dou
     require_ctx(c);
     set_device(c);
     validate_options(o, c->mesh);
+    const chui::RecordingScope recording_scope(recording(c));
     const uint64_t na = active ? n_active : n;
     hipStream_t s = c->stream;
     const std::size_t nb = std::max<uint64_t>(n, 1) * sizeof(double);

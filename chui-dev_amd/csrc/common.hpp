@@ -32,6 +32,25 @@ inline unsigned grid_for(std::size_t n, unsigned block) {
   return static_cast<unsigned>(g == 0 ? 1 : g);
 }
 
+// Set while the calling thread issues work on a stream that records a HIP graph.
+// Growing a buffer there would free memory that recorded kernels use, and an
+// allocation, a free or a read-back spoils the recording, so they are refused
+// before any runtime call.
+inline thread_local bool t_recording = false;
+struct RecordingScope {
+  const bool outer = t_recording;
+  explicit RecordingScope(bool recording) { t_recording = outer || recording; }
+  RecordingScope(const RecordingScope&) = delete;
+  RecordingScope& operator=(const RecordingScope&) = delete;
+  ~RecordingScope() { t_recording = outer; }
+};
+inline void require_not_recording(const char* what) {
+  if (t_recording)
+    throw std::logic_error(std::string(what) +
+                           " while a graph is recorded: run the same calls (sources, targets and options) once on "
+                           "this context before capturing");
+}
+
 // Grow-only device buffer. Allocation happens only when a call needs more
 // capacity than any earlier call; steady-state solves allocate nothing.
 struct DeviceBuffer {
@@ -48,6 +67,7 @@ struct DeviceBuffer {
   }
   void reserve(std::size_t need) {
     if (need <= bytes) return;
+    require_not_recording("a device buffer would grow");
     release();
     CHUI_HIP(hipMalloc(&ptr, need));
     bytes = need;
@@ -82,6 +102,7 @@ struct PinnedReadback {
   // copies bytes (<= kBytes) from dev to host after the stream's prior work
   void read(void* host, const void* dev, std::size_t bytes, hipStream_t s) {
     if (bytes > kBytes) throw std::logic_error("pinned readback larger than its block");
+    require_not_recording("a count would be read back");
     if (!ptr) CHUI_HIP(hipHostMalloc(&ptr, kBytes, hipHostMallocDefault));
     CHUI_HIP(hipMemcpyAsync(ptr, dev, bytes, hipMemcpyDeviceToHost, s));
     CHUI_HIP(hipStreamSynchronize(s));
