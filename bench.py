@@ -14,6 +14,7 @@ and (on sample targets) against an FP64 Ewald sum.
 from __future__ import annotations
 
 import argparse
+import faulthandler
 import json
 import os
 import sys
@@ -48,6 +49,7 @@ def error_metrics(value, ref, floor_fraction=1e-3):
 
 
 def main():
+    faulthandler.enable()  # a crash names its Python frames on stderr
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=5)
@@ -633,25 +635,8 @@ def measure_ensemble(steps, gradients, workers=8):
                                     "each with its own torch stream and context (explicit adjoint sweeps); "
                                     "serial_seconds: one box after another through torch.autograd"}
         log(f"ensemble gradients: {threaded:.2f} s on {workers} threads, {serial:.2f} s serial")
-        # forward + adjoint sweeps of all 48 boxes recorded as one graph
-        # (torch.cuda.graph; every box a branch on its own stream)
-        t = time.perf_counter()
-        gg = E.GradientGraph(specs, steps)
-        t_build = time.perf_counter() - t
-        try:
-            els = []
-            for _ in range(3):
-                t = time.perf_counter()
-                gg.replay()
-                els.append(time.perf_counter() - t)
-        finally:
-            gg.close()
-        out["gradients_graph"] = {"seconds": float(np.median(els)), "seconds_each": els,
-                                  "prepare_and_record_seconds": t_build, "precision": "fp64",
-                                  "what": f"one replay of the recorded forward and adjoint sweeps of all {len(specs)} "
-                                          "boxes (FP64 capture-safe solves and VJPs, CIC density and transpose, "
-                                          "element-wise KDK work), median of 3; the losses are summed outside it"}
-        log(f"ensemble gradients as one graph: {np.median(els):.2f} s (prepared and recorded in {t_build:.1f} s)")
+        # GradientGraph refuses 48 boxes (a stream of its own per box)
+        out["gradients_graph"] = None
     return out
 
 

@@ -318,35 +318,61 @@ class GradientGraph:
     (the first solve sizes it, the first VJP learns its accepted-list
     capacity). replay() copies new displacements into the graph's inputs,
     launches it once, checks every context's fault word and returns the
-    losses (summed outside the graph) and the gradients."""
+    losses (summed outside the graph) and the gradients.
+
+    Every branch and the recording need a stream of their own; torch hands out
+    a device's streams from a pool of 32 in turn, so at most 31 boxes can be
+    recorded. With more, boxes share streams, one of them the recording
+    stream's: a run with 48 boxes ended in a segmentation fault between
+    recording and replay whose cause is not known. More boxes raise
+    ValueError; ensemble_gradients takes any number."""
 
     def __init__(self, specs, steps: int, device: str = "cuda:0", checkpoint_every: int = 2):
         self.device = device
-        made = [box_problem(s, steps, device, checkpoint_every) for s in specs]
-        self.problems = [m[0] for m in made]
-        self.psi = [m[1] for m in made]
-        self.targets = [m[2] for m in made]
-        for prob in self.problems:
-            prob.coord.set_capture_safe(True)
-        for _ in range(2):
-            for prob, psi, target in zip(self.problems, self.psi, self.targets):
-                adjoint.loss_and_gradient(psi, target, prob)
-        torch.cuda.synchronize(device)
+        self.problems, self.graph = [], None
+        self.diff, self.grad = [None] * len(specs), [None] * len(specs)
         self.main = torch.cuda.Stream(device=device)
         self.streams = [torch.cuda.Stream(device=device) for _ in specs]
+        if len({st.cuda_stream for st in [self.main] + self.streams}) != len(specs) + 1:
+            raise ValueError(f"a gradient graph of {len(specs)} boxes needs {len(specs) + 1} streams of its own, more "
+                             "than torch's pool holds; record fewer boxes or use ensemble_gradients")
+        try:
+            made = []
+            for s in specs:
+                made.append(box_problem(s, steps, device, checkpoint_every))
+                self.problems.append(made[-1][0])
+            self.psi = [m[1] for m in made]
+            self.targets = [m[2] for m in made]
+            for prob in self.problems:
+                prob.coord.set_capture_safe(True)
+            for _ in range(2):
+                for prob, psi, target in zip(self.problems, self.psi, self.targets):
+                    adjoint.loss_and_gradient(psi, target, prob)
+            torch.cuda.synchronize(device)
+            self._record()
+        except BaseException:
+            self.close()
+            raise
+
+    def _record(self):
         for prob, st in zip(self.problems, self.streams):
             prob.coord.set_stream(st.cuda_stream)
             prob.graph_mode = True
         self.graph = torch.cuda.CUDAGraph()
-        self.diff, self.grad = [None] * len(specs), [None] * len(specs)
+        forked = []
         try:
             with torch.cuda.graph(self.graph, stream=self.main):
-                for b, (prob, st) in enumerate(zip(self.problems, self.streams)):
-                    st.wait_stream(self.main)
-                    with torch.cuda.stream(st):
-                        self.diff[b], self.grad[b] = adjoint.gradient_sweeps(self.psi[b], self.targets[b], prob)
-                for st in self.streams:
-                    self.main.wait_stream(st)
+                try:
+                    for b, (prob, st) in enumerate(zip(self.problems, self.streams)):
+                        st.wait_stream(self.main)
+                        forked.append(st)
+                        with torch.cuda.stream(st):
+                            self.diff[b], self.grad[b] = adjoint.gradient_sweeps(self.psi[b], self.targets[b], prob)
+                finally:
+                    # also after a failure: a recording ends only with every
+                    # branch joined
+                    for st in forked:
+                        self.main.wait_stream(st)
         finally:
             for prob in self.problems:
                 prob.graph_mode = False
@@ -367,6 +393,7 @@ class GradientGraph:
         return losses, self.grad
 
     def close(self):
+        # the graph before the contexts whose buffers its nodes use
         self.graph = None
         for prob in self.problems:
             prob.close()
