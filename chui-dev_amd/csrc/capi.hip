@@ -420,8 +420,21 @@ chui::WalkParams base_walk_params(const Ctx* c, const chui_treepm_options* o, co
     const double sep = wp.cubic ? o->box_size[0] / 4294967296.0 : 1.0;
     const double r2 = wp.rcut2 / (sep * sep);
     wp.rcut2_sep = static_cast<float>(r2);
-    wp.prune2_sep = static_cast<float>(r2 * (1.0 + 1.0e-5));
+    wp.cell_prune2_sep = static_cast<float>(r2 * (1.0 + 1.0e-5));
     wp.contain2_sep = static_cast<float>(r2 * (1.0 - 1.0e-5));
+    // A node box's separation from a target box takes five FP32 roundings per
+    // axis (the difference's conversion, the unit, the product, two
+    // subtractions), each of at most 2^-24 of half the axis: coarse nodes of a
+    // box of several hundred r_cut would be pruned with a pair inside r_cut if
+    // the cutoff were widened by a fraction of r_cut alone (5e-6 of it covers
+    // the squares and their sum).
+    double slack2 = 0.0;
+    for (int a = 0; a < 3; ++a) {
+      const double slack = 5.0 * std::ldexp(0.5 * o->box_size[a], -24);
+      slack2 += slack * slack;
+    }
+    const double reach = (sp.rcut + std::sqrt(slack2)) / sep;
+    wp.prune2_sep = static_cast<float>(reach * reach * (1.0 + 1.0e-5));
   }
   for (int a = 0; a < 3; ++a) {
     // a run of targets shares one traversal when it lies within +-r_cut of its

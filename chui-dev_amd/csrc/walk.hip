@@ -2030,9 +2030,10 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
   else walk.template operator()<false>(node_count);
   fold();
 
-  // Replay the reference's walk over the octree
-  // cells (no pair work) for its per-target node counters.
+  // Replay the reference's walk over the octree cells (no pair work) for its
+  // per-target node counters.
   {
+    const float cell_prune2 = P.cell_prune2_sep;
     uint32_t cnxt = valid ? 0u : node_count;
     uint32_t n = wave_min_u32(cnxt);
     while (n < node_count) {
@@ -2045,7 +2046,7 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
       const float ax_ = fabsf(fx_delta(g.cx, px, s0)), ay_ = fabsf(fx_delta(g.cy, py, s1)),
                   az_ = fabsf(fx_delta(g.cz, pz, s2));
       const float ex = fmaxf(0.0f, ax_ - h), ey = fmaxf(0.0f, ay_ - h), ez = fmaxf(0.0f, az_ - h);
-      const bool keep = act && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > prune2);
+      const bool keep = act && !(fmaf(ex, ex, fmaf(ey, ey, ez * ez)) > cell_prune2);
       cnt[1] += act && !keep;
       if (lk.child_count == 0) {
         cnt[4] += keep;

@@ -39,7 +39,10 @@ struct WalkParams {
   // cubic-cell table of H(t) = L(sqrt t)/t^{3/2}, t = r^2/(4 a^2).
   int cubic;
   float fx_to_len[3];  // L / 2^32
-  float rcut2_sep, prune2_sep, contain2_sep;
+  // prune2_sep covers the roundings of a box separation anywhere in the box;
+  // cell_prune2_sep (r_cut and 5e-6 of it) prunes the counters' replay of the
+  // octree cells.
+  float rcut2_sep, prune2_sep, cell_prune2_sep, contain2_sep;
   float c4, c8;        // 1/(4 a^2), 1/(8 a^3)
   float t_to_cell;     // r^2 -> table cell coordinate
   // Largest half-extent (fixed-point units, per axis) of a wave's targets for

@@ -84,3 +84,79 @@ def test_box_walk_matches_counting_walk(case, precision):
         assert np.all(timed == 0.0)
     else:
         assert rel_l2(timed, counted) < (2e-6 if precision == L.PRECISION_MIXED else 1e-12)
+
+
+# ---- large boxes: L / r_cut in the hundreds and thousands ----------------------
+# Node boxes are tested in FP32 differences of 32-bit fixed point, which round
+# by up to 64 units at separations of a quarter box; r_cut is 2^32 / (L / r_cut)
+# units. The sources below are a chain along x cut by the root's centre plane
+# just inside r_cut of the target, so that the half beyond the plane is one leaf
+# whose nearest source is the pair at r_cut, and the positions are drawn until
+# rounded_excess, the arithmetic of that test, puts the leaf beyond
+# r_cut (1 + 5e-6): a margin that does not cover the rounding loses the pair.
+CHAIN = 1200
+INSIDE = 1e-6  # the pair lies at r_cut (1 - INSIDE): both precisions count it
+
+
+def float_up(x):
+    f = np.float32(x)
+    return np.where(f.astype(np.float64) < x, np.nextafter(f, np.float32(np.inf)), f)
+
+
+def rounded_excess(target, first, last, L, cubic, half_units):
+    """Separation of a leaf [first, last] and a target along x in the kernel's
+    FP32 steps, lengths in the separation unit (fixed point, or L / 2^32)."""
+    scale = 4294967296.0 / L
+    d = np.floor(0.5 * (first + last) * scale).astype(np.int64) - np.floor(target * scale).astype(np.int64)
+    half = 0.5 * (last - first)
+    unit = np.float32(1.0 if cubic else L / 4294967296.0)
+    hx = float_up(half * scale + 2.0) if cubic else float_up(half + 2.0 / scale)
+    return (np.abs(d.astype(np.float32) * unit) - hx) - np.float32(half_units) * unit
+
+
+def boundary_chain(ratio, L, cubic, half_units):
+    """x of the chain (its target is particle CHAIN // 2 - 1) and r_cut."""
+    rng = np.random.default_rng(int(ratio))
+    for _ in range(400):
+        rc = L / (ratio * (1.0 + 0.01 * rng.random()))
+        lo = 1e-4 * L * rng.random(4096)
+        hi = L * (1.0 - 1.6 / CHAIN) + lo * rng.random(4096)
+        target = 0.5 * (lo + hi) - rc * rng.uniform(0.45, 0.55, 4096)
+        first = target + rc * (1.0 - INSIDE)
+        sep = L / 4294967296.0 if cubic else 1.0
+        e = rounded_excess(target, first, hi, L, cubic, half_units)
+        lost = np.flatnonzero(e.astype(np.float64) * sep > rc * (1.0 + 5.5e-6))
+        if lost.size:
+            k = lost[0]
+            n = CHAIN // 2
+            left = np.linspace(lo[k], target[k] - 0.3 * rc, n - 2)
+            right = np.linspace(first[k] + 0.3 * rc, hi[k], n - 1)
+            # one source before the centre, so that the widest gap is the wrap
+            mid = 0.5 * (lo[k] + hi[k]) - 0.01 * rc
+            return np.concatenate([left, [mid, target[k], first[k]], right]), rc
+    raise AssertionError("no separation where the rounding shows")
+
+
+@pytest.mark.parametrize("ratio", [500, 2000])
+@pytest.mark.parametrize("box", [(1.0, 1.0, 1.0), (1.3, 1.3, 0.8)], ids=["cubic", "slab"])
+def test_pairs_just_inside_the_cutoff_of_a_large_box(box, ratio):
+    cubic = len(set(box)) == 1
+    mesh = 32
+    for precision, half_units in ((L.PRECISION_FP64, 4.000004), (L.PRECISION_MIXED, 2.0)):
+        x, rc = boundary_chain(ratio, box[0], cubic, half_units)
+        y, z = np.full(CHAIN, 0.4 * box[1]), np.full(CHAIN, 0.3 * box[2])
+        m = np.random.default_rng(3).uniform(0.5, 1.5, CHAIN)
+        o = options_struct(box, eps=0.0, leaf=1024, rcut_cells=rc / (np.cbrt(box[0] * box[1] * box[2]) / mesh))
+        o.target_mapping = L.TARGETS_PER_LANE
+        o.short_range_only = 1
+        target = CHAIN // 2 - 1
+        active = np.array([target])
+        o.precision = L.PRECISION_FP64
+        ref = short_range(x, y, z, m, o, mesh, active, True)[:, target]
+        o.precision = precision
+        # FP32 pairs and fixed-point positions: 1e-4 of this target's few pairs
+        # is far below the lost pair's share
+        bound = 1e-12 if precision == L.PRECISION_FP64 else 1e-4
+        for counted in (False, True):
+            got = short_range(x, y, z, m, o, mesh, active, counted)[:, target]
+            assert np.linalg.norm(got - ref) < bound * np.linalg.norm(ref), (precision, counted)
