@@ -2384,7 +2384,8 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
   const float4* const lcell = ltab - P.log_base;
   const uint32_t lbase = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_f32x4*)ltab - P.log_base));
 
-  const float far = 64.0f * sqrtf(rc2);
+  // beyond r_cut of every target whose offset the origin admits (2^28 units per axis)
+  const float far = 2.0f * fmaf(268435456.0f, fmaxf(u0, fmaxf(u1, u2)), sqrtf(rc2));
   // --- the counting walk's origin (SHARED), else the segment's ---
   uint32_t wox = 0, woy = 0, woz = 0;
   bool wave_origin = false;
@@ -2710,7 +2711,7 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
             while (wn >= static_cast<uint32_t>(kWindow) || (last && wn)) {
               const uint32_t cn = wn < static_cast<uint32_t>(kWindow) ? wn : static_cast<uint32_t>(kWindow);
               if (static_cast<uint32_t>(lane) >= cn) {
-                // dummies beyond r_cut of everything fill the last window (in
+                // dummies beyond r_cut of every target fill the last window (in
                 // fixed point half a period from the box centre per axis)
                 win[slot_of(lane)] = !SHARED || wave_origin ? make_float4(far, far, far, 0.0f)
                                                  : make_float4(__uint_as_float(ox ^ 0x80000000u),

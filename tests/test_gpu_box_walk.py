@@ -160,3 +160,19 @@ def test_pairs_just_inside_the_cutoff_of_a_large_box(box, ratio):
         for counted in (False, True):
             got = short_range(x, y, z, m, o, mesh, active, counted)[:, target]
             assert np.linalg.norm(got - ref) < bound * np.linalg.norm(ref), (precision, counted)
+
+
+def test_window_fill_lies_beyond_every_target():
+    # two targets L / 10 apart share a wave's origin halfway between them; the
+    # records that fill a window past its sources must lie beyond r_cut of
+    # both, wherever r_cut = L / 1280 puts them: neither has a pair
+    box, mesh = 1.0, 32
+    rc = box / 1280
+    for cells in (60.0, 64.2, 70.0):
+        p = np.array([0.5 - cells * rc, 0.5 + cells * rc])
+        for eps in (0.0, 0.01 * rc):
+            o = options_struct(box, eps=eps, rcut_cells=mesh / 1280)
+            o.precision = L.PRECISION_MIXED
+            o.target_mapping = L.TARGETS_PER_LANE
+            o.short_range_only = 1
+            assert np.all(short_range(p, p, p, np.ones(2), o, mesh, None, False) == 0.0), (cells, eps)
