@@ -9,6 +9,8 @@ Every tree equals the oracle's bit for bit (no tolerance).
 """
 from __future__ import annotations
 
+import time
+
 import numpy as np
 import pytest
 
@@ -42,6 +44,13 @@ def tight(n, width):
     return x, y, z, m
 
 
+def coincident(n, distinct):
+    # points at `distinct` places about 1e-13 apart: one leaf at the smallest cell
+    rng = np.random.default_rng(n)
+    p = 2.0 + 1e-13 * rng.integers(0, distinct, (3, n)) if distinct > 1 else np.full((3, n), 2.0)
+    return p[0].copy(), p[1].copy(), p[2].copy(), rng.uniform(0.5, 1.5, n)
+
+
 def check_tree(coord, sources, leaf):
     x, y, z, m = sources
     acc = tuple(empty_dev(x.size, torch.float64) for _ in range(3))
@@ -56,6 +65,15 @@ def check_tree(coord, sources, leaf):
     assert diag["leaf_count"] == int(np.all(ref["child_index"] == 0xFFFFFFFF, axis=1).sum())
 
 
+def check_build_only(coord, sources):
+    acc = tuple(empty_dev(1, torch.float64) for _ in range(3))
+    active = to_dev(np.zeros(1, np.int32))[0]
+    o = options_struct(BOX, eps=0.02, leaf=16)
+    o.short_range_only = 1
+    coord.solve_active_set_with_pm_cadence(*to_dev(*sources), ForceAccumulator(acc, active), o, False)
+    coord.synchronize()
+
+
 @pytest.mark.parametrize("n,leaf", [(1, 16), (2, 1), (511, 16), (512, 16), (513, 17), (1025, 32), (1200, 33),
                                     (1030, 64), (1500, 65), (2500, 1), (3000, 300), (5000, 1024), (20000, 3)])
 def test_tree_matches_oracle(n, leaf):
@@ -68,3 +86,15 @@ def test_rebuilds_of_changing_depth_match_oracle():
         for sources in (uniform(700), tight(3000, 2.0**-15), uniform(200), tight(3000, 2.0**-18), uniform(5000),
                         clustered(4000, 3, BOX)):
             check_tree(coord, sources, 16)
+
+
+@pytest.mark.parametrize("n,distinct", [(65, 1), (70, 3), (2000, 4), (40000, 1)])
+def test_leaf_at_the_smallest_cell_matches_oracle(n, distinct):
+    with TreePmCoordinator((16, 16, 16)) as coord:
+        sources = coincident(n, distinct)
+        check_tree(coord, sources, 16)
+        # a leaf holds any number of coincident sources; ordering it takes no
+        # time that grows with their square (40000 would take seconds)
+        start = time.perf_counter()
+        check_build_only(coord, sources)
+        assert time.perf_counter() - start < 1.0
