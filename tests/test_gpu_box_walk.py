@@ -176,3 +176,41 @@ def test_window_fill_lies_beyond_every_target():
             o.target_mapping = L.TARGETS_PER_LANE
             o.short_range_only = 1
             assert np.all(short_range(p, p, p, np.ones(2), o, mesh, None, False) == 0.0), (cells, eps)
+
+
+# ---- above 2^20 sources: the segment's own origin ------------------------------
+@pytest.mark.parametrize("kind", ["uniform", "clustered", "slab"])
+@pytest.mark.parametrize("stride", [None, 1001], ids=["all", "sparse"])
+def test_mixed_walk_above_2_20_sources_matches_counting_walk(kind, stride):
+    # a ragged count, spread masses; clusters give waves whose segments are
+    # halved, windows that overflow and last windows that are filled up
+    n = (1 << 20) + 4097
+    box = (60.0, 90.0, 120.0) if kind == "slab" else (100.0, 100.0, 100.0)
+    rng = np.random.default_rng(11)
+    p = rng.uniform(0.0, 1.0, (3, n))
+    if kind == "clustered":
+        c = rng.uniform(0.0, 1.0, (3, 200))
+        k = n // 4
+        p[:, :k] = np.mod(c[:, rng.integers(0, 200, k)] + rng.normal(0.0, 3e-3, (3, k)), 1.0)
+    x, y, z = (np.minimum(p[a] * box[a], np.nextafter(box[a], 0.0)) for a in range(3))
+    m = rng.uniform(0.5, 1.5, n)
+    mesh = 128
+    o = options_struct(box, G=1.0, eps=0.1)  # close pairs soft: their separations round differently
+    o.precision = L.PRECISION_MIXED
+    o.target_mapping = L.TARGETS_PER_LANE
+    o.short_range_only = 1
+    active = None if stride is None else np.arange(0, n, stride)
+    timed = short_range(x, y, z, m, o, mesh, active, False)
+    counted = short_range(x, y, z, m, o, mesh, active, True)
+    # The sums' order differs (FP32, the 2e-6 above), and a pair whose
+    # separation rounds across r_cut is counted by one walk only, with 1.8e-2
+    # of Newton's force: a share 3 d of a target's pairs for a relative rounding
+    # d. Offsets of some r_cut round by 2^-24 of themselves in each walk, so d is
+    # about 1e-7 (one pair in 7e6 differs at these counts); one in 2.6e6 is allowed.
+    rc = 4.5 * 1.25 * np.cbrt(np.prod(box)) / mesh
+    targets = n if active is None else active.size
+    pairs = targets * n / np.prod(box) * 4.0 / 3.0 * np.pi * rc**3 * (4.0 if kind == "clustered" else 1.0)
+    flips = np.sqrt(1.0 + pairs / 2.6e6) * 1.5 * 1.8e-2 / rc**2
+    assert np.all(np.isfinite(timed))
+    err, norm = np.linalg.norm(timed - counted), np.linalg.norm(counted)
+    assert err < 2e-6 * norm + flips

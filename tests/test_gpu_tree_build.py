@@ -98,3 +98,10 @@ def test_leaf_at_the_smallest_cell_matches_oracle(n, distinct):
         start = time.perf_counter()
         check_build_only(coord, sources)
         assert time.perf_counter() - start < 1.0
+
+
+@pytest.mark.parametrize("n", [(1 << 21) - 3, (1 << 21) + 5])
+def test_tree_on_both_sides_of_the_device_frame(n):
+    # up to 2^21 sources the build's frame stays on the device, beyond it is read back
+    with TreePmCoordinator((96, 96, 96)) as coord:
+        check_tree(coord, uniform(n), 16)
