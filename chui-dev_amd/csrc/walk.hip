@@ -1094,14 +1094,23 @@ template <class T> __device__ __forceinline__ T scan_max(T v, int lane) {
   return v;
 }
 
-// inclusive maximum over the lanes up to this one (all 64 active)
-__device__ __forceinline__ uint32_t group_scan_max(uint32_t v) {
-  v = dpp_max_step(v, CHUI_DPP(v, 0x111, 0xf, 0u));  // row_shr:1
-  v = dpp_max_step(v, CHUI_DPP(v, 0x112, 0xf, 0u));  // row_shr:2
-  v = dpp_max_step(v, CHUI_DPP(v, 0x114, 0xf, 0u));  // row_shr:4
-  v = dpp_max_step(v, CHUI_DPP(v, 0x118, 0xf, 0u));  // row_shr:8
-  v = dpp_max_step(v, CHUI_DPP(v, 0x142, 0xa, 0u));  // row_bcast:15
-  v = dpp_max_step(v, CHUI_DPP(v, 0x143, 0xc, 0u));  // row_bcast:31
+// inclusive sum / maximum over the lanes up to this one (all 64 active)
+__device__ __forceinline__ uint32_t wave_scan_sum(uint32_t v) {
+  v += CHUI_DPP(v, 0x111, 0xf, 0u);  // row_shr:1
+  v += CHUI_DPP(v, 0x112, 0xf, 0u);  // row_shr:2
+  v += CHUI_DPP(v, 0x114, 0xf, 0u);  // row_shr:4
+  v += CHUI_DPP(v, 0x118, 0xf, 0u);  // row_shr:8
+  v += CHUI_DPP(v, 0x142, 0xa, 0u);  // row_bcast:15
+  v += CHUI_DPP(v, 0x143, 0xc, 0u);  // row_bcast:31
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_scan_max(uint32_t v) {
+  v = dpp_max_step(v, CHUI_DPP(v, 0x111, 0xf, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x112, 0xf, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x114, 0xf, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x118, 0xf, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x142, 0xa, 0u));
+  v = dpp_max_step(v, CHUI_DPP(v, 0x143, 0xc, 0u));
   return v;
 }
 // LDS written by some lanes of the wave is read by others after this
@@ -1417,11 +1426,7 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
         for (uint32_t c = 0; c < nl; c += kWave) {
           const uint32_t e = c + lane;
           const uint32_t own = e < nl ? leaves[e].e - leaves[e].b : 0u;
-          uint32_t incl = own;
-          for (int off = 1; off < kWave; off <<= 1) {
-            const uint32_t o = __shfl_up(incl, off, kWave);
-            if (lane >= off) incl += o;
-          }
+          const uint32_t incl = wave_scan_sum(own);
           if (e < nl) leaf_pre[e] = total + incl - own;
           total += readlane_u32(incl, kWave - 1);
         }
@@ -1437,7 +1442,7 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
           const uint32_t st = e < nl ? leaf_pre[e] - g0 : static_cast<uint32_t>(kWave);
           if (st < static_cast<uint32_t>(kWave)) mark[st] = lane + 1u;
           wave_sync();
-          const uint32_t lf = e0 + group_scan_max(mark[lane]);
+          const uint32_t lf = e0 + wave_scan_max(mark[lane]);
           const uint32_t g = g0 + lane;
           const bool on = g < total;
           const uint32_t j = on ? leaves[lf].b + (g - leaf_pre[lf]) : 0u;
@@ -2139,25 +2144,6 @@ struct BoxFrame {
   float to_len;
 };
 
-// inclusive sum / maximum over the lanes up to this one (all 64 active)
-__device__ __forceinline__ uint32_t wave_scan_sum(uint32_t v) {
-  v += CHUI_DPP(v, 0x111, 0xf, 0u);  // row_shr:1
-  v += CHUI_DPP(v, 0x112, 0xf, 0u);  // row_shr:2
-  v += CHUI_DPP(v, 0x114, 0xf, 0u);  // row_shr:4
-  v += CHUI_DPP(v, 0x118, 0xf, 0u);  // row_shr:8
-  v += CHUI_DPP(v, 0x142, 0xa, 0u);  // row_bcast:15
-  v += CHUI_DPP(v, 0x143, 0xc, 0u);  // row_bcast:31
-  return v;
-}
-__device__ __forceinline__ uint32_t wave_scan_max(uint32_t v) {
-  v = dpp_max_step(v, CHUI_DPP(v, 0x111, 0xf, 0u));
-  v = dpp_max_step(v, CHUI_DPP(v, 0x112, 0xf, 0u));
-  v = dpp_max_step(v, CHUI_DPP(v, 0x114, 0xf, 0u));
-  v = dpp_max_step(v, CHUI_DPP(v, 0x118, 0xf, 0u));
-  v = dpp_max_step(v, CHUI_DPP(v, 0x142, 0xa, 0u));
-  v = dpp_max_step(v, CHUI_DPP(v, 0x143, 0xc, 0u));
-  return v;
-}
 // centre and half-extent of v over this lane's row of 16 lanes (all active);
 // the half-extent covers the rounding of the centre
 __device__ __forceinline__ void row_bounds(float v, float& centre, float& half) {
