@@ -452,10 +452,15 @@ chui::WalkParams base_walk_params(const Ctx* c, const chui_treepm_options* o, co
     const double lim = std::min(268435456.0, 2147483648.0 - rcut_units - 16777216.0);
     wp.fast_half_extent[a] = lim > 0.0 ? static_cast<uint32_t>(lim) : 0u;
   }
+  // FP64 runs may be wider, since their groups of 16 targets cull again:
+  // +-r_cut 96^3 5.00 against 4.39 ms, VJP of 64^3 2.47 against 2.34 ms;
+  // +-4 r_cut 4.38 against 4.52 ms, but 2.88 against 2.30 ms and a 32^3 step 606
+  // against 538 us
   wp.box_max64 = 2.0 * sp.rcut;
   wp.box_single = std::min({wp.fast_half_extent[0], wp.fast_half_extent[1], wp.fast_half_extent[2]}) >= 2u ? 1 : 0;
   // up to 2^20 sources a pair on the other side of r_cut shows in the force
-  // field's relative L2 (walkmix_box_kernel)
+  // field's relative L2: its side is kept independent of the launch shape
+  // (walkmix_box_kernel)
   wp.shared_origin = c->tree.n <= (1u << 20) ? 1 : 0;
   wp.node_count = static_cast<uint32_t>(c->tree.node_count);
   wp.mesh_row = mesh_row;
@@ -773,13 +778,14 @@ void solve_device_impl(Ctx* c, const double* x, const double* y, const double* z
   wp.identity_targets = identity;
   // the mixed walk's counting variant also produces the nearest-pair lane
   wp.count = (diag != nullptr || wcount != nullptr || (mixed && near2 != nullptr)) ? 1 : 0;
-  // one target per wave when asked, or when few sources are active: 64
-  // visit-ordered targets then lie far apart and a shared walk covers the
-  // union of their neighbourhoods, costing about a full walk whatever the
-  // active count. The measured short-range-only crossovers fall with the
-  // source count: mixed 2-3% active at 256^3 (clustered, 1065 pairs per
-  // target), 12% at 128^3 and 35% at 64^3; FP64 15% at 128^3. Auto switches
-  // at f(n) = min(0.25, f0 (2^24 / n)^0.75), f0 = 0.025 (mixed) or 0.03 (FP64).
+  // one target per wave when asked, or when few sources are active. Auto
+  // switches at f(n) = min(0.25, f0 (2^24 / n)^0.75), f0 = 0.025 (mixed) or 0.03
+  // (FP64): the short-range-only crossovers of a shared walk that covered the
+  // union of its 64 targets' neighbourhoods (mixed 2-3% active at 256^3, 12% at
+  // 128^3, 35% at 64^3; FP64 15% at 128^3). The present shared walk cuts distant
+  // targets into segments and is faster above 0.2 to 1% (per lane and per wave:
+  // 256^3 mixed 2% 10.1 and 13.1 ms; 128^3 mixed 5% 1.49 and 1.99, FP64 10% 2.5
+  // and 11.1; 64^3 mixed 1% 0.50 and 0.49), so the line lies too high.
   const double f0 = mixed ? 0.025 : 0.03;
   const double f_switch = std::min(0.25, f0 * std::pow(16777216.0 / static_cast<double>(std::max<uint64_t>(n, 1)), 0.75));
   const bool sparse = static_cast<double>(n_active) <= f_switch * static_cast<double>(n);

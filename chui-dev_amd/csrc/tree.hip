@@ -1,4 +1,4 @@
-// tree.hip — periodic unwrap, octant-path keys, level-synchronous octree build,
+// tree.hip — periodic unwrap, octant-path keys, octree from shared key digits,
 // preorder numbering, in-leaf Morton order and FP64 multipoles on gfx950.
 //
 // The reference builds its octree top-down by recursive stable octant
@@ -8,8 +8,9 @@
 //   1. every particle computes its 21-level octant path against the exact FP64
 //      centre sequence c +- h/2 (the centres the recursion would visit);
 //   2. one stable radix sort by that path gives the preorder leaf sequence;
-//   3. nodes are discovered level by level with binary searches on the sorted
-//      paths (a node is split while count > leaf_size and half > 1e-12);
+//   3. the nodes follow from the octant digits that sorted paths share, all
+//      levels in one pass (a node is split while count > leaf_size and
+//      half > 1e-12);
 //   4. inside each leaf the particles are put back into Morton order, because
 //      stable partitions preserve the Morton order of a leaf's members.
 // All FP64 arithmetic that decides topology or feeds multipoles is written in
@@ -1307,7 +1308,8 @@ __global__ __launch_bounds__(256) void leaf_order_kernel(uint32_t total_nodes, c
       big &= big - 1ull;
       const uint32_t bb = readlane_u32(b, s), bc = readlane_u32(c, s);
       // coincident sources come in order from the stable sort, any number of
-      // them in one leaf: they are only copied
+      // them in one leaf: they are only copied (a solve of 6000: ranked 282 ms,
+      // copied 1.1 ms)
       bool sorted = true;
       for (uint32_t e0 = 0; e0 + 1u < bc && sorted; e0 += kWave) {
         bool ok = true;
@@ -1343,8 +1345,8 @@ __global__ __launch_bounds__(256) void leaf_order_kernel(uint32_t total_nodes, c
 // Moments of one subtree per block, all its levels in one launch (bound by the
 // loads of each level waiting for the level below; a launch per level took 13
 // to 15 launches of 4 to 60 us, hence subtrees of max(512, n / 1024) particles:
-// a thousand or more blocks, and at most a few thousand nodes above them). A subtree's
-// nodes of each depth are consecutive, from the first child of the first split
+// above 5e5 particles a thousand or more blocks and at most a few thousand nodes
+// above them; 32^3 has about 64 blocks). A subtree's nodes of each depth are consecutive, from the first child of the first split
 // node of the depth above to the last child of the last.
 __global__ __launch_bounds__(256) void moment_subtree_kernel(MomArgs a, MomArrays o, const uint32_t* __restrict__ lv,
                                                              const uint32_t* __restrict__ subs,

@@ -78,7 +78,7 @@ struct TreeParams {
   bool mixed = false;  // emit the fixed-point records; the FP64 records follow on demand
   // Capture-safe build: no read-back and no allocation once prepared; every
   // per-build value stays on the device and data-dependent failures set bits
-  // of *fault (mixed precision only).
+  // of *fault.
   bool capture_safe = false;
   unsigned long long* fault = nullptr;
   // An ordinary build that sizes every buffer as a capture-safe build of the
@@ -102,7 +102,7 @@ struct Tree {
   std::size_t prepared_n = 0;
   bool counts_on_device = false;
   bool sized_for_capture = false;  // the last ordinary build sized its buffers for capture-safe builds
-  DeviceBuffer frame;  // Frame of the last capture-safe build
+  DeviceBuffer frame;  // Frame of the last build that kept it on the device
   UnwrapResult unwrap{};
   bool mass_uniform = false;
   double uniform_mass = 0.0;
@@ -133,7 +133,7 @@ struct Tree {
 };
 
 // Bounds/canonical check, periodic unwrap on all three axes, Morton/path keys,
-// stable sort, level-synchronous octree, preorder numbering, in-leaf Morton
+// stable sort, octree from shared key digits, preorder numbering, in-leaf Morton
 // order and multipoles. Inputs are device pointers (caller positions/masses).
 void build_tree(Tree& t, const double* x, const double* y, const double* z, const double* m,
                 const TreeParams& p, double softening, hipStream_t s);
@@ -149,8 +149,9 @@ void ensure_records64(Tree& t, hipStream_t s);
 
 // Mesh-deposit units of the last built tree: the shallowest subtrees whose
 // particles span at most d.max_cells cells (or leaves that never do). Reads
-// back the unit and block counts, or after a capture-safe build leaves them on
-// the device (DepositUnits::dev_counts) and sizes the launch by a bound.
+// back the unit and block counts, or after a capture-safe build and for up to
+// kFrameMax sources leaves them on the device (DepositUnits::dev_counts) and
+// sizes the launch by a bound.
 DepositUnits build_deposit_units(Tree& t, const DepositTiling& d, hipStream_t s);
 
 // Morton keys + stable order of given (unwrapped) device coordinates.

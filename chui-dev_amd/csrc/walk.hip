@@ -1667,9 +1667,10 @@ __device__ __forceinline__ void group_walk_body(const WalkParams& P, const Group
 
 // Two waves per SIMD (256 VGPRs) where the FP64 node expansions are inline:
 // the body needs about that many; at 168 VGPRs (3 waves) it spilled 384-512
-// bytes per lane and ran 2% (FP64) to 29% (mixed) slower at 256^3. The mixed
-// walk with FP32 node expansions (RADIAL false) holds 142 VGPRs and runs 3
-// waves per SIMD (4 waves: 128 VGPRs with spills, 16% slower).
+// bytes per lane and ran 2% (FP64) to 29% (mixed) slower at 256^3 (the walk
+// before the stack; now 256 VGPRs spill 24 to 27 of them). The mixed walk with
+// FP32 node expansions (RADIAL false) holds 152 VGPRs without spills and runs 3
+// waves per SIMD (4 waves: 128 VGPRs with spills, 16% slower, before the stack).
 template <int SCHEME, bool TAB>
 __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(2))) void group_walk64_kernel(
     WalkParams P, GroupParams G, WalkData D, const uint32_t* __restrict__ leaf_of_pos, WalkOutputs out,
@@ -1741,7 +1742,6 @@ __global__ void leaf_of_pos_kernel(const NodeLink* __restrict__ link, std::size_
 // ---- mixed walk -----------------------------------------------------------------
 // CUBIC: equal box lengths, so separations stay in fixed-point units (one
 // scale factor for all axes) and only the pair kernel converts to lengths.
-// COUNT: keep the per-target counters (diagnostic launches only).
 //
 // A leaf that any lane keeps is staged in the wave's LDS window with one
 // coalesced load (one source per lane). Every lane then evaluates the residual
@@ -1762,20 +1762,8 @@ __global__ void leaf_of_pos_kernel(const NodeLink* __restrict__ link, std::size_
 // Waves that straddle a jump of the space-filling order (targets far apart)
 // store raw fixed-point coordinates and form int32(q_s - q_t) per pair.
 //
-// Box-classified traversal (BOX, the timed walk). A wave whose targets lie in
-// a box of half-extent at most box_half_max (2 r_cut) per axis walks the tree
-// once for that box instead of node by node for its 64 lanes: the lanes classify 64
-// consecutive preorder nodes at a time against the box (pruned when the
-// node's tight particle box lies beyond r_cut of the target box, i.e. beyond
-// r_cut of every target), a scalar loop follows the visited chain through the
-// window, and the kept leaves' sources go to a 128-entry ring in LDS that is
-// evaluated one 64-source window at a time with the pair kernel above (each
-// lane keeps only its own pairs inside r_cut). Only internal nodes of cells
-// small enough for the strict acceptance (h < 0.041 r_cut) and not within
-// 25 h of every target (where 2h/r < 0.08 fails for all of them) can be
-// accepted by some lane; their subtrees are walked lane by lane as above.
-// The pairs and multipoles are therefore those of the lane-by-lane walk;
-// only the summation order differs.
+// The timed walk is walkmix_box_kernel below: the same pairs and multipoles
+// from a traversal per box of targets, summed in another order.
 constexpr int kWindow = 64;
 constexpr int kPairGroup = 2;  // box walk: table reads in flight together
 
@@ -2119,10 +2107,13 @@ void walkmix_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long lon
 // are scanned across the lanes, each leaf marks its first slot of the batch,
 // and a running maximum spreads the leaf over its slots. The next batch's
 // records are in flight while the current one is culled and evaluated.
-constexpr uint32_t kBoxGroup = 16;     // targets per evaluation group: a DPP row
+constexpr uint32_t kBoxGroup = 16;     // FP64: targets per evaluation group, a DPP row
 constexpr uint32_t kBoxWindow = 128;   // records staged between evaluations
 constexpr uint32_t kBoxList = 80;      // 64 records in up to 16 slices, one slot of padding each (LDS banks)
-constexpr float kBoxCompact = 0.3f;    // half-extent in r_cut up to which a segment stays one group
+// FP64: half-extent in r_cut up to which a segment stays one group. The value
+// hardly matters: with 0.15 and 0.6 solves of 96^3, VJPs of 64^3 and steps of
+// 32^3 take the time they take with 0.3, to 1 %.
+constexpr float kBoxCompact = 0.3f;
 constexpr int kBoxWide = 96;
 constexpr int kBoxStack = kBoxWide + 56 + 7 * 21 + 13;
 
@@ -2316,18 +2307,25 @@ __device__ __forceinline__ uint32_t box_segment(uint32_t seg, uint32_t per_wave,
 // second half of the window takes a batch's overflow and stages the leaves of
 // the lane-by-lane walks.
 //
-// The pairs' separations are the counting walk's: FP32 differences of offsets
-// from one origin, the centre of the 64 targets that share one of its waves,
-// or fixed-point differences where those span too much for it (SHARED). In FP32 a pair
-// within about 1e-7 of r_cut may fall on either side of it, and the residual
-// is still 1.8e-2 of Newtonian there: about one pair in 2.6e7 does, one per
-// 64^3 box, which moves a 32^3 box's force field by 2e-6 in relative L2 (1e-7
-// otherwise). So up to 2^20 sources both walks decide each pair alike; beyond,
+// The pairs' separations are FP32 differences of offsets from an origin (or
+// fixed-point differences where the origin's targets span too much for it). In
+// FP32 a pair within about 1e-7 of r_cut may fall on either side of it, and the
+// residual is still 1.8e-2 of Newtonian there, so one pair moves a 32^3 box's
+// force field by up to 2e-6 in relative L2 (1e-7 otherwise). Up to 2^20 sources
+// the origin is that of the 64 targets that share a wave of the counting walk
+// (SHARED), so the side does not depend on how the targets are cut into waves
+// and segments. It may still differ from the counting walk's, whose offsets
+// are scaled to other units: one pair in 6e6 of a random 2^20 box does, one in
+// 6e6 of a 96^3 lattice, one in 5e5 of a 32^3 one, no fewer than with segment
+// origins (65 and 64 targets, 14 and 20, 6 and 4). The errors against FP64 are
+// alike too (1.2e-6 and 1.0e-6, 3.5e-6 and 2.7e-6, 1.0e-6 and 0.7e-6). Beyond,
 // where single pairs do not show, the origin is the segment's centre, which the
 // box test can share (256^3: 4 % of the solve). SHARED holds both forms of a
 // pair: 4 waves per SIMD without spills instead of 5 with 27 registers spilled
 // (eleven boxes of 32^3 to 96^3: 6.01 to 5.34 ms; one of 100003: 1083 to 1020
 // us). FP64 decisions took 27 VALU instructions per pair against 16.
+// With segment origins 5 waves (96 VGPRs, 11 spilled, 18 KB of LDS) are bound
+// by VALU issue at 256^3: the SIMDs issue vector instructions in every cycle.
 template <int SCHEME, bool CUBIC, bool LOG, int WAVES, bool FRAME, bool SHARED>
 __global__ __launch_bounds__(WAVES * kWave) __attribute__((amdgpu_waves_per_eu(SHARED ? 4 : 5)))
 void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long long* __restrict__ counters,
@@ -2372,7 +2370,7 @@ void walkmix_box_kernel(WalkParams P, WalkData D, WalkOutputs out, unsigned long
 
   // beyond r_cut of every target whose offset the origin admits (2^28 units per axis)
   const float far = 2.0f * fmaf(268435456.0f, fmaxf(u0, fmaxf(u1, u2)), sqrtf(rc2));
-  // --- the counting walk's origin (SHARED), else the segment's ---
+  // --- the origin of the 64 targets around (SHARED), else the segment's ---
   uint32_t wox = 0, woy = 0, woz = 0;
   bool wave_origin = false;
   if constexpr (!SHARED) {
@@ -3052,6 +3050,11 @@ __global__ __launch_bounds__(kWalkThreads) void walk64_target_kernel(WalkParams 
 // a multipole are walked lane by lane with walk64_kernel's tests (cell prune,
 // accept64, node_accel64). The pairs and multipoles are walk64_kernel's; the
 // pair arithmetic and the summation order differ at the round-off level.
+// What bounds it at 96^3 is waiting: 1.4 of 3 possible waves are resident per
+// SIMD on average (13824 waves of uneven length), spend half of their cycles
+// waiting, and spill 114 VGPRs (444 bytes per lane); the SIMDs issue vector
+// instructions in 36 % of the cycles. The JVP at 64^3: 1.2 of 2 waves, 167
+// VGPRs spilled, 30 %.
 constexpr int kH64Cells = kH64MaxCells;
 
 // JVP: the transpose of the acceleration Jacobian applied to lam, as in
@@ -3327,7 +3330,7 @@ __global__ __launch_bounds__(kWalkThreads) __attribute__((amdgpu_waves_per_eu(JV
       // lies beyond r_cut, so their terms are zero) are dropped
       const double cull2 = rc2 * (1.0 + 1.0e-9);
       uint32_t wn = 0;  // records in the window
-      // evaluation groups as in walkmix_box_kernel
+      // evaluation groups of kBoxGroup targets, or the whole segment
       const double compact = kBoxCompact * rc;
       const bool one = TL <= kBoxGroup || (ex <= compact && ey <= compact && ez <= compact);
       const uint32_t lgG = one ? lgT : 4u, GL = 1u << lgG, lgGS = 6u - lgG;
@@ -3757,8 +3760,9 @@ std::vector<float> log_residual_table(double scale, double eps, double a, int32_
 
 std::vector<double> gaussian_quintic_table(double t_max, int cells, double factor) {
   // Interpolation at the Chebyshev points of each cell: error below
-  // 2 (h/4)^6 max|H^(6)| / 6!, under 1e-16 for cells of width 0.04 and
-  // about 1e-13 at width 0.2 (t_max = 50 on 255 cells). The 6 x 6
+  // 2 (h/4)^6 max|H^(6)| / 6!, largest in the first whole cell: 4e-16 for cells
+  // of width 0.04 (r_cut up to 6.4 a), 9e-14 at width 0.1 (10 a) and 6e-12 at
+  // width 0.2 (14 a; t_max = 50 on 255 cells). The 6 x 6
   // Vandermonde system in u is solved in long double. The first cell covers
   // t >= 0 only, u in [0, 1/2].
   const double h = t_max / cells;
