@@ -1035,10 +1035,11 @@ __global__ __launch_bounds__(kWalkThreads) void walk64_kernel(WalkParams P, Walk
 //      only for its counters, when they are read.
 // Four waves share a block for the FP64 pair table's cells up to r_cut: 12 KB
 // of LDS instead of gathers from a 128 KB table in memory. What bounds it is
-// the latency of the walk's dependent loads at 2 to 3 waves per SIMD, then FP64
-// issue in the pairs. Kernel time, 128^3 bodies and a 256^3 mesh in FP64: 23.1
-// ms, with the window and the table in LDS 21, with the stack 12.2; 1500001
-// bodies mixed: 15.0 to 10.8 ms.
+// waiting, most of it for the walk's dependent loads: of 2 (FP64) or 3 (mixed)
+// possible waves per SIMD 1.4 are resident on average and wait in 59 % of their
+// cycles, and the SIMDs issue vector instructions in a third. Kernel time,
+// 128^3 bodies and a 256^3 mesh in FP64: 23.1 ms, with the window and the table
+// in LDS 21, with the stack 12.2; 1500001 bodies mixed: 15.0 to 10.8 ms.
 // Groups above 64 targets are evaluated 64 targets at a time, repeating the
 // (identical) tree walk for each.
 //
